@@ -460,22 +460,26 @@ int finalize(dsb_handle* h) {
     CK(hipGetDevice(&dev));
     CK(hipDeviceGetAttribute(&h->ncu, hipDeviceAttributeMultiprocessorCount, dev));
     // split-K partials: the largest ks·M·N over the cycle's bf16/fp32 products
-    // that gemm_split_count splits, and the largest ks·tail tile partials of
-    // those gemm_tail_split splits. Each product is (output width, base
-    // reduction depth, LoRA segment): qkv and o recompute, gh, gxn2, gctx,
-    // gxn1, the head's dH. A layer with the projection's LoRA reduces over
-    // base + segment, one without over the base alone; both are sized, so the
-    // split a product takes at run time always fits.
-    const int shapes[][3] = {{W3, D, 3 * r}, {D, q, r},  {I, D, r},         {D, 2 * I, 2 * r},
-                             {q, D, r},      {D, W3, 3 * r}, {D, h->vchunk, 0}};
+    // that gemm_plan splits, and the largest ks·tail tile partials of those
+    // gemm_tail_split splits. Each product is (output width, base reduction
+    // depth, LoRA segment, epilogue bytes per element): qkv and o recompute,
+    // gh, gxn2, gctx, gxn1, the head's dH. A layer with the projection's LoRA
+    // reduces over base + segment, one without over the base alone; both are
+    // sized, so the split a product takes at run time always fits.
+    const struct {
+      int n, k, seg;
+      double ob;
+    } shapes[] = {{W3, D, 3 * r, 2},    {D, q, r, 4},      {I, D, r, 8},
+                  {D, 2 * I, 2 * r, 4}, {q, D, r, 2},      {D, W3, 3 * r, 4},
+                  {D, h->vchunk, 0, 8}};
     long need = 0;
     for (const auto& sh : shapes) {
-      for (const int K : {sh[1], sh[1] + sh[2]}) {
-        const int ks = gemm_split_count(N, sh[0], K);
-        if (ks > 1) need = std::max(need, (long)ks * N * sh[0]);
+      for (const int K : {sh.k, sh.k + sh.seg}) {
+        const GemmPlan pl = gemm_plan(N, sh.n, K, sh.ob, true);
+        need = std::max(need, gemm_part_elems(N, sh.n, pl.ks));
         int tail = 0;
-        const int kt = gemm_tail_split(N, sh[0], K, h->ncu, &tail);
-        if (ks == 1 && kt > 1) need = std::max(need, (long)kt * tail * 65536);
+        const int kt = gemm_tail_split(N, sh.n, K, h->ncu, &tail);
+        if (pl.ks == 1 && kt > 1) need = std::max(need, (long)kt * tail * 65536);
       }
     }
     h->part_elems = need;
@@ -696,7 +700,13 @@ struct KScope {
 };
 
 const char* cfg_name(int cfg) {
-  return cfg == GEMM_BIG ? "gemm256" : cfg == GEMM_MID ? "gemm128" : "gemm64";
+  switch (cfg) {
+    case GEMM_BIG: return "gemm256";
+    case GEMM_WIDE: return "gemm256x128";
+    case GEMM_MID: return "gemm128";
+    case GEMM_NARROW: return "gemm128x64";
+    default: return "gemm64";
+  }
 }
 
 // One NT GEMM launch of the cycle (M = live tokens), timed under
@@ -706,22 +716,24 @@ template <class Epi>
 int gemm(dsb_handle* h, const char* epi, const GemmProblem& p, const Epi& e, hipStream_t st,
          double ob, double xrow) {
   const double K = (double)p.K1 + p.K2;
-  if constexpr (std::is_same<Epi, EpiBF16>::value || std::is_same<Epi, EpiSwiGLUBwd>::value ||
-                std::is_same<Epi, EpiF32>::value) {
-    // too few 256×256 tiles for the chip: split K (unless a tile is forced)
-    const int ksplit = h->gemm_cfg >= 0 ? 1 : gemm_split_count(p.M, p.N, p.K1 + p.K2);
-    if (ksplit > 1 && (long)ksplit * p.M * p.N <= h->part_elems) {
-      const bool t128 = gemm_split_tile(p.M, p.N, p.K1 + p.K2) == 128;
-      KScope ks(h, st, std::string(t128 ? "gemm128sk_" : "gemm256sk_") + epi, 2.0 * p.N * K, 0, 0,
+  constexpr bool can_split = SplitPart<Epi>::enabled;
+  GemmPlan pl = h->gemm_cfg >= 0
+                    ? GemmPlan{h->gemm_cfg, 1}
+                    : gemm_plan(p.M, p.N, p.K1 + p.K2, ob + xrow / p.N, can_split, p.glu_half);
+  if (gemm_part_elems(p.M, p.N, pl.ks) > h->part_elems)
+    pl = gemm_plan(p.M, p.N, p.K1 + p.K2, ob + xrow / p.N, false, p.glu_half);
+  if constexpr (can_split) {
+    if (pl.ks > 1) {
+      KScope ks(h, st, std::string(cfg_name(pl.cfg)) + "sk_" + epi, 2.0 * p.N * K, 0, 0,
                 2.0 * K + ob * p.N + xrow, 0, 2.0 * p.N * K);
       GemmProblem q = p;
       q.part = h->part;
-      LK(launch_gemm_split(q, e, ksplit, st));
+      LK(launch_gemm_split(q, e, pl, st));
       return 0;
     }
     // a partly filled last round of tiles: split K over the tail tiles
     int tail = 0;
-    const int kt = h->gemm_cfg >= 0 || ksplit > 1
+    const int kt = h->gemm_cfg >= 0 || pl.cfg != GEMM_BIG
                        ? 1
                        : gemm_tail_split(p.M, p.N, p.K1 + p.K2, h->ncu, &tail);
     if (kt > 1 && (long)kt * tail * 65536 <= h->part_elems) {
@@ -731,10 +743,9 @@ int gemm(dsb_handle* h, const char* epi, const GemmProblem& p, const Epi& e, hip
       return 0;
     }
   }
-  const int cfg = h->gemm_cfg >= 0 ? h->gemm_cfg : pick_gemm_cfg(p.M, p.N);
-  KScope ks(h, st, std::string(cfg_name(cfg)) + "_" + epi, 2.0 * p.N * K, 0, 0,
+  KScope ks(h, st, std::string(cfg_name(pl.cfg)) + "_" + epi, 2.0 * p.N * K, 0, 0,
             2.0 * K + ob * p.N + xrow, 0, 2.0 * p.N * K);
-  LK(launch_gemm(p, e, st, cfg));
+  LK(launch_gemm(p, e, st, pl.cfg));
   return 0;
 }
 
@@ -1321,12 +1332,11 @@ int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
     }
     {
       // the other 2·n·Vc·D: dH = dH·α + P·W_chunk
-      const int cfg = h->gemm_cfg >= 0 ? h->gemm_cfg : pick_gemm_cfg(N, D);
-      const bool split = head_dh_split(ha, c0) > 1;
+      const GemmPlan pl = head_dh_plan(ha, c0);
       int tail = 0;
       const bool tsplit = head_dh_tail(ha, c0, &tail) > 1;
       KScope ks(h, st,
-                std::string(split ? "gemm256sk" : tsplit ? "gemm256t" : cfg_name(cfg)) + "_f32",
+                std::string(tsplit ? "gemm256t" : cfg_name(pl.cfg)) + (pl.ks > 1 ? "sk" : "") + "_f32",
                 2.0 * Vc * D, 0, 0, 2.0 * Vc + 8.0 * D, 0, 2.0 * Vc * D);
       LK(head_chunk_dh(ha, c0, st));
     }
@@ -2044,13 +2054,13 @@ int dsb_op_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, const vo
     }
     cfg = -1;
   }
-  const int ks = cfg == -2 ? gemm_split_count(M, N, K1 + K2) : 1;
-  if (cfg == -2) cfg = -1;
-  if (ks > 1) {
-    OPCK(hipMalloc((void**)&p.part, sizeof(float) * (size_t)ks * M * N));
+  const double ob = out_f32 ? (accumulate ? 8.0 : 4.0) : (R ? 4.0 : 2.0);
+  const GemmPlan pl = cfg >= 0 ? GemmPlan{cfg, 1} : gemm_plan(M, N, K1 + K2, ob, cfg == -2);
+  if (pl.ks > 1) {
+    OPCK(hipMalloc((void**)&p.part, sizeof(float) * (size_t)gemm_part_elems(M, N, pl.ks)));
     hipError_t e1;
-    if (out_f32) e1 = launch_gemm_split(p, EpiF32{(float*)C, ldc, N, accumulate}, ks, s);
-    else e1 = launch_gemm_split(p, EpiBF16{(bf16*)C, ldc, N, (const bf16*)R, ldr}, ks, s);
+    if (out_f32) e1 = launch_gemm_split(p, EpiF32{(float*)C, ldc, N, accumulate}, pl, s);
+    else e1 = launch_gemm_split(p, EpiBF16{(bf16*)C, ldc, N, (const bf16*)R, ldr}, pl, s);
     const hipError_t e2 = e1 == hipSuccess ? hipStreamSynchronize(s) : e1;
     (void)hipFree(p.part);
     OPCK(e2);
@@ -2058,10 +2068,10 @@ int dsb_op_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, const vo
   }
   if (out_f32) {
     EpiF32 e{(float*)C, ldc, N, accumulate};
-    OPCK(launch_gemm(p, e, s, cfg));
+    OPCK(launch_gemm(p, e, s, pl.cfg));
   } else {
     EpiBF16 e{(bf16*)C, ldc, N, (const bf16*)R, ldr};
-    OPCK(launch_gemm(p, e, s, cfg));
+    OPCK(launch_gemm(p, e, s, pl.cfg));
   }
   OPCK(hipStreamSynchronize(s));
   return 0;
@@ -2079,7 +2089,7 @@ int dsb_op_gemm_glu(const void* A, int64_t lda, const void* B, int64_t ldb, cons
   p.glu_half = I;
   EpiGLU e{(bf16*)GU, ldgu, (bf16*)H, ldh, I};
   hipStream_t s = (hipStream_t)stream;
-  OPCK(launch_gemm(p, e, s));
+  OPCK(launch_gemm(p, e, s, gemm_plan(M, 2 * I, K1 + K2, H ? 3.0 : 2.0, false, I).cfg));
   OPCK(hipStreamSynchronize(s));
   return 0;
 }

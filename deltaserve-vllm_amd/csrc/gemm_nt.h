@@ -9,7 +9,7 @@
 //
 // Main loop. BK = 64: each K tile is a 128-byte run of every operand row,
 // fetched by direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds; 8 lanes
-// cover one row, so every request is a whole 128-byte line) into one of two
+// cover one row, so every request is a whole 128-byte line) into a ring of
 // LDS stages. Each wave owns a (BM/WM)×(BN/WN) sub-tile of
 // v_mfma_f32_16x16x32_bf16 accumulators, tied to their AGPRs by inline-asm
 // MFMAs (with the builtin the compiler gave each MFMA's result registers
@@ -38,6 +38,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "dsb_common.h"
@@ -324,7 +325,7 @@ DSB_DEV int fkn(int k) {
   return ((2 * (k & 3)) ^ (((k >> 3) & 1) << 3)) & (CPR - 1);
 }
 
-template <int BM, int BN, int WM, int WN, class Epi, bool KN = false>
+template <int BM, int BN, int WM, int WN, class Epi, bool KN = false, int NA = 2, int NB = 3>
 __global__ __launch_bounds__(WM* WN * 64)
 __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel(GemmProblem p, Epi epi) {
   constexpr int BK = 64;
@@ -336,13 +337,19 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   static_assert(TM % 32 == 0 && TN % 32 == 0, "wave tile must be 32-aligned");
   static_assert(IA >= 1 && IB >= 1 && BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "loader split");
   static_assert(NW % 2 == 0, "row-block parity is the wave's");
-  static_assert(IAB < 64, "vmcnt range");
-  // LDS: two A slots, then three B slots (elements). A K tile is loaded one
-  // step ahead of its use, the B tile two: B is the operand every XCD fetches
-  // (A's row panels are the XCD's own), so its loads miss L2 more often and
-  // get the longer lead.
+  static_assert(NB == NA || NB == NA + 1, "load order");
+  // Loads are issued in the order ..., A(j), B(j + NB − NA), ...: those after
+  // the last load of tile k + 1 that may still be in flight at step k's wait,
+  // and at the prologue's wait for its first tile.
+  constexpr int WSTEP = (NA - 2) * IAB + (NB > NA ? IB : 0);
+  constexpr int WPRO = WSTEP + IAB;
+  static_assert(WPRO < 64, "vmcnt range");
+  // LDS: NA slots of A tiles, then NB of B tiles (elements). A K tile is
+  // loaded NA − 1 steps ahead of its use, the B tile NB − 1 (256 × 256: one
+  // and two; B is the operand every XCD fetches, A's row panels are the XCD's
+  // own, so B's loads miss L2 more often and get the longer lead).
   constexpr int SA = BM * BK, SB = BN * BK;
-  __shared__ __attribute__((aligned(16))) bf16 smem[2 * SA + 3 * SB];
+  __shared__ __attribute__((aligned(16))) bf16 smem[NA * SA + NB * SB];
 
   int M = p.M;
   if (p.M_dev) M = min(M, *p.M_dev);
@@ -440,9 +447,10 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   const unsigned lds0 = lds_addr(smem);
 
   // Loads of K tile kt into stage slot `slot`, issued one at a time by
-  // issue_one(j) so they can be spread over a run of MFMAs. Tiles past the
-  // end (kt >= nk) fall past K of the second segment and fill the slot with
-  // zeros without touching memory.
+  // issue_one(j) so they can be spread over a run of MFMAs. Tiles past this
+  // block's range (kt >= kt1) get an empty descriptor: their loads fill the
+  // slot with zeros without touching memory, and loads complete in issue
+  // order all the same, so the waits' counts are constants.
   // A fill of K tile ktA into A slot sa and of K tile ktB into B slot sb;
   // dstB is biased by −SA elements, so B row offsets keep the SA of the
   // fragment-read layout (brow, btr).
@@ -454,7 +462,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   };
   auto a_slot = [&](int sa) { return lds0 + (unsigned)(sa * SA * 2) + (unsigned)(8 * wave * BK * 2); };
   auto b_slot = [&](int sb) {
-    return lds0 + (unsigned)((SA + sb * SB) * 2) + (unsigned)(8 * wave * BK * 2);
+    return lds0 + (unsigned)(((NA - 1) * SA + sb * SB) * 2) + (unsigned)(8 * wave * BK * 2);
   };
   auto make_fill = [&](int ktA, int sa, int ktB, int sb) {
     Fill f;
@@ -463,6 +471,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
       const int k0 = s1 ? ktA * BK : (ktA - nk1) * BK;
       const int kb = (k0 * 2) | ((k0 + lch * 8 < (s1 ? p.K1 : K2)) ? 0 : OOB);
       f.dA = s1 ? dA1 : dA2;
+      f.dA[2] = ktA < kt1 ? f.dA[2] : 0u;
       f.voA = (s1 ? voA1 : voA2) + kb;
       f.stA = s1 ? stA1 : stA2;
     }
@@ -474,6 +483,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
         f.dB = kn_rsrc(s1, k0);
       else
         f.dB = s1 ? dB1 : dB2;
+      f.dB[2] = ktB < kt1 ? f.dB[2] : 0u;
       f.voB = (s1 ? voB1 : voB2) + kb;
       f.s1B = s1;
     }
@@ -556,7 +566,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     }
   };
   auto a_base = [&](int sa) { return (const bf16*)smem + sa * SA; };
-  auto b_base = [&](int sb) { return (const bf16*)smem + SA + sb * SB; };
+  auto b_base = [&](int sb) { return (const bf16*)smem + (NA - 1) * SA + sb * SB; };
   constexpr int NM = FM * FN, NR = FM + (KN ? 2 : 1) * FN, H1 = IAB / 2;
   auto bfrag = [&](int buf, int fn) {
     if constexpr (KN)
@@ -620,53 +630,55 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     return f;
   };
 
-  // Prologue: tile kt0 loaded and published, slice 0 of it read, and in
-  // flight, in this order: A and B of tile kt0+1, then B of tile kt0+2.
+  // Prologue: every slot's tile requested at once (one latency, not one for
+  // the first tile and another for the next), then the first tile awaited and
+  // published and slice 0 of it read.
   {
     const Fill f = make_fill(kt0, 0, kt0, 0);
+    if constexpr (NB > NA) {
 #pragma unroll
-    for (int j = 0; j < IAB; ++j) issue_one(f, j);
+      for (int j = IA; j < IAB; ++j) issue_one(f, j);
+    }
+#pragma unroll
+    for (int t = 0; t < NA; ++t) {
+      const Fill g = make_fill(kt0 + t, t, kt0 + t + NB - NA, t + NB - NA);
+#pragma unroll
+      for (int j = 0; j < IAB; ++j) issue_one(g, j);
+    }
   }
-  wait_vm<0>();
+  wait_vm<WPRO>();
   lds_barrier();
 #pragma unroll
   for (int i = 0; i < NR; ++i) read_one(a_base(0), b_base(0), 0, 0, i);
-  {
-    const Fill f = make_fill(kt0 + 1, 1, kt0 + 1, 1);
-#pragma unroll
-    for (int j = 0; j < IAB; ++j) issue_one(f, j);
-    const Fill fb = make_fill(kt0 + 1, 1, kt0 + 2, 2);
-#pragma unroll
-    for (int j = IA; j < IAB; ++j) issue_one(fb, j);
-  }
 
-  // Step kt computes on A slot (kt−kt0)&1 and B slot (kt−kt0)%3 (fragments of
-  // slice 0 already in buffer 0). Its mid-step wait leaves in flight only the
-  // B loads of tile kt+2 (issued last, in the step before): A and B of tile
-  // kt+1 have landed. After that barrier its slots are free, and it issues A
-  // of tile kt+2 and then B of tile kt+3 into them.
+  // Step kt computes on A slot (kt−kt0) % NA and B slot (kt−kt0) % NB
+  // (fragments of slice 0 already in buffer 0). Its mid-step wait leaves in
+  // flight the loads issued after those of tile kt+1. After that barrier tile
+  // kt's slots are free, and it issues A of tile kt+NA and then B of tile
+  // kt+NB into them.
+  int ca = 0, cb = 0;
   auto step = [&](int kt, auto&& mk) {
-    const int ca = (kt - kt0) & 1, cb = (kt - kt0) % 3;
     const bf16* ba = a_base(ca);
     const bf16* bb = b_base(cb);
-    const Fill next = mk(kt + 2, ca, kt + 3, cb);
+    const Fill next = mk(kt + NA, ca, kt + NB, cb);
+    ca = ca + 1 == NA ? 0 : ca + 1;
+    cb = cb + 1 == NB ? 0 : cb + 1;
     __builtin_amdgcn_sched_barrier(0);
     mma(0, 0, NM / 2, ba, bb, 1, 1, NR, next, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
     wait_lgkm0();
-    wait_vm<IB>();
+    wait_vm<WSTEP>();
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
     mma(0, NM / 2, NM, ba, bb, 1, 1, 0, next, 0, H1);
     __builtin_amdgcn_sched_barrier(0);
-    mma(1, 0, NM, a_base(ca ^ 1), b_base(cb == 2 ? 0 : cb + 1), 0, 0, NR, next, H1, IAB - H1);
+    mma(1, 0, NM, a_base(ca), b_base(cb), 0, 0, NR, next, H1, IAB - H1);
     __builtin_amdgcn_sched_barrier(0);
   };
-  // Steps whose prefetches (A tile kt+2, B tile kt+3) stay in segment 1 use
+  // Steps whose prefetches (A tile kt+NA, B tile kt+NB) stay in segment 1 use
   // the invariant segment-1 fill; the last few steps select the segment per
-  // tile. (Tiles past this block's range that the last steps prefetch are
-  // other blocks' tiles or zero fills past K: loaded, never multiplied.)
-  const int nfast = max(kt0, min(kt1, nk1 - 3));
+  // tile, and load nothing past this block's range.
+  const int nfast = max(kt0, min(kt1, nk1) - NB);
   int kt = kt0;
   for (; kt < nfast; ++kt) step(kt, make_fill1);
   for (; kt < kt1; ++kt) step(kt, make_fill);
@@ -968,9 +980,85 @@ struct EpiF32 {
   }
 };
 
-// Tile configurations. Big: 256×256, 4 waves of 128×128 (256 accumulators per
-// lane). Mid: 128×128, 4 waves of 64×64. Skinny: 64×64, 4 waves of 32×32.
-enum GemmCfg { GEMM_BIG = 0, GEMM_MID = 1, GEMM_SKINNY = 2 };
+// Tile configurations, all of 4 waves (2×2). LDS slots (A, B) and the blocks
+// a CU holds by LDS: 256×256 (2, 3) 160 KB, 1; 256×128 (3, 3) 144 KB, 1;
+// 128×128 (2, 3) 80 KB, 2; 128×64 (3, 3) 72 KB, 2; 64×64 (5, 5) 80 KB, 2.
+// A deeper ring of the 128×128 tile ((3, 3), (5, 5)) measured the same as
+// (2, 3) within 3 %; 128×256 and 256×64 tiles, and 4×1 waves, measured the
+// same as or behind one of these five everywhere.
+enum GemmCfg { GEMM_BIG = 0, GEMM_MID = 1, GEMM_SKINNY = 2, GEMM_WIDE = 3, GEMM_NARROW = 4 };
+constexpr int kGemmCfgs = 5;
+
+struct GemmTile {
+  int bm, bn, occ;  // occ: blocks a CU holds
+  double step;      // µs of one 64-deep K step of one block
+};
+inline GemmTile gemm_tile(int cfg) {
+  switch (cfg) {
+    case GEMM_BIG: return {256, 256, 1, 1.18};
+    case GEMM_WIDE: return {256, 128, 1, 0.74};
+    case GEMM_MID: return {128, 128, 2, 0.51};
+    case GEMM_NARROW: return {128, 64, 2, 0.36};
+    default: return {64, 64, 2, 0.26};
+  }
+}
+
+// Estimated time (µs) of an M × N × K product with tile `cfg` and ks K slices,
+// `ob` bytes read and written per output element by its epilogue. The
+// constants are a fit (rms 10 %) to 3700 timings of the five tiles at 1 to 16
+// slices, weights cold, over the products of the model widths the repository
+// configures at 96 to 4718 rows:
+//   main loop: the busiest CU's blocks, one after the other (blocks that
+//     share a CU share its LDS bandwidth, so co-residency hides prologues
+//     but no step time), at least the operands at 6.8 TB/s;
+//   epilogue: its bytes at 7.8 TB/s over the CUs in use;
+//   a split: fp32 partials written, then read by one more launch.
+// The tile and split with the least estimate ran within 1 % of the fastest
+// measured one on average (16 % at worst); the rule it replaces (256×256 or,
+// under 192 such tiles, 128×128, and 256 / tiles K slices of 256×256 up to 128
+// tiles) 23 %.
+inline double gemm_cost(int M, int N, int K, double ob, int cfg, int ks) {
+  const GemmTile t = gemm_tile(cfg);
+  const double tiles = (double)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+  const int nk = (K + 63) / 64, steps = (nk + ks - 1) / ks;
+  const double blocks = tiles * ks;
+  const double per_cu = std::ceil(blocks / 256), rounds = std::ceil(blocks / (256 * t.occ));
+  const double operands = 2.0 * K * ((double)M + N);
+  double us = 5.0 + std::max(per_cu * steps * t.step + rounds * 0.5, operands / 6.8e6);
+  us += per_cu * t.bm * t.bn * (ks > 1 ? 4.0 : ob) * std::min(blocks, 256.0) / 7.8e6;
+  if (ks > 1) us += 2.9 + (4.0 * ks * M * N + ob * M * N) / 3.9e6;
+  return us;
+}
+
+// The tile and the number of K slices (1: none) of a product.
+struct GemmPlan {
+  int cfg, ks;
+};
+// can_split: the epilogue has apply8 (SplitPart) and the caller provides the
+// partials' buffer (gemm_part_elems); glu_half: the gated layout's half (the
+// tile's columns hold whole halves).
+inline GemmPlan gemm_plan(int M, int N, int K, double ob, bool can_split, int glu_half = 0) {
+  GemmPlan best{GEMM_BIG, 1};
+  double bt = 0;
+  const int nk = (K + 63) / 64;
+  for (int cfg = 0; cfg < kGemmCfgs; ++cfg) {
+    const GemmTile t = gemm_tile(cfg);
+    if (glu_half > 0 && glu_half % (t.bn / 2)) continue;
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    // slices: at least 3 K tiles each, and the split's blocks within one round
+    const int most = can_split && N % 8 == 0 ? std::min(16, nk / 3) : 1;
+    for (int ks = 1; ks <= std::max(1, most); ++ks) {
+      if (ks > 1 && tiles * ks > 256 * t.occ) break;
+      const double c = gemm_cost(M, N, K, ob, cfg, ks);
+      if (bt == 0 || c < bt) {
+        bt = c;
+        best = GemmPlan{cfg, ks};
+      }
+    }
+  }
+  return best;
+}
+inline long gemm_part_elems(int M, int N, int ks) { return ks > 1 ? (long)ks * M * N : 0; }
 
 // Sum of the split-K partials of p (in split order, so the result does not
 // depend on scheduling) through epi.apply8, 8 columns per thread, live rows
@@ -998,86 +1086,52 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(GemmProblem p, i
   epi.apply8(m, n, v);
 }
 
-template <int BM, int BN, int WM, int WN, class Epi>
+template <int BM, int BN, int WM, int WN, int NA = 2, int NB = 3, class Epi>
 hipError_t launch_gemm_cfg(const GemmProblem& p, const Epi& e, hipStream_t s, int ks = 1) {
   const int nbm = (p.M + BM - 1) / BM, nbn = (p.N + BN - 1) / BN;
   if (nbm == 0 || nbn == 0) return hipSuccess;
   const dim3 grid(nbm * nbn, ks);
   if (p.b_kn)
-    hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, WM, WN, Epi, true>), grid, dim3(WM * WN * 64), 0,
+    hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, WM, WN, Epi, true, NA, NB>), grid, dim3(WM * WN * 64), 0,
                        s, p, e);
   else
-    hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, WM, WN, Epi, false>), grid, dim3(WM * WN * 64),
+    hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, WM, WN, Epi, false, NA, NB>), grid, dim3(WM * WN * 64),
                        0, s, p, e);
   return hipGetLastError();
 }
 
-inline GemmCfg pick_gemm_cfg(int M, int N) {
-  if (N <= 64) return GEMM_SKINNY;
-  const long big_tiles = (long)((M + 255) / 256) * ((N + 255) / 256);
-  if (big_tiles >= 192) return GEMM_BIG;
-  // One 256-row block (a serving-size cycle): the product streams its
-  // weights, and 128-wide tiles only fetch each weight panel twice (once per
-  // 128-row half); from 64 tiles up the 256-wide tile streams faster (M = 256,
-  // K = 5120: N = 17408 97 µs against 120, N = 34816 140 against 227).
-  if (M <= 256 && big_tiles >= 64) return GEMM_BIG;
-  return GEMM_MID;
-}
-
 template <class Epi>
-hipError_t launch_gemm(const GemmProblem& p, const Epi& e, hipStream_t s, int cfg = -1) {
-  if (cfg < 0) cfg = pick_gemm_cfg(p.M, p.N);
+hipError_t launch_gemm(const GemmProblem& p, const Epi& e, hipStream_t s, int cfg, int ks = 1) {
   if constexpr (std::is_same<Epi, EpiGLU>::value) {
-    // the gated layout needs two 32-column fragments per wave half
-    if (cfg == GEMM_BIG && p.glu_half % 128 == 0) return launch_gemm_cfg<256, 256, 2, 2>(p, e, s);
-    if (p.glu_half % 64 != 0) return hipErrorInvalidValue;
-    return launch_gemm_cfg<128, 128, 2, 2>(p, e, s);
-  } else {
-    switch (cfg) {
-      case GEMM_BIG: return launch_gemm_cfg<256, 256, 2, 2>(p, e, s);
-      case GEMM_MID: return launch_gemm_cfg<128, 128, 2, 2>(p, e, s);
-      default: return launch_gemm_cfg<64, 64, 2, 2>(p, e, s);
-    }
+    // the gated layout needs whole halves in a tile: a forced tile that is too
+    // wide gives way to a narrower one
+    if (cfg == GEMM_BIG && p.glu_half % 128) cfg = GEMM_MID;
+    if ((cfg == GEMM_MID || cfg == GEMM_WIDE) && p.glu_half % 64) return hipErrorInvalidValue;
+  }
+  switch (cfg) {
+    case GEMM_BIG: return launch_gemm_cfg<256, 256, 2, 2, 2, 3>(p, e, s, ks);
+    case GEMM_WIDE: return launch_gemm_cfg<256, 128, 2, 2, 3, 3>(p, e, s, ks);
+    case GEMM_MID: return launch_gemm_cfg<128, 128, 2, 2, 2, 3>(p, e, s, ks);
+    case GEMM_NARROW: return launch_gemm_cfg<128, 64, 2, 2, 3, 3>(p, e, s, ks);
+    default: return launch_gemm_cfg<64, 64, 2, 2, 5, 5>(p, e, s, ks);
   }
 }
 
-// K split over the grid's y dimension for problems with too few 256×256
-// tiles to fill the chip: `ks` blocks per tile each store the fp32 partial
-// of a slice of K to p.part ([ks, M, N]), then one reduction launch sums them
-// and applies the epilogue (those with apply8: EpiBF16, EpiF32, EpiSwiGLUBwd);
-// N a multiple of 8.
-// Splits so the tiles × splits blocks fit one round of the 256 CUs (a second,
-// partly filled round costs more than it spreads), at least 4 K tiles each;
-// 1 when the problem has more than 128 tiles (the fp32 partials' traffic
-// would buy no more parallelism).
-// The split's tile: 128 × 128 for one 256-row block over K ≤ 8192 when those
-// tiles stay within 128 (a serving-size cycle's K = 5120–7168 products: the
-// smaller tiles need fewer K slices to fill the CUs, so less partial traffic;
-// M = 256, N = 5120, K = 5120: 32 µs against 37), else 256 × 256.
-inline int gemm_split_tile(int M, int N, int K) {
-  const long mid = (long)((M + 127) / 128) * ((N + 127) / 128);
-  return M <= 256 && K <= 8192 && mid <= 128 ? 128 : 256;
-}
-inline int gemm_split_count(int M, int N, int K) {
-  const int t = gemm_split_tile(M, N, K);
-  const long tiles = (long)((M + t - 1) / t) * ((N + t - 1) / t);
-  const int nk = (K + 63) / 64;
-  if (tiles > 128 || N % 8 != 0 || nk < 8) return 1;
-  const int ks = std::min((int)(256 / tiles), std::min(8, nk / 4));
-  return ks >= 2 ? ks : 1;
-}
+// K split over the grid's y dimension: `ks` blocks per tile each store the
+// fp32 partial of a slice of K to p.part ([ks, M, N]), then one reduction
+// launch sums them and applies the epilogue (those with apply8: EpiBF16,
+// EpiF32, EpiSwiGLUBwd); N a multiple of 8.
 template <class Epi>
-hipError_t launch_gemm_split(const GemmProblem& p, const Epi& e, int ks, hipStream_t s) {
+hipError_t launch_gemm_split(const GemmProblem& p, const Epi& e, const GemmPlan& pl,
+                             hipStream_t s) {
   static_assert(SplitPart<Epi>::enabled, "split-K epilogues");
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
-  if (!p.part || p.N % 8 != 0 || ks < 2) return hipErrorInvalidValue;
-  const hipError_t e0 = gemm_split_tile(p.M, p.N, p.K1 + p.K2) == 128
-                           ? launch_gemm_cfg<128, 128, 2, 2>(p, e, s, ks)
-                           : launch_gemm_cfg<256, 256, 2, 2>(p, e, s, ks);
+  if (!p.part || p.N % 8 != 0 || pl.ks < 2) return hipErrorInvalidValue;
+  const hipError_t e0 = launch_gemm(p, e, s, pl.cfg, pl.ks);
   if (e0 != hipSuccess) return e0;
   const long n = (long)p.M * (p.N / 8);
   hipLaunchKernelGGL(gemm_split_reduce_kernel<Epi>, dim3((unsigned)((n + 255) / 256)), dim3(256),
-                     0, s, p, ks, e);
+                     0, s, p, pl.ks, e);
   return hipGetLastError();
 }
 

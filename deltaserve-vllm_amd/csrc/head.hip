@@ -325,16 +325,18 @@ hipError_t head_finalize(const HeadArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-int head_dh_split(const HeadArgs& a, int c0) {
-  if (a.gemm_cfg >= 0 || !a.part) return 1;
+GemmPlan head_dh_plan(const HeadArgs& a, int c0) {
+  if (a.gemm_cfg >= 0) return GemmPlan{a.gemm_cfg, 1};
   const int Nc8 = (min(a.vchunk, a.V - c0) + 7) / 8 * 8;
-  const int ks = gemm_split_count(a.n, a.D, Nc8);
-  return ks > 1 && (long)ks * a.n * a.D <= a.part_elems ? ks : 1;
+  GemmPlan pl = gemm_plan(a.n, a.D, Nc8, 8.0, a.part != nullptr);
+  if (gemm_part_elems(a.n, a.D, pl.ks) > a.part_elems) pl = gemm_plan(a.n, a.D, Nc8, 8.0, false);
+  return pl;
 }
 
 int head_dh_tail(const HeadArgs& a, int c0, int* tail) {
   *tail = 0;
-  if (a.gemm_cfg >= 0 || !a.part || head_dh_split(a, c0) > 1) return 1;
+  const GemmPlan pl = head_dh_plan(a, c0);
+  if (a.gemm_cfg >= 0 || !a.part || pl.ks > 1 || pl.cfg != GEMM_BIG) return 1;
   const int Nc8 = (min(a.vchunk, a.V - c0) + 7) / 8 * 8;
   const int kt = gemm_tail_split(a.n, a.D, Nc8, a.ncu, tail);
   return kt > 1 && (long)kt * *tail * 65536 <= a.part_elems ? kt : 1;
@@ -349,15 +351,15 @@ hipError_t head_chunk_dh(const HeadArgs& a, int c0, hipStream_t s) {
   q.b_kn = 1;
   q.kb_rows = min(a.vchunk, a.V - c0);
   EpiF32 ef{a.dH, (long)a.D, a.D, c0 > 0 ? 1 : 0, a.alpha};
-  const int ks = head_dh_split(a, c0);
-  if (ks > 1) {
+  const GemmPlan pl = head_dh_plan(a, c0);
+  if (pl.ks > 1) {
     q.part = a.part;
-    return launch_gemm_split(q, ef, ks, s);
+    return launch_gemm_split(q, ef, pl, s);
   }
   int tail = 0;
   const int kt = head_dh_tail(a, c0, &tail);
   if (kt > 1) return launch_gemm_tail(q, ef, kt, tail, a.part, s);
-  return launch_gemm(q, ef, s, a.gemm_cfg);
+  return launch_gemm(q, ef, s, pl.cfg);
 }
 
 hipError_t head_fwd_bwd(const HeadArgs& a, hipStream_t s) {

@@ -195,9 +195,10 @@ hipError_t head_prob(const HeadArgs& a, int c0, hipStream_t s);
 hipError_t head_rescale(const HeadArgs& a, int c0, hipStream_t s);
 hipError_t head_chunk_dh(const HeadArgs& a, int c0, hipStream_t s);
 hipError_t head_finalize(const HeadArgs& a, hipStream_t s);
-// K splits head_chunk_dh uses for chunk c0 (1: none), over the whole product
-// or (head_dh_tail) over the tiles of its partly filled last round
-int head_dh_split(const HeadArgs& a, int c0);
+// the tile and K slices head_chunk_dh uses for chunk c0, and the K splits over
+// the tiles of its partly filled last round (1: none)
+struct GemmPlan;
+GemmPlan head_dh_plan(const HeadArgs& a, int c0);
 int head_dh_tail(const HeadArgs& a, int c0, int* tail);
 
 // ---- optim.hip

@@ -439,3 +439,49 @@ def test_clip_adamw():
         assert max_rel(dm[i], ms[i]) < 1e-5
         assert max_rel(dv[i], vs[i]) < 1e-5
         assert max_rel(dw[i], ws[i]) < 1e-5
+
+
+@pytest.mark.parametrize("kn", [False, True])
+@pytest.mark.parametrize("cfg", [3, 4, -1, -2])
+@pytest.mark.parametrize("M,N,K,K2", [(1, 8, 8, 8), (257, 136, 64, 0), (300, 264, 328, 48),
+                                      (504, 1024, 4096, 24), (130, 1032, 1024, 48),
+                                      (2048, 3072, 512, 24)])
+def test_gemm_tiles(cfg, M, N, K, K2, kn):
+    """The 256×128 and 128×64 tiles (cfg 3, 4) and the tile and split the
+    cost model picks without and with a split (-1, -2): one row past a tile,
+    ragged columns, K shorter than the load ring (1 and 2 K tiles against 3 to
+    5 slots), the LoRA segment's tile inside the ring's tail. fp32 output
+    against an fp32 product: a sum of K products of N(0, 1) values in any
+    order is within K·2^-24 of the largest partial sum, about 1e-5 of the
+    largest output here."""
+    from deltaserve_amd import ops
+    A, B = _bf(_rnd(M, K, seed=61)), _bf(_rnd(N, K, seed=62))
+    A2 = _bf(_rnd(M, K2, seed=63)) if K2 else None
+    B2 = _bf(_rnd(N, K2, seed=64)) if K2 else None
+    ref = A.float() @ B.float().t()
+    if K2:
+        ref += A2.float() @ B2.float().t()
+    got = ops.gemm_nt(A.to(DEV), _b_operand(B, kn), None if A2 is None else A2.to(DEV),
+                      _b_operand(B2, kn), out_dtype=torch.float32, cfg=cfg, b_kn=kn)
+    assert max_rel(got, ref) < 1e-5
+
+
+@pytest.mark.parametrize("M,I,K,K2", [(96, 192, 256, 16), (130, 3072, 1024, 32), (256, 14336, 256, 16),
+                                      (70, 8192, 64, 0)])
+def test_gemm_glu_tiles(M, I, K, K2):
+    """Gate‖up products whose cost-model tiles are 64×64, 128×64 or 256×128
+    (I = 192: a half that whole 256-wide tiles do not divide)."""
+    from deltaserve_amd import ops
+    A, B = _bf(_rnd(M, K, seed=71)), _bf(_rnd(2 * I, K, seed=72))
+    A2 = _bf(_rnd(M, K2, seed=73)) if K2 else None
+    B2 = _bf(_rnd(2 * I, K2, seed=74)) if K2 else None
+    ref = A.float() @ B.float().t()
+    if K2:
+        ref += A2.float() @ B2.float().t()
+    GU, H = ops.gemm_glu(A.to(DEV), B.to(DEV), None if A2 is None else A2.to(DEV),
+                         None if B2 is None else B2.to(DEV))
+    assert max_rel(GU, ref) < 8e-3
+    g, u = GU[:, :I].float(), GU[:, I:].float()
+    want = (g * torch.sigmoid(g) * u).to(torch.bfloat16)
+    # bf16 rounding of the same fp32 value: at most one ulp apart
+    assert ((H.float() - want.float()).abs() <= want.float().abs() * 2 ** -7 + 1e-30).all()
