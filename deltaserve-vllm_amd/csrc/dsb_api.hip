@@ -39,36 +39,6 @@ void set_error(const char* fmt, ...) {
 }
 const char* get_error() { return g_err; }
 
-// ------------------------------------------------------------ small kernels
-
-// labels[t] = pred[t] ? ids[t + 1] : -1; out-of-range ids raise err bit 1.
-__global__ void labels_kernel(const int64_t* __restrict__ ids, const int* __restrict__ pred,
-                              int* __restrict__ labels, int n, const int* n_dev, int V,
-                              int* err) {
-  int N = n;
-  if (n_dev) N = min(N, *n_dev);
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= N) return;
-  int lab = -1;
-  if (pred[t]) {
-    const int64_t id = ids[t + 1];
-    if (id < 0 || id >= V) {
-      atomicOr(err, 1);
-    } else {
-      lab = (int)id;
-    }
-  }
-  labels[t] = lab;
-}
-
-hipError_t build_labels(const int64_t* ids, const int* pred, int* labels, int n,
-                        const int* n_dev, int V, int* err, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(labels_kernel, dim3((n + 255) / 256), dim3(256), 0, s, ids, pred, labels, n,
-                     n_dev, V, err);
-  return hipGetLastError();
-}
-
 // ------------------------------------------------------------ host helpers
 
 // Integer packing of a cycle (trainer.py:510-518, head.py:63-72).
@@ -211,7 +181,8 @@ struct GraphSet {  // the cycle's graphs for one attention grid capacity
 
 struct dsb_handle {
   dsb_desc d{};
-  int D, Hq, Hkv, hd, q, kv, W3, I, V, r, L, N, max_tiles, ntn, vchunk, nvc, ce_bn;
+  int D, Hq, Hkv, hd, q, kv, W3, I, V, r, L, N, max_tiles, vchunk, nvc;
+  HeadArgs head{};  // the LM head's plan (tiles, K slices, statistics layout)
   // the adapter's rank (rv) and the rank the kernels run at (r: rv rounded up
   // to a multiple of 8; the padded rows of A and columns of B are zeros in the
   // bf16 operands, so they add nothing, and their gradients are not stored)
@@ -444,7 +415,7 @@ int finalize(dsb_handle* h) {
   CKR(dalloc(h, &h->grm32, NN * D));
   CKR(dalloc(h, &h->ores, NN * q));
   CKR(dalloc(h, &h->normed, NN * D));
-  CKR(dalloc(h, &h->stats, NN * h->ntn));
+  CKR(dalloc(h, &h->stats, NN * h->head.ntn));
   CKR(dalloc(h, &h->tgt_logit, NN));
   CKR(dalloc(h, &h->lse_h, NN));
   CKR(dalloc(h, &h->loss_row, NN));
@@ -463,16 +434,20 @@ int finalize(dsb_handle* h) {
     // that gemm_plan splits, and the largest ks·tail tile partials of those
     // gemm_tail_split splits. Each product is (output width, base reduction
     // depth, LoRA segment, epilogue bytes per element): qkv and o recompute,
-    // gh, gxn2, gctx, gxn1, the head's dH. A layer with the projection's LoRA
+    // gh, gxn2, gctx, gxn1, and the head's dH by its own plan. A layer with the projection's LoRA
     // reduces over base + segment, one without over the base alone; both are
     // sized, so the split a product takes at run time always fits.
     const struct {
       int n, k, seg;
       double ob;
     } shapes[] = {{W3, D, 3 * r, 2},    {D, q, r, 4},      {I, D, r, 8},
-                  {D, 2 * I, 2 * r, 4}, {q, D, r, 2},      {D, W3, 3 * r, 4},
-                  {D, h->vchunk, 0, 8}};
-    long need = 0;
+                  {D, 2 * I, 2 * r, 4}, {q, D, r, 2},      {D, W3, 3 * r, 4}};
+    long need = head_part_elems(h->head);
+    {
+      int tail = 0;
+      const int kt = gemm_tail_split(N, D, h->vchunk, h->ncu, &tail);
+      if (h->head.dh_ks == 1 && kt > 1) need = std::max(need, (long)kt * tail * 65536);
+    }
     for (const auto& sh : shapes) {
       for (const int K : {sh.k, sh.k + sh.seg}) {
         const GemmPlan pl = gemm_plan(N, sh.n, K, sh.ob, true);
@@ -880,16 +855,17 @@ int dual(dsb_handle* h, const DualSpec* sp, int count, int r, hipStream_t s) {
 }
 
 HeadArgs head_args(dsb_handle* h) {
-  HeadArgs ha{};
+  HeadArgs ha = h->head;
   ha.normed = h->normed; ha.ldh = h->D; ha.W = h->lm_w;
+  ha.ids = h->ids; ha.pred = h->d_pred; ha.err = &h->d_hdr->err;
   ha.labels = h->labels;
-  ha.n = h->N; ha.n_dev = &h->d_hdr->n; ha.D = h->D; ha.V = h->V; ha.stats = h->stats;
-  ha.ntn = h->ntn; ha.ce_bn = h->ce_bn;
+  ha.n_dev = &h->d_hdr->n; ha.stats = h->stats;
   ha.tgt_logit = h->tgt_logit; ha.lse = h->lse_h; ha.loss_row = h->loss_row;
   ha.run_m = h->run_m; ha.run_l = h->run_l; ha.alpha = h->alpha;
   ha.loss_out = &h->d_hdr->loss; ha.inv_nvalid = &h->d_hdr->inv_nvalid;
-  ha.dlog = h->dlog; ha.vchunk = h->vchunk; ha.dH = h->dH; ha.gemm_cfg = h->gemm_cfg;
-  ha.part = h->part; ha.part_elems = h->part_elems; ha.ncu = h->ncu;
+  ha.dlog = h->dlog; ha.dH = h->dH;
+  ha.part = ha.tail_part = h->part;
+  ha.tail_elems = h->part_elems; ha.ncu = h->gemm_cfg >= 0 ? 0 : h->ncu;
   return ha;
 }
 
@@ -897,7 +873,7 @@ HeadArgs head_args(dsb_handle* h) {
 // 2c and 2c+1 run the LM head's chunk c — its logits product with the tile
 // statistics and probabilities, then the rescale to the row's running
 // softmax reference and the dH product (segment 0 first builds the RoPE
-// table, the LoRA operand casts, the final norm and the labels; segment 2C-1
+// table, the LoRA operand casts, the final norm, the labels and target logits; segment 2C-1
 // ends with dH, the LSE and the loss and the final-norm backward); then one
 // segment per decoder layer, last layer first (forward recompute +
 // backward); the last segment runs the per-layer clip, AdamW and the publish
@@ -1296,7 +1272,7 @@ int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
       }
       // with the layer overlap, the last layer's recompute (which needs the
       // RoPE tables and the bf16 LoRA operands just written) runs beside the
-      // rest of this segment: the final norm, the labels and the first
+      // rest of this segment: the final norm, the labels, the target logits and the first
       // vocabulary chunk's logits
       if (h->overlap && !h->ktiming) CKR(fork_recompute(h, h->L - 1, st));
       {
@@ -1304,8 +1280,8 @@ int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
         LK(rmsnorm_fwd(h->final_in, h->act_ld, h->norm_w, h->normed, D, N, nd, D, eps, st));
       }
       {
-        KScope ks(h, st, "labels", 0, 0, 0, 16, 0, 0);
-        LK(build_labels(h->ids, h->d_pred, h->labels, N, nd, h->V, &h->d_hdr->err, st));
+        KScope ks(h, st, "ce_init", 0, 0, 0, 4.0 * D + 36, 0, 0);
+        LK(head_init(ha, st));
       }
     }
     const int c = seg / 2;
@@ -1313,18 +1289,14 @@ int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
     if ((seg & 1) == 0) {
       {
         // 2·n·Vc·D of the head's algorithmic 4·M·D·V (the logits product)
-        KScope ks(h, st, h->ce_bn == 128 ? "gemm256x128_ce_prob" : "gemm256_ce_prob",
-                  2.0 * Vc * D, 0, 0, 2.0 * D + 8.0 * Vc / h->ce_bn, 0,
-                  2.0 * Vc * D + 2.0 * Vc);
+        KScope ks(h, st, std::string(cfg_name(ha.ce_cfg)) + "_ce_prob", 2.0 * Vc * D, 0, 0,
+                  2.0 * D + 8.0 * Vc / ha.ce_bn, 0, 2.0 * Vc * D + 2.0 * Vc);
         LK(head_prob(ha, c0, st));
       }
       {
-        // bytes: the tile statistics and running state of every row, and the
-        // P pass over every row (4·Vc bytes) in the first chunk; later chunks
-        // scale only the rows whose maximum lies in them, which the count
-        // leaves out (a lower bound)
-        KScope ks(h, st, "ce_rescale", 0, 0, 0, 8.0 * Vc / h->ce_bn + 12 + (c0 == 0 ? 4.0 * Vc : 0.0),
-                  0, 0);
+        // bytes: the statistics and running state of every row (rows whose
+        // reference moves also scale their probabilities: left out)
+        KScope ks(h, st, "ce_rescale", 0, 0, 0, 8.0 * Vc / ha.ce_bn + 20, 0, 0);
         LK(head_rescale(ha, c0, st));
       }
       if (seg == 0 && h->overlap && !h->ktiming) CKR(join_recompute(h, st));
@@ -1332,11 +1304,11 @@ int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
     }
     {
       // the other 2·n·Vc·D: dH = dH·α + P·W_chunk
-      const GemmPlan pl = head_dh_plan(ha, c0);
       int tail = 0;
       const bool tsplit = head_dh_tail(ha, c0, &tail) > 1;
       KScope ks(h, st,
-                std::string(tsplit ? "gemm256t" : cfg_name(pl.cfg)) + (pl.ks > 1 ? "sk" : "") + "_f32",
+                std::string(tsplit ? "gemm256t" : cfg_name(ha.dh_cfg)) + (ha.dh_ks > 1 ? "sk" : "") +
+                    "_f32",
                 2.0 * Vc * D, 0, 0, 2.0 * Vc + 8.0 * D, 0, 2.0 * Vc * D);
       LK(head_chunk_dh(ha, c0, st));
     }
@@ -1613,15 +1585,12 @@ int dsb_create(const dsb_desc* d, dsb_handle** out) {
   // width of the bf16 dlogits tile (16384 columns: 268 MB at 8192 rows)
   h->vchunk = d->vocab_chunk > 0 ? d->vocab_chunk : 16384;
   h->vchunk = (int)std::min<long>(h->vchunk, ((long)h->V + 255) / 256 * 256);
-  // CE passes: 128-wide vocab tiles when 256-wide ones would leave a chunk's
-  // launch with under 192 tiles (short cycles: 256 tokens give 64), so the
-  // launch streams the head's weights over twice the CUs
-  h->ce_bn = (long)((h->N + 255) / 256) * (h->vchunk / 256) < 192 ? 128 : 256;
-  h->ntn = (h->V + h->ce_bn - 1) / h->ce_bn;
   h->nvc = (h->V + h->vchunk - 1) / h->vchunk;
   h->gemm_cfg = d->gemm_tile == 256 ? GEMM_BIG
               : d->gemm_tile == 128 ? GEMM_MID
               : d->gemm_tile == 64  ? GEMM_SKINNY : -1;
+  h->head.n = h->N; h->head.D = h->D; h->head.V = h->V; h->head.vchunk = h->vchunk;
+  head_plan(h->head, h->gemm_cfg, true);
   h->layers.resize(h->L);
   h->ktiming = (d->flags & DSB_FLAG_KTIMING) != 0;
   // Layer overlap pays where the products leave CUs idle: 256-token to
@@ -2265,34 +2234,27 @@ int dsb_op_head(const void* normed, int64_t ldh, const void* lm_w, const int64_t
   const int nv = pack_cycle(seq_lens, nseq, n, nullptr, pred.data(), nullptr);
   if (nv < 0) return fail(nullptr, "dsb_op_head: seq_lens must sum to n");
   TmpDev tmp;
-  const int ntn = (V + 255) / 256;
-  const int vchunk = std::min(vocab_chunk > 0 ? vocab_chunk : 16384, ((V + 255) / 256) * 256);
+  HeadArgs a{};
+  a.n = n; a.D = D; a.V = V;
+  a.vchunk = std::min(vocab_chunk > 0 ? vocab_chunk : 16384, ((V + 255) / 256) * 256);
+  head_plan(a, -1, false);
   int* dpred = tmp.alloc<int>(n + 1);
-  int* labels = tmp.alloc<int>(n + 1);
-  float2* stats = tmp.alloc<float2>((size_t)(n + 1) * ntn);
-  float* tl = tmp.alloc<float>(n + 1);
-  float* lse = tmp.alloc<float>(n + 1);
-  float* lr = tmp.alloc<float>(n + 1);
-  float* rm = tmp.alloc<float>(n + 1);
-  float* rl = tmp.alloc<float>(n + 1);
-  float* al = tmp.alloc<float>(n + 1);
-  float* scal = tmp.alloc<float>(4);
   int* err = tmp.alloc<int>(1);
-  bf16* dlog = tmp.alloc<bf16>((size_t)(n + 1) * vchunk);
-  if (!dpred || !labels || !stats || !tl || !lse || !lr || !rm || !rl || !al || !scal || !err ||
-      !dlog)
+  float* scal = tmp.alloc<float>(4);
+  a.labels = tmp.alloc<int>(n + 1);
+  a.stats = tmp.alloc<float2>((size_t)(n + 1) * a.ntn);
+  for (float** p : {&a.tgt_logit, &a.lse, &a.loss_row, &a.run_m, &a.run_l, &a.alpha})
+    if (!(*p = tmp.alloc<float>(n + 1))) return fail(nullptr, "dsb_op_head: hipMalloc failed");
+  a.dlog = tmp.alloc<bf16>((size_t)(n + 1) * a.vchunk);
+  if (!dpred || !err || !scal || !a.labels || !a.stats || !a.dlog)
     return fail(nullptr, "dsb_op_head: hipMalloc failed");
   float hsc[4] = {nv > 0 ? 1.f / nv : 0.f, 0.f, 0.f, 0.f};
   OPCK(hipMemcpy(scal, hsc, sizeof(hsc), hipMemcpyHostToDevice));
   if (n > 0) OPCK(hipMemcpy(dpred, pred.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
   OPCK(hipMemset(err, 0, sizeof(int)));
-  OPCK(build_labels(ids, dpred, labels, n, nullptr, V, err, s));
-  HeadArgs a{};
   a.normed = (const bf16*)normed; a.ldh = ldh; a.W = (const bf16*)lm_w;
-  a.labels = labels; a.n = n; a.n_dev = nullptr; a.D = D; a.V = V; a.stats = stats; a.ntn = ntn;
-  a.tgt_logit = tl; a.lse = lse; a.loss_row = lr; a.loss_out = scal + 1; a.inv_nvalid = scal;
-  a.run_m = rm; a.run_l = rl; a.alpha = al;
-  a.dlog = dlog; a.vchunk = vchunk; a.dH = dH; a.gemm_cfg = -1;
+  a.ids = ids; a.pred = dpred; a.err = err; a.n_dev = nullptr;
+  a.loss_out = scal + 1; a.inv_nvalid = scal; a.dH = dH;
   OPCK(head_fwd_bwd(a, s));
   OPCK(hipStreamSynchronize(s));
   int herr = 0;

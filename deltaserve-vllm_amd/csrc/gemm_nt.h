@@ -67,6 +67,10 @@ struct GemmProblem {
   // partial to part + z·M·N (row stride N) instead of running the epilogue;
   // gemm_split_reduce then sums the partials in order and applies it.
   float* part = nullptr;
+  // with part: accumulate into the partials, part = part·part_scale[row] + new
+  // (a sum carried over several products, the caller adding the slices once)
+  int part_acc = 0;
+  const float* part_scale = nullptr;
   // Tail launch (launch_gemm_tail): the launch's block x takes tile
   // tile0 + x of the problem's tile order; with tpart set, a block stores its
   // fp32 partial as one BM × BN tile (row stride BN) at
@@ -690,7 +694,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   if constexpr (SplitPart<Epi>::enabled) {
     if (p.part) {
       const typename SplitPart<Epi>::type ep{p.part + (long)blockIdx.y * p.M * p.N, (long)p.N,
-                                             p.N, 0};
+                                             p.N, p.part_acc, p.part_scale};
       ep.template run<FM, FN, WM, WN>(acc, m0 + wm * TM, n0 + wn * TN, M, lane, wave,
                                       (void*)smem);
       return;

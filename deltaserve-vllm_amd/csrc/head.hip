@@ -7,21 +7,27 @@
 //   grad_rows = dlogits · W. Rows that predict nothing (the last token of each
 //   sequence) carry label -1 and contribute neither loss nor gradient.
 //
-// Two vocabulary-wide products, with the softmax normalised online across
-// chunks as flash attention normalises across key tiles:
-//   per chunk c: logits = H·W_cᵀ (GEMM; its epilogue writes, per 256-column
-//     vocabulary tile t, the reference m_t = max(the tile's row max, the
-//     running max M of the earlier chunks) and Σ exp(logit − m_t), the target
-//     logit where the tile holds it, and P = bf16(exp(logit − m_t)));
-//   ce_rescale: per row, the chunk max M_c = max_t m_t, the running max M and
-//     sum L updated (M' = max(M, M_c), L' = L·e^(M−M') + Σ_t s_t·e^(m_t−M')),
-//     α = e^(M−M'), and P scaled in place by e^(m_t − M') (P = exp(logit − M'))
-//     on the rows where some m_t differs from M' (every row of the first
-//     chunk; later, only the rows whose maximum lies in the chunk);
+// Two vocabulary-wide products, with the softmax taken against a per-row
+// reference M that is known before the first product:
+//   ce_init: M = the row's target logit (a dot of the row with W[target]);
+//   per chunk c: logits = H·W_cᵀ (GEMM; its epilogue writes P = bf16(exp(logit
+//     − M)) and, per wave-wide run of vocabulary columns, Σ exp(logit − M).
+//     Any reference within a few tens of the row maximum serves: bf16 and
+//     fp32 keep their relative precision over that range. Only where a sum
+//     passes 2^57 (a logit more than about 40 above M) does the run take its
+//     own maximum m_t as its reference instead);
+//   ce_rescale: per row L += Σ_t s_t·e^(m_t − M) and, on the rows where some
+//     m_t differs from M, M' = max_t m_t, α = e^(M − M') and P scaled in place
+//     to M';
 //   dH = dH·α + P·W_c (GEMM, fp32 accumulate with the per-row α);
 //   after the last chunk: dH = (dH/L − W[target]) / n_valid (the onehot term
 //   exactly, in fp32), LSE = M + ln L, loss_row = LSE − target logit, and a
 //   single-block deterministic sum gives the cycle loss.
+// With the tile maxima as references (every row of the first chunk rescaled,
+// later ones where the row maximum lay in the chunk) the rescale took 48 µs
+// per chunk at 8192 rows and 14 µs at 504, whose rows' serial passes over P
+// set the time; reading the statistics alone takes 8.6 and 5.4 µs, and ce_init,
+// once per cycle, 24 and 4 µs.
 // Against the reference's 2 passes (logits for the LSE, then dlogits, both
 // chunked, head.py:78-80, :92-94) this keeps its 2·M·D·V of logits and
 // 2·M·D·V of dH and needs no third product. P passes through bf16 (the MFMA
@@ -34,176 +40,155 @@
 namespace dsb {
 
 namespace {
-constexpr int CE_BN = 256;
 
-// Per vocab tile (ce_bn columns) of chunk [c0, c0 + Vc): (reference m_t, sum
-// exp(logit − m_t)) per row into stats[m, c0/ce_bn + tile], m_t being the
-// tile's row max or, from the second chunk on, the running max when that is
-// larger; the target logit
-// where the tile holds it, and P[m, j] = bf16(exp(logit[m, c0 + j] − m_t)) for
-// the chunk's columns j < Vc; columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are
-// written as zero so the dH product runs its K loop over whole 16-byte chunks.
+// A run's sum of exp(logit − M) up to which M stays its reference: every term
+// is then at most 2^57, far inside fp32 and bf16 range, and so are the sums
+// and the dH accumulators (V and the weights add at most 2^30).
+constexpr float kSumLimit = 0x1p57f;
+
+// Per run of TN vocabulary columns (a wave tile's width) of chunk [c0, c0 + Vc)
+// and row: (reference m_t, Σ exp(logit − m_t)) into stats[m, (c0 + column) / TN]
+// and P[m, j] = bf16(exp(logit[m, c0 + j] − m_t)) for the chunk's columns
+// j < Vc; columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are written as zero so the
+// dH product runs its K loop over whole 16-byte chunks. m_t is run_m[m] unless
+// the run's sum passes kSumLimit (or is NaN), then the run's maximum.
+// A lane holds 4·FN values of a row, so the exponentials and the row sums are
+// taken in the accumulator layout (two shuffles per row) and only bf16 values
+// are staged for the row-contiguous stores; no barrier, each wave its own
+// rows and columns. The epilogue it replaces (a maximum pass, an exchange
+// between the waves of a row, fp32 staging and four shuffles per 8 values)
+// made the product of a 16384-column chunk take 951 µs at 8192 rows × 4096
+// against 791 now (the chunk's dH product, whose code did not change, 873 and
+// 798 µs in the same two runs), 147 → 116 µs at 2048 × 2048 and 30.5 → 25.3 µs
+// at 504 × 1024.
 struct EpiCEProb {
-  const int* labels;
   float2* stats;
   int ntn;
-  float* tgt_logit;
   bf16* P;
   long ldp;
   int c0, Vc, Nc8;
-  // the running max over the earlier chunks (null for the first chunk): each
-  // tile's reference is max(tile max, running max), so a row whose maximum is
-  // not in this chunk has one reference for all its tiles and needs no rescale
   const float* run_m;
   template <int FM, int FN, int WM, int WN>
   DSB_DEV void run(const f32x4 (&acc)[FM][FN], int mw, int nw, int M, int lane, int wave,
                    void* smem) const {
-    constexpr int TM = FM * 16, TN = FN * 16, BMl = WM * TM;
-    constexpr int PITCH = TN + 4, CG = TN / 8, RPI = 64 / CG;
-    constexpr int STG = WM * WN * 32 * PITCH;  // for the staging rows of every wave
-    static_assert((STG + 2 * BMl + WN * BMl) * 4 <= 2 * (WM * TM + WN * TN) * 64 * 2,
-                  "epilogue scratch fits the stages");
-    const int wn = wave % WN, wm = wave / WN;
-    const int n0 = nw - wn * TN;
-    const int pn = c0 / (WN * TN) + n0 / (WN * TN);
-    // lane l holds row l%16 of each 16-row block, columns 4(l/16) .. +3 of
-    // each 16-column block: a row's values of the wave tile sit in the four
-    // lanes l%16 + 16q, combined with two shuffles
+    constexpr int TN = FN * 16, PITCH = TN + 8, CG = TN / 8;
+    if (nw >= Vc || mw >= M) return;  // no live column or row in the wave tile
     const int l16 = lane & 15, lq = lane >> 4;
-    float* fs = reinterpret_cast<float*>(smem);
-    float* red = fs;               // [WN][BMl] per-wave row maxima, before the staging rows
-    float* rowmax = fs + STG;      // [BMl] the tile's row maxima
-    float* rowsum = rowmax + BMl;  // [WN][BMl] per-wave row sums of exp(logit − max)
-    int* tcol = reinterpret_cast<int*>(rowsum + WN * BMl);  // [BMl] target column in the chunk, or -1
-    // 1) row maxima over the tile's live columns (every column of the wave
-    //    tile is live except in the chunk's last tile: one wave-uniform test)
     const bool whole = nw + TN <= Vc;
+    const int run = (c0 + nw) / TN;
+    bf16* buf = reinterpret_cast<bf16*>(smem) + wave * 32 * PITCH;
+    // the rows' references, all loaded before the first is used (rows past M
+    // read row M − 1 and are not stored)
+    float ref0[FM];
 #pragma unroll
-    for (int fm = 0; fm < FM; ++fm) {
-      float v = -INFINITY;
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float x = acc[fm][fn][i];
-          v = (whole || nw + fn * 16 + 4 * lq + i < Vc) ? fmaxf(v, x) : v;
-        }
-      v = fmaxf(v, __shfl_xor(v, 16, 64));
-      v = fmaxf(v, __shfl_xor(v, 32, 64));
-      if (lq == 0) red[wn * BMl + wm * TM + fm * 16 + l16] = v;
-    }
-    // The accumulators' copies read above die here: the empty asm claims to
-    // rewrite each one in its AGPRs, so phase 2 reads them from there again
-    // instead of the compiler keeping VGPR copies across the barriers.
-    auto& accw = const_cast<f32x4 (&)[FM][FN]>(acc);
-#pragma unroll
-    for (int fm = 0; fm < FM; ++fm)
-#pragma unroll
-      for (int fn = 0; fn < FN; ++fn) asm volatile("" : "+a"(accw[fm][fn]));
-    __syncthreads();
-    if (wn == 0 && lq == 0) {
-      // the rows' labels and running maxima, all loaded before the first is
-      // used (rows past M read row M − 1 and are not used): loads behind a
-      // per-row test would each wait for the one before
-      int lab[FM];
-      float rmx[FM];
-#pragma unroll
-      for (int fm = 0; fm < FM; ++fm) lab[fm] = labels[min(mw + fm * 16 + l16, M - 1)];
-      if (run_m) {
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) rmx[fm] = run_m[min(mw + fm * 16 + l16, M - 1)];
-      } else {
-#pragma unroll
-        for (int fm = 0; fm < FM; ++fm) rmx[fm] = -INFINITY;
-      }
-#pragma unroll
-      for (int fm = 0; fm < FM; ++fm) {
-        const int row = wm * TM + fm * 16 + l16, m = mw + fm * 16 + l16;
-        float b = red[row];
-#pragma unroll
-        for (int j = 1; j < WN; ++j) b = fmaxf(b, red[j * BMl + row]);
-        if (run_m) b = fmaxf(b, rmx[fm]);
-        rowmax[row] = b;
-        const int t = m < M ? lab[fm] - c0 : -1;
-        tcol[row] = t >= 0 && t < Vc ? t : -1;
-      }
-    }
-    // the maxima are visible, and every wave is past its reads of `red`,
-    // before the staging rows overwrite it
-    __syncthreads();
-    // 2) P = bf16(exp(logit − max)) through the staging rows (one exp per
-    //    logit), each row's sum of the fp32 values reduced on the way: the
-    //    CG lanes of a staged row are consecutive
-    const int m0 = mw - wm * TM;
-    float* buf = fs + wave * 32 * PITCH;
-    const int rsub = lane / CG, cg = lane % CG;
-    const int n = nw + cg * 8;
+    for (int fm = 0; fm < FM; ++fm) ref0[fm] = run_m[min(mw + fm * 16 + l16, M - 1)];
 #pragma unroll
     for (int b = 0; b < FM / 2; ++b) {
       if (mw + b * 32 >= M) break;  // uniform: the rest of the wave tile is past M
-      stage32<FM, FN, PITCH>(acc, b, buf, lane);
 #pragma unroll
-      for (int it = 0; it < 32 / RPI; ++it) {
-        const int row = it * RPI + rsub, lrow = wm * TM + b * 32 + row, m = m0 + lrow;
-        const f32x4 x = *reinterpret_cast<const f32x4*>(buf + row * PITCH + cg * 8);
-        const f32x4 y = *reinterpret_cast<const f32x4*>(buf + row * PITCH + cg * 8 + 4);
-        const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
-        const float bm = rowmax[lrow];
-        // the target logit, where the row's target column is one of these 8
-        const int tj = tcol[lrow] - n;
-        if (m < M && (unsigned)tj < 8u) {
-          float x = v[0];
+      for (int h = 0; h < 2; ++h) {
+        const int fm = 2 * b + h;
+        bf16x4 pk[FN];
+        // lane: row l16, columns 16·fn + 4·lq + i
+        auto take = [&](float ref) {
+          float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int i = 1; i < 8; ++i) x = tj == i ? v[i] : x;
-          tgt_logit[m] = x;
+          for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              float e = __expf(acc[fm][fn][i] - ref);
+              if (!whole) e = nw + fn * 16 + 4 * lq + i < Vc ? e : 0.f;
+              part[i] += e;
+              pk[fn][i] = (bf16)e;
+            }
+          float v = (part[0] + part[1]) + (part[2] + part[3]);
+          v += __shfl_xor(v, 16, 64);
+          return v + __shfl_xor(v, 32, 64);
+        };
+        float ref = ref0[fm];
+        float sum = take(ref);
+        if (__any(!(sum <= kSumLimit))) {
+          // rare: the rows past the limit against their run's own maximum
+          float v = -INFINITY;
+#pragma unroll
+          for (int fn = 0; fn < FN; ++fn)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              v = whole || nw + fn * 16 + 4 * lq + i < Vc ? fmaxf(v, acc[fm][fn][i]) : v;
+          v = fmaxf(v, __shfl_xor(v, 16, 64));
+          v = fmaxf(v, __shfl_xor(v, 32, 64));
+          ref = sum <= kSumLimit ? ref : fmaxf(ref, v);
+          sum = take(ref);
         }
-        float e[8], part = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          e[i] = (whole || n + i < Vc) ? __expf(v[i] - bm) : 0.f;
-          part += e[i];
-        }
-#pragma unroll
-        for (int o = 1; o < CG; o <<= 1) part += __shfl_xor(part, o, 64);
-        if (cg == 0) rowsum[wn * BMl + lrow] = part;
-        const int lim = Nc8 - n;
-        if (m < M && lim > 0) {
-          bf16* d = P + (long)m * ldp + n;
-          if (lim >= 8) {
-            stg128(d, pack8(e));
-          } else {
-            for (int i = 0; i < lim; ++i) d[i] = (bf16)e[i];
-          }
-        }
-      }
-    }
-    __syncthreads();
-    // 3) the tile's (max, sum) per row
-    if (wn == 0 && lq == 0) {
-#pragma unroll
-      for (int fm = 0; fm < FM; ++fm) {
-        const int row = wm * TM + fm * 16 + l16;
+        for (int fn = 0; fn < FN; ++fn)
+          *reinterpret_cast<bf16x4*>(buf + (16 * h + l16) * PITCH + fn * 16 + 4 * lq) = pk[fn];
         const int m = mw + fm * 16 + l16;
-        float s = 0.f;
+        if (lq == 0 && m < M) stats[(long)m * ntn + run] = make_float2(ref, sum);
+      }
 #pragma unroll
-        for (int j = 0; j < WN; ++j) s += rowsum[j * BMl + row];
-        if (m < M) stats[(long)m * ntn + pn] = make_float2(rowmax[row], s);
+      for (int it = 0; it < 32 * CG / 64; ++it) {
+        const int c = lane + 64 * it, row = c / CG, m = mw + b * 32 + row;
+        const int n = nw + (c % CG) * 8;
+        const u32x4 v = *reinterpret_cast<const u32x4*>(buf + row * PITCH + (c % CG) * 8);
+        if (m < M && n < Nc8) stg128(P + (long)m * ldp + n, v);
       }
     }
   }
 };
 
+// Width of the runs the logits product's statistics cover: its wave tile's.
+constexpr int ce_run(int cfg) {
+  return cfg == GEMM_BIG ? 128 : cfg == GEMM_NARROW ? 32 : 64;
+}
+
 }  // namespace
 
+// One wave per live row: the label (ids[t + 1] where row t predicts, −1
+// elsewhere; an id outside [0, V) raises err bit 1), the target logit, which is
+// also the row's first softmax reference (0 for rows without a target), and
+// L = 0, α = 1.
+__global__ __launch_bounds__(256) void ce_init_kernel(HeadArgs a) {
+  int N = a.n;
+  if (a.n_dev) N = min(N, *a.n_dev);
+  const int m = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
+  if (m >= N) return;
+  int lab = -1;
+  if (a.pred[m]) {
+    const int64_t id = a.ids[m + 1];
+    if (id >= 0 && id < a.V)
+      lab = (int)id;
+    else if (l == 0)
+      atomicOr(a.err, 1);
+  }
+  float dot = 0.f;
+  if (lab >= 0) {
+    const bf16 *x = a.normed + (long)m * a.ldh, *w = a.W + (long)lab * a.D;
+    for (int k = l; k < a.D / 8; k += 64) {
+      float xf[8], wf[8];
+      unpack8(ldg128(x + 8 * k), xf);
+      unpack8(ldg128(w + 8 * k), wf);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) dot += xf[e] * wf[e];
+    }
+    dot = wave_sum(dot);
+  }
+  if (l == 0) {
+    a.labels[m] = lab;
+    a.tgt_logit[m] = dot;
+    a.run_m[m] = dot;
+    a.run_l[m] = 0.f;
+    a.alpha[m] = 1.f;
+  }
+}
+
 // Chunk [c0, c0 + Vc) after its logits product, one wave per live row: the
-// chunk max M_c of the tile references m_t and its sum, the running max M and
-// sum L (first chunk: M = −inf, L = 0) moved to M' = max(M, M_c), α = e^(M − M')
-// for the dH accumulator, and P scaled in place by e^(m_t − M') per tile, so
-// P = bf16(exp(logit − M')). After the first chunk every m_t is at least M, so
-// a row whose maximum is not in this chunk has m_t = M = M' for every tile and
-// its P is left as it is; so are the rows without a target, whose dH the
-// finalize sets to zero whatever the product accumulated (P <= 1: finite).
-__global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0, int first) {
+// runs' largest reference M_c, the row's reference M and sum L moved to
+// M' = max(M, M_c), α = e^(M − M') for the dH accumulator, and, on rows where
+// some run's reference is not M', P scaled in place by e^(m_t − M') so that
+// P = bf16(exp(logit − M')). Rows without a target keep their P: the finalize
+// sets their dH to zero whatever the product accumulated.
+__global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0) {
   int N = a.n;
   if (a.n_dev) N = min(N, *a.n_dev);
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
@@ -211,18 +196,18 @@ __global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0, int
   const int bn = a.ce_bn, Vc = min(a.vchunk, a.V - c0), Nc8 = (Vc + 7) / 8 * 8;
   const int nt = (Vc + bn - 1) / bn;
   const float2* st = a.stats + (long)m * a.ntn + c0 / bn;
+  const float mo = a.run_m[m];
   float mc = -INFINITY;
   for (int j = l; j < nt; j += 64) mc = fmaxf(mc, st[j].x);
   mc = wave_max(mc);
-  const float mo = first ? -INFINITY : a.run_m[m];
   const float mn = fmaxf(mo, mc);
   float sc = 0.f;
   for (int j = l; j < nt; j += 64) sc += st[j].y * __expf(st[j].x - mn);
   sc = wave_sum(sc);
   if (l == 0) {
-    const float al = first ? 0.f : __expf(mo - mn);
+    const float al = __expf(mo - mn);
     a.run_m[m] = mn;
-    a.run_l[m] = (first ? 0.f : a.run_l[m] * al) + sc;
+    a.run_l[m] = a.run_l[m] * al + sc;
     a.alpha[m] = al;
   }
   if (a.labels[m] < 0) return;
@@ -243,9 +228,10 @@ __global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0, int
 }
 
 // After the last chunk, one wave per live row: LSE = M + ln L, loss_row =
-// LSE − target logit, dH = (dH/L − W[target]) / n_valid; rows without a target
-// get dH = 0 and no loss.
-__global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a) {
+// LSE − target logit, dH = (dH/L − W[target]) / n_valid, with dH the sum in
+// order of the `ks` accumulated K-slice partials when the product was split;
+// rows without a target get dH = 0 and no loss.
+__global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
   int N = a.n;
   if (a.n_dev) N = min(N, *a.n_dev);
   const int m = blockIdx.x * 4 + (threadIdx.x >> 6), l = threadIdx.x & 63;
@@ -265,11 +251,19 @@ __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a) {
   }
   const float inv = 1.f / L, sc = *a.inv_nvalid;
   const bf16* w = a.W + (long)t * a.D;
+  const float* src = ks > 1 ? a.part + (long)m * a.D : dr;
+  const long plane = (long)a.n * a.D;
   for (int k = l; k < a.D / 8; k += 64) {
     float wf[8];
     unpack8(ldg128(w + 8 * k), wf);
+    f32x4 x0 = *reinterpret_cast<const f32x4*>(src + 8 * k);
+    f32x4 x1 = *reinterpret_cast<const f32x4*>(src + 8 * k + 4);
+#pragma unroll 4
+    for (int z = 1; z < ks; ++z) {
+      x0 += *reinterpret_cast<const f32x4*>(src + z * plane + 8 * k);
+      x1 += *reinterpret_cast<const f32x4*>(src + z * plane + 8 * k + 4);
+    }
     f32x4* d = reinterpret_cast<f32x4*>(dr + 8 * k);
-    const f32x4 x0 = d[0], x1 = d[1];
     d[0] = f32x4{(x0[0] * inv - wf[0]) * sc, (x0[1] * inv - wf[1]) * sc,
                  (x0[2] * inv - wf[2]) * sc, (x0[3] * inv - wf[3]) * sc};
     d[1] = f32x4{(x1[0] * inv - wf[4]) * sc, (x1[1] * inv - wf[5]) * sc,
@@ -299,25 +293,87 @@ static GemmProblem chunk_logits_problem(const HeadArgs& a, int c0) {
                      a.n, Vc, a.D, 0, a.n_dev};
 }
 
+void head_plan(HeadArgs& a, int gemm_cfg, bool can_split) {
+  // The logits product's tile (the 64-wide one has no epilogue here): by cost,
+  // over a full chunk, 2 bytes per element out.
+  a.ce_cfg = GEMM_BIG;
+  double bt = 0;
+  for (int cfg : {GEMM_BIG, GEMM_WIDE, GEMM_MID, GEMM_NARROW}) {
+    const double c = gemm_cost(a.n, a.vchunk, a.D, 2.0, cfg, 1);
+    if (bt == 0 || c < bt) {
+      bt = c;
+      a.ce_cfg = cfg;
+    }
+  }
+  a.ce_bn = ce_run(a.ce_cfg);
+  a.ntn = (a.V + a.ce_bn - 1) / a.ce_bn;
+  // The dH product's tile and K slices, the same for every chunk. A split
+  // keeps one fp32 accumulator per slice across the chunks (read and written
+  // by the product's epilogue) and the finalize adds the slices once, so a
+  // chunk has no reduction launch: 8 bytes per slice's element and a share of
+  // that one pass. 504 rows × 1024, K = 16384: 48 + 7.5 µs (256×256 tiles in 8
+  // slices, 64 blocks, and a reduction per chunk) → 30 µs (128×128 in 8, 256
+  // blocks); 256 rows × 5120: 55 + 13.7 → 48 µs.
+  a.dh_cfg = gemm_cfg >= 0 ? gemm_cfg : GEMM_BIG;
+  a.dh_ks = 1;
+  if (gemm_cfg >= 0) return;
+  bt = 0;
+  const int nk = (a.vchunk + 63) / 64, nch = head_num_chunks(a);
+  for (int cfg = 0; cfg < kGemmCfgs; ++cfg) {
+    const GemmTile t = gemm_tile(cfg);
+    const long tiles = (long)((a.n + t.bm - 1) / t.bm) * ((a.D + t.bn - 1) / t.bn);
+    for (int ks = 1; ks <= (can_split && a.D % 8 == 0 ? std::min(16, nk / 3) : 1); ++ks) {
+      if (ks > 1 && tiles * ks > 256 * t.occ) break;
+      // ks blocks per tile run as ks · tiles plain ones of a K / ks product
+      // whose epilogue reads and writes the accumulator
+      double c = gemm_cost(a.n, a.D, (nk + ks - 1) / ks * 64, 0.0, cfg, 1);
+      const double blocks = (double)tiles * ks;
+      if (ks > 1) {
+        const double steps = (nk + ks - 1) / ks, operands = 2.0 * a.vchunk * ((double)a.n + a.D);
+        c = 5.0 + std::max(std::ceil(blocks / 256) * steps * t.step + 0.5, operands / 6.8e6) +
+            4.0 * ks * a.n * a.D / 3.9e6 / nch;
+      }
+      c += std::ceil(blocks / 256) * t.bm * t.bn * 8.0 * std::min(blocks, 256.0) / 7.8e6;
+      if (bt == 0 || c < bt) {
+        bt = c;
+        a.dh_cfg = cfg;
+        a.dh_ks = ks;
+      }
+    }
+  }
+}
+
+long head_part_elems(const HeadArgs& a) { return gemm_part_elems(a.n, a.D, a.dh_ks); }
+
+hipError_t head_init(const HeadArgs& a, hipStream_t s) {
+  if (a.n <= 0) return hipSuccess;
+  hipLaunchKernelGGL(ce_init_kernel, dim3((a.n + 3) / 4), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t head_prob(const HeadArgs& a, int c0, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
   const int Vc = min(a.vchunk, a.V - c0), Nc8 = (Vc + 7) / 8 * 8;
-  EpiCEProb epi{a.labels, a.stats, a.ntn, a.tgt_logit, a.dlog, (long)a.vchunk, c0, Vc, Nc8,
-                c0 > 0 ? a.run_m : nullptr};
-  if (a.ce_bn == 128) return launch_gemm_cfg<256, 128, 2, 2>(chunk_logits_problem(a, c0), epi, s);
-  return launch_gemm_cfg<256, CE_BN, 2, 2>(chunk_logits_problem(a, c0), epi, s);
+  EpiCEProb epi{a.stats, a.ntn, a.dlog, (long)a.vchunk, c0, Vc, Nc8, a.run_m};
+  const GemmProblem p = chunk_logits_problem(a, c0);
+  switch (a.ce_cfg) {
+    case GEMM_BIG: return launch_gemm_cfg<256, 256, 2, 2, 2, 3>(p, epi, s);
+    case GEMM_WIDE: return launch_gemm_cfg<256, 128, 2, 2, 3, 3>(p, epi, s);
+    case GEMM_MID: return launch_gemm_cfg<128, 128, 2, 2, 2, 3>(p, epi, s);
+    case GEMM_NARROW: return launch_gemm_cfg<128, 64, 2, 2, 3, 3>(p, epi, s);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t head_rescale(const HeadArgs& a, int c0, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(ce_rescale_kernel, dim3((a.n + 3) / 4), dim3(256), 0, s, a, c0,
-                     c0 == 0 ? 1 : 0);
+  hipLaunchKernelGGL(ce_rescale_kernel, dim3((a.n + 3) / 4), dim3(256), 0, s, a, c0);
   return hipGetLastError();
 }
 
 hipError_t head_finalize(const HeadArgs& a, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(ce_finalize_kernel, dim3((a.n + 3) / 4), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(ce_finalize_kernel, dim3((a.n + 3) / 4), dim3(256), 0, s, a, a.dh_ks);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(ce_loss_kernel, dim3(1), dim3(1024), 0, s, a.loss_row, a.n, a.n_dev,
@@ -325,24 +381,16 @@ hipError_t head_finalize(const HeadArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
-GemmPlan head_dh_plan(const HeadArgs& a, int c0) {
-  if (a.gemm_cfg >= 0) return GemmPlan{a.gemm_cfg, 1};
-  const int Nc8 = (min(a.vchunk, a.V - c0) + 7) / 8 * 8;
-  GemmPlan pl = gemm_plan(a.n, a.D, Nc8, 8.0, a.part != nullptr);
-  if (gemm_part_elems(a.n, a.D, pl.ks) > a.part_elems) pl = gemm_plan(a.n, a.D, Nc8, 8.0, false);
-  return pl;
-}
-
 int head_dh_tail(const HeadArgs& a, int c0, int* tail) {
   *tail = 0;
-  const GemmPlan pl = head_dh_plan(a, c0);
-  if (a.gemm_cfg >= 0 || !a.part || pl.ks > 1 || pl.cfg != GEMM_BIG) return 1;
+  if (!a.tail_part || a.dh_ks > 1 || a.dh_cfg != GEMM_BIG) return 1;
   const int Nc8 = (min(a.vchunk, a.V - c0) + 7) / 8 * 8;
   const int kt = gemm_tail_split(a.n, a.D, Nc8, a.ncu, tail);
-  return kt > 1 && (long)kt * *tail * 65536 <= a.part_elems ? kt : 1;
+  return kt > 1 && (long)kt * *tail * 65536 <= a.tail_elems ? kt : 1;
 }
 
 hipError_t head_chunk_dh(const HeadArgs& a, int c0, hipStream_t s) {
+  if (a.n <= 0) return hipSuccess;
   const int Nc8 = (min(a.vchunk, a.V - c0) + 7) / 8 * 8;
   // dH = dH·α + P[:, chunk] · W[chunk, :]: the head read in place as the
   // [K, N] operand, rows past the vocabulary loading as zeros
@@ -351,20 +399,25 @@ hipError_t head_chunk_dh(const HeadArgs& a, int c0, hipStream_t s) {
   q.b_kn = 1;
   q.kb_rows = min(a.vchunk, a.V - c0);
   EpiF32 ef{a.dH, (long)a.D, a.D, c0 > 0 ? 1 : 0, a.alpha};
-  const GemmPlan pl = head_dh_plan(a, c0);
-  if (pl.ks > 1) {
+  if (a.dh_ks > 1) {
+    // each K slice accumulates its own partial; a slice past a short last
+    // chunk's K only applies α
+    if (!a.part || a.D % 8) return hipErrorInvalidValue;
     q.part = a.part;
-    return launch_gemm_split(q, ef, pl, s);
+    q.part_acc = c0 > 0 ? 1 : 0;
+    q.part_scale = a.alpha;
+    return launch_gemm(q, ef, s, a.dh_cfg, a.dh_ks);
   }
   int tail = 0;
   const int kt = head_dh_tail(a, c0, &tail);
-  if (kt > 1) return launch_gemm_tail(q, ef, kt, tail, a.part, s);
-  return launch_gemm(q, ef, s, pl.cfg);
+  if (kt > 1) return launch_gemm_tail(q, ef, kt, tail, a.tail_part, s);
+  return launch_gemm(q, ef, s, a.dh_cfg);
 }
 
 hipError_t head_fwd_bwd(const HeadArgs& a, hipStream_t s) {
   hipError_t e;
   if (a.n <= 0) return hipSuccess;
+  if ((e = head_init(a, s)) != hipSuccess) return e;
   for (int c0 = 0; c0 < a.V; c0 += a.vchunk) {
     if ((e = head_prob(a, c0, s)) != hipSuccess) return e;
     if ((e = head_rescale(a, c0, s)) != hipSuccess) return e;

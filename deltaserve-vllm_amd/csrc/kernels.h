@@ -164,15 +164,19 @@ bool lora_dual_supported(int R1, int R2, int C);
 struct HeadArgs {
   const bf16* normed; long ldh;   // [n, D]
   const bf16* W;                  // [V, D]
-  const int* labels;              // [n] target id or -1
+  const int64_t* ids;             // [n] token ids
+  const int* pred;                // [n] 1 where row t predicts ids[t + 1]
+  int* err;                       // bit 1: a target id outside [0, V)
+  int* labels;                    // [n] target id or -1 (head_init)
   int n; const int* n_dev;
   int D, V;
-  float2* stats;                  // [n_cap, ntn] per vocab tile (max, sum exp)
+  float2* stats;                  // [n_cap, ntn] per run of ce_bn columns (reference, sum exp)
   int ntn;                        // ceil(V / ce_bn)
-  int ce_bn = 256;                // vocab tile width of the CE passes (256 or 128)
+  int ce_bn, ce_cfg;              // run width and tile of the logits product (head_plan)
+  int dh_cfg, dh_ks;              // tile and K slices of the dH product (head_plan)
   float* tgt_logit;               // [n_cap]
   float* lse;                     // [n_cap] row LSE (natural log), after the last chunk
-  float* run_m;                   // [n_cap] running row max across chunks
+  float* run_m;                   // [n_cap] the row's softmax reference M
   float* run_l;                   // [n_cap] running Σ exp(logit − run_m)
   float* alpha;                   // [n_cap] the dH accumulator's factor for the chunk
   float* loss_row;                // [n_cap]
@@ -181,24 +185,29 @@ struct HeadArgs {
   bf16* dlog; int vchunk;         // [n_cap, vchunk] bf16 probabilities of one vocab
                                   // chunk; vchunk a multiple of 256
   float* dH;                      // [n, D] fp32
-  int gemm_cfg;                   // tile of the dH product (-1: by shape)
-  float* part = nullptr;          // split-K partials for the dH product (null: no split)
-  long part_elems = 0;
-  int ncu = 0;                    // compute units (tail split of the dH product; 0: none)
+  // head_part_elems floats when dh_ks > 1: the dH product's accumulators, one
+  // per K slice, live from the first chunk to the finalize
+  float* part = nullptr;
+  float* tail_part = nullptr;     // partials of a tail split of the dH product (null: none)
+  long tail_elems = 0;
+  int ncu = 0;                    // compute units (tail split; 0: none)
 };
-// Chunk c0 (a multiple of vchunk): head_prob (logits, tile statistics and
-// probabilities), head_rescale (online-softmax reference), head_chunk_dh
-// (dH·α + P·W); head_finalize after the last chunk (dH, LSE, loss).
+// Tiles, K slices and the statistics' layout for a's n, D, V and vchunk
+// (gemm_cfg: forced tile of the dH product, -1 by cost; can_split: a.part will
+// be provided); then head_init (after
+// the final norm), per chunk c0 (a multiple of vchunk) head_prob (logits,
+// statistics and probabilities), head_rescale (softmax reference) and
+// head_chunk_dh (dH·α + P·W), and head_finalize after the last (dH, LSE, loss).
+void head_plan(HeadArgs& a, int gemm_cfg, bool can_split);
+long head_part_elems(const HeadArgs& a);
 int head_num_chunks(const HeadArgs& a);
 hipError_t head_fwd_bwd(const HeadArgs& a, hipStream_t s);
+hipError_t head_init(const HeadArgs& a, hipStream_t s);
 hipError_t head_prob(const HeadArgs& a, int c0, hipStream_t s);
 hipError_t head_rescale(const HeadArgs& a, int c0, hipStream_t s);
 hipError_t head_chunk_dh(const HeadArgs& a, int c0, hipStream_t s);
 hipError_t head_finalize(const HeadArgs& a, hipStream_t s);
-// the tile and K slices head_chunk_dh uses for chunk c0, and the K splits over
-// the tiles of its partly filled last round (1: none)
-struct GemmPlan;
-GemmPlan head_dh_plan(const HeadArgs& a, int c0);
+// K splits over the tiles of the dH product's partly filled last round (1: none)
 int head_dh_tail(const HeadArgs& a, int c0, int* tail);
 
 // ---- optim.hip
@@ -223,9 +232,5 @@ hipError_t save_rows(const void* x, long ldx, const void* r, long ldr, long x_ro
                      long ldbuf, long buf_rows, hipStream_t s);
 hipError_t save_ids(const int64_t* ids, long ids_len, const int64_t* src, const int64_t* dst, int count,
                     int64_t* out, long out_len, hipStream_t s);
-
-// ---- misc (dsb_api.hip)
-hipError_t build_labels(const int64_t* ids, const int* pred_flag, int* labels, int n,
-                        const int* n_dev, int V, int* err, hipStream_t s);
 
 }  // namespace dsb

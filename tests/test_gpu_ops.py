@@ -485,3 +485,38 @@ def test_gemm_glu_tiles(M, I, K, K2):
     want = (g * torch.sigmoid(g) * u).to(torch.bfloat16)
     # bf16 rounding of the same fp32 value: at most one ulp apart
     assert ((H.float() - want.float()).abs() <= want.float().abs() * 2 ** -7 + 1e-30).all()
+
+
+@pytest.mark.parametrize("n,V,vchunk,std", [(40, 700, 256, 6.0), (300, 2100, 512, 40.0),
+                                            (300, 2100, 0, 0.0), (700, 4100, 1024, 6.0)])
+def test_head_reference_moves(n, V, vchunk, std):
+    """Rows whose target logit lies far below the row maximum (logit spread
+    `std` nats, up to a few hundred: runs past the softmax reference's limit
+    in the first, a middle or the last chunk) beside rows where it is the
+    maximum, and all-equal logits (std 0): loss and dH against fp64. A run's
+    probabilities are bf16 (2^-9 relative), so dH is within 1e-2 of its largest
+    value as in test_head; the loss is fp32 sums of exponentials."""
+    from deltaserve_amd import ops
+    D = 256
+    seq_lens = [n - n // 3, n // 3]
+    x = _bf(_rnd(n, D, seed=81))
+    W = _bf(_rnd(V, D, seed=82) * (std / math.sqrt(D)))
+    ids = torch.randint(0, V, (n,), generator=torch.Generator().manual_seed(83))
+    logits = x.double() @ W.double().t()
+    ids[1:n // 2] = logits[:n // 2 - 1].argmax(1)   # targets at the maximum
+    loss, nv, dH = ops.head_backward(x.to(DEV), W.to(DEV), ids.to(DEV), seq_lens, vocab_chunk=vchunk)
+    _, _, rows, tgt, n_valid = O.pack(seq_lens)
+    lg = logits[rows]
+    ref_loss = (torch.logsumexp(lg, 1) - lg[torch.arange(n_valid), ids[tgt]]).mean().item()
+    p = torch.softmax(lg, 1)
+    p[torch.arange(n_valid), ids[tgt]] -= 1
+    ref = torch.zeros(n, D, dtype=torch.float64)
+    ref[rows] = (p @ W.double()) / n_valid
+    assert nv == n_valid
+    assert abs(loss - ref_loss) < 1e-4 * ref_loss
+    assert torch.isfinite(dH).all()
+    if std:
+        assert max_rel(dH, ref.float()) < 1e-2
+        assert cosine(dH, ref.float()) > 0.9999
+    else:
+        assert dH.abs().max().item() == 0.0
