@@ -26,6 +26,7 @@
 #include "../../include/dsb.h"
 #include "gemm_nt.h"
 #include "kernels.h"
+#include "workspace.h"
 
 namespace dsb {
 
@@ -2001,48 +2002,39 @@ int dsb_op_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, const vo
   GemmProblem p{(const bf16*)A, lda, (const bf16*)B, ldb, (const bf16*)A2, lda2,
                 (const bf16*)B2, ldb2, M, N, K1, K2, nullptr};
   p.b_kn = b_kn ? 1 : 0;
-  // cfg -2: split K as the cycle does for problems with too few 256-wide
-  // tiles; cfg -3: split K over the tiles of a partly filled last round, as
-  // the cycle does (partials in a buffer allocated for the call); by shape
-  // otherwise
-  if (cfg == -3) {
-    int dev = 0, ncu = 0, tail = 0;
+  const double ob = out_f32 ? (accumulate ? 8.0 : 4.0) : (R ? 4.0 : 2.0);
+  // -1 and -2: the cycle's tile and K split; -3: a K split over the tiles of a
+  // partly filled last round
+  GemmPlan pl = cfg >= 0    ? GemmPlan{cfg, 1}
+                : cfg == -3 ? GemmPlan{GEMM_BIG, 1}
+                            : gemm_plan(M, N, K1 + K2, ob, true);
+  int kt = 1, tail = 0;
+  if (cfg < 0 && pl.ks == 1 && pl.cfg == GEMM_BIG) {
+    int dev = 0, ncu = 0;
     OPCK(hipGetDevice(&dev));
     OPCK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    const int kt = gemm_tail_split(M, N, K1 + K2, ncu, &tail);
-    if (kt > 1) {
-      float* tp = nullptr;
-      OPCK(hipMalloc((void**)&tp, sizeof(float) * (size_t)kt * tail * 65536));
-      hipError_t e1;
-      if (out_f32) e1 = launch_gemm_tail(p, EpiF32{(float*)C, ldc, N, accumulate}, kt, tail, tp, s);
-      else e1 = launch_gemm_tail(p, EpiBF16{(bf16*)C, ldc, N, (const bf16*)R, ldr}, kt, tail, tp, s);
-      const hipError_t e2 = e1 == hipSuccess ? hipStreamSynchronize(s) : e1;
-      (void)hipFree(tp);
-      OPCK(e2);
-      return 0;
+    kt = gemm_tail_split(M, N, K1 + K2, ncu, &tail);
+    if (cfg == -3 && kt == 1) pl = gemm_plan(M, N, K1 + K2, ob, false);
+  }
+  Scratch tmp(s);
+  float* part = nullptr;
+  if (pl.ks > 1 || kt > 1) {
+    part = tmp.dev<float>(pl.ks > 1 ? gemm_part_elems(M, N, pl.ks) : (size_t)kt * tail * 65536);
+    if (!part) return fail(nullptr, "dsb_op_gemm: hipMalloc failed");
+  }
+  auto run = [&](const auto& e) {
+    if (kt > 1) return launch_gemm_tail(p, e, kt, tail, part, s);
+    if (pl.ks > 1) {
+      p.part = part;
+      return launch_gemm_split(p, e, pl, s);
     }
-    cfg = -1;
-  }
-  const double ob = out_f32 ? (accumulate ? 8.0 : 4.0) : (R ? 4.0 : 2.0);
-  const GemmPlan pl = cfg >= 0 ? GemmPlan{cfg, 1} : gemm_plan(M, N, K1 + K2, ob, cfg == -2);
-  if (pl.ks > 1) {
-    OPCK(hipMalloc((void**)&p.part, sizeof(float) * (size_t)gemm_part_elems(M, N, pl.ks)));
-    hipError_t e1;
-    if (out_f32) e1 = launch_gemm_split(p, EpiF32{(float*)C, ldc, N, accumulate}, pl, s);
-    else e1 = launch_gemm_split(p, EpiBF16{(bf16*)C, ldc, N, (const bf16*)R, ldr}, pl, s);
-    const hipError_t e2 = e1 == hipSuccess ? hipStreamSynchronize(s) : e1;
-    (void)hipFree(p.part);
-    OPCK(e2);
-    return 0;
-  }
-  if (out_f32) {
-    EpiF32 e{(float*)C, ldc, N, accumulate};
-    OPCK(launch_gemm(p, e, s, pl.cfg));
-  } else {
-    EpiBF16 e{(bf16*)C, ldc, N, (const bf16*)R, ldr};
-    OPCK(launch_gemm(p, e, s, pl.cfg));
-  }
-  OPCK(hipStreamSynchronize(s));
+    return launch_gemm(p, e, s, pl.cfg);
+  };
+  if (out_f32)
+    OPCK(run(EpiF32{(float*)C, ldc, N, accumulate}));
+  else
+    OPCK(run(EpiBF16{(bf16*)C, ldc, N, (const bf16*)R, ldr}));
+  OPCK(tmp.finish());
   return 0;
 }
 
@@ -2121,21 +2113,10 @@ int dsb_op_rope_bwd(void* g, int64_t ldg, const void* qkv_pre, int64_t ldp, cons
 }  // extern "C"
 
 namespace {
-struct TmpDev {
-  std::vector<void*> ptrs;
-  ~TmpDev() {
-    for (void* p : ptrs) (void)hipFree(p);
-  }
-  template <class T>
-  T* alloc(size_t count) {
-    void* p = nullptr;
-    if (hipMalloc(&p, count * sizeof(T) + 256) != hipSuccess) return nullptr;
-    ptrs.push_back(p);
-    return (T*)p;
-  }
-};
-
-int attn_setup(const int32_t* seq_lens, int nseq, TmpDev& tmp, AttnArgs& a, int* n_out) {
+// The attention tables of a packing (tiles in query and key order, tile and
+// row counts), one staged copy on the call's stream.
+int attn_setup(const int32_t* seq_lens, int nseq, Scratch& tmp, hipStream_t s, AttnArgs& a,
+               int* n_out) {
   std::vector<int4> tiles;
   long n = 0;
   for (int i = 0; i < nseq; ++i) n += seq_lens[i];
@@ -2143,22 +2124,20 @@ int attn_setup(const int32_t* seq_lens, int nseq, TmpDev& tmp, AttnArgs& a, int*
     return fail(nullptr, "attention: bad seq_lens");
   std::vector<int4> by_q, by_k;
   order_tiles(tiles, by_q, by_k);
-  int4* dt = tmp.alloc<int4>(2 * tiles.size() + 2);
-  int* dn = tmp.alloc<int>(2);
-  if (!dt || !dn) return fail(nullptr, "attention: hipMalloc failed");
-  int hv[2] = {(int)tiles.size(), (int)n};
-  if (!tiles.empty() &&
-      (hipMemcpy(dt, by_q.data(), by_q.size() * sizeof(int4), hipMemcpyHostToDevice) != hipSuccess ||
-       hipMemcpy(dt + tiles.size(), by_k.data(), by_k.size() * sizeof(int4),
-                 hipMemcpyHostToDevice) != hipSuccess))
-    return fail(nullptr, "attention: copy failed");
-  if (hipMemcpy(dn, hv, sizeof(hv), hipMemcpyHostToDevice) != hipSuccess)
+  const size_t nt = tiles.size();
+  int4* dt = tmp.dev<int4>(2 * nt + 1);
+  int4* ht = tmp.host<int4>(2 * nt + 1);
+  if (!dt || !ht) return fail(nullptr, "attention: hipMalloc failed");
+  std::copy(by_q.begin(), by_q.end(), ht);
+  std::copy(by_k.begin(), by_k.end(), ht + nt);
+  ht[2 * nt] = int4{(int)nt, (int)n, 0, 0};
+  if (hipMemcpyAsync(dt, ht, (2 * nt + 1) * sizeof(int4), hipMemcpyHostToDevice, s) != hipSuccess)
     return fail(nullptr, "attention: copy failed");
   a.tiles = dt;
-  a.tiles_k = dt + tiles.size();
-  a.ntiles_dev = dn;
-  a.max_tiles = (int)tiles.size();
-  a.n_dev = dn + 1;
+  a.tiles_k = dt + nt;
+  a.ntiles_dev = reinterpret_cast<const int*>(dt + 2 * nt);
+  a.max_tiles = (int)nt;
+  a.n_dev = a.ntiles_dev + 1;
   a.n = (int)n;
   *n_out = (int)n;
   return 0;
@@ -2174,16 +2153,16 @@ int dsb_op_attn_fwd(const void* q, int64_t ldq, const void* k, int64_t ldk, cons
   if (Hq <= 0 || Hkv <= 0 || Hq % Hkv) return fail(nullptr, "attn: bad head counts");
   if (head_dim != 128 && head_dim != 64) return fail(nullptr, "attn: head_dim 128 or 64");
   hipStream_t s = (hipStream_t)stream;
-  TmpDev tmp;
+  Scratch tmp(s);
   AttnArgs a{};
   int n = 0;
-  if (attn_setup(seq_lens, nseq, tmp, a, &n)) return -1;
+  if (attn_setup(seq_lens, nseq, tmp, s, a, &n)) return -1;
   a.q = (const bf16*)q; a.ldq = ldq; a.k = (const bf16*)k; a.ldk = ldk;
   a.v = (const bf16*)v; a.ldv = ldv; a.ctx = (bf16*)ctx; a.ldc = ldc;
   a.o32 = o32; a.ldo32 = (long)Hq * head_dim; a.lse = lse; a.ld_stat = n; a.Hq = Hq; a.Hkv = Hkv;
   a.hd = head_dim; a.scale = 1.f / std::sqrt((float)head_dim);
   OPCK(attn_fwd(a, s));
-  OPCK(hipStreamSynchronize(s));
+  OPCK(tmp.finish());
   return 0;
 }
 
@@ -2199,11 +2178,11 @@ int dsb_op_attn_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, cons
       (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)dout | (uintptr_t)o32) & 15))
     return fail(nullptr, "attn: rows must be 16-byte aligned (ld multiple of 8)");
   hipStream_t s = (hipStream_t)stream;
-  TmpDev tmp;
+  Scratch tmp(s);
   AttnArgs a{};
   int n = 0;
-  if (attn_setup(seq_lens, nseq, tmp, a, &n)) return -1;
-  float* dsum = tmp.alloc<float>((size_t)Hq * (n + 1));
+  if (attn_setup(seq_lens, nseq, tmp, s, a, &n)) return -1;
+  float* dsum = tmp.dev<float>((size_t)Hq * (n + 1));
   if (!dsum) return fail(nullptr, "attn: hipMalloc failed");
   a.q = (const bf16*)q; a.ldq = ldq; a.k = (const bf16*)k; a.ldk = ldk;
   a.v = (const bf16*)v; a.ldv = ldv; a.o32 = (float*)o32; a.ldo32 = (long)Hq * head_dim;
@@ -2211,15 +2190,14 @@ int dsb_op_attn_bwd(const void* q, int64_t ldq, const void* k, int64_t ldk, cons
   a.lse = (float*)lse; a.dsum = dsum; a.ld_stat = n; a.dout = (const bf16*)dout; a.lddo = lddo;
   a.dq = (bf16*)dq; a.lddq = lddq; a.dk = (bf16*)dk; a.lddk = lddk; a.dv = (bf16*)dv;
   a.lddv = lddv; a.Hq = Hq; a.Hkv = Hkv;
-  // the dK/dV head split the cycle takes for short token counts, partials in
-  // a buffer allocated for the call
+  // the dK/dV head split the cycle takes for short token counts
   a.kv_part_elems = (long)(Hq / Hkv) * n * 2 * Hkv * head_dim;
   if (attn_dkdv_head_split(a) > 1) {
-    a.kv_part = tmp.alloc<float>((size_t)a.kv_part_elems);
+    a.kv_part = tmp.dev<float>((size_t)a.kv_part_elems);
     if (!a.kv_part) return fail(nullptr, "attn: hipMalloc failed");
   }
   OPCK(attn_bwd(a, s));
-  OPCK(hipStreamSynchronize(s));
+  OPCK(tmp.finish());
   return 0;
 }
 
@@ -2230,38 +2208,54 @@ int dsb_op_head(const void* normed, int64_t ldh, const void* lm_w, const int64_t
     return fail(nullptr, "dsb_op_head: D and ldh multiples of 8, V positive, vocab_chunk a "
                          "multiple of 256");
   hipStream_t s = (hipStream_t)stream;
-  std::vector<int32_t> pred(n > 0 ? n : 1);
-  const int nv = pack_cycle(seq_lens, nseq, n, nullptr, pred.data(), nullptr);
+  Scratch tmp(s);
+  // staged: the prediction flags, then {1/n_valid, loss, ids' error flag}
+  struct Result {
+    float inv_nvalid, loss;
+    int err, pad;
+  };
+  const size_t off = ((size_t)n * sizeof(int) + 15) / 16 * 16;
+  char* hs = tmp.host<char>(off + sizeof(Result));
+  char* ds = tmp.dev<char>(off + sizeof(Result));
+  if (!hs || !ds) return fail(nullptr, "dsb_op_head: hipMalloc failed");
+  const int nv = pack_cycle(seq_lens, nseq, n, nullptr, (int32_t*)hs, nullptr);
   if (nv < 0) return fail(nullptr, "dsb_op_head: seq_lens must sum to n");
-  TmpDev tmp;
+  Result* hr = reinterpret_cast<Result*>(hs + off);
+  Result* dr = reinterpret_cast<Result*>(ds + off);
+  *hr = Result{nv > 0 ? 1.f / nv : 0.f, 0.f, 0, 0};
   HeadArgs a{};
   a.n = n; a.D = D; a.V = V;
   a.vchunk = std::min(vocab_chunk > 0 ? vocab_chunk : 16384, ((V + 255) / 256) * 256);
-  head_plan(a, -1, false);
-  int* dpred = tmp.alloc<int>(n + 1);
-  int* err = tmp.alloc<int>(1);
-  float* scal = tmp.alloc<float>(4);
-  a.labels = tmp.alloc<int>(n + 1);
-  a.stats = tmp.alloc<float2>((size_t)(n + 1) * a.ntn);
-  for (float** p : {&a.tgt_logit, &a.lse, &a.loss_row, &a.run_m, &a.run_l, &a.alpha})
-    if (!(*p = tmp.alloc<float>(n + 1))) return fail(nullptr, "dsb_op_head: hipMalloc failed");
-  a.dlog = tmp.alloc<bf16>((size_t)(n + 1) * a.vchunk);
-  if (!dpred || !err || !scal || !a.labels || !a.stats || !a.dlog)
+  head_plan(a, -1, true);
+  const long NN = n + 1;
+  a.labels = tmp.dev<int>(NN);
+  a.stats = tmp.dev<float2>(NN * a.ntn);
+  float* rows = tmp.dev<float>(6 * NN);
+  a.dlog = tmp.dev<bf16>(NN * a.vchunk);
+  int tail = 0;
+  if (a.dh_ks == 1 && a.dh_cfg == GEMM_BIG) {
+    int dev = 0;
+    OPCK(hipGetDevice(&dev));
+    OPCK(hipDeviceGetAttribute(&a.ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    const int kt = gemm_tail_split(n, D, a.vchunk, a.ncu, &tail);
+    a.tail_elems = kt > 1 ? (long)kt * tail * 65536 : 0;
+  }
+  if (a.dh_ks > 1) a.part = tmp.dev<float>((size_t)head_part_elems(a));
+  if (a.tail_elems > 0) a.tail_part = tmp.dev<float>((size_t)a.tail_elems);
+  if (!a.labels || !a.stats || !rows || !a.dlog || (a.dh_ks > 1 && !a.part) ||
+      (a.tail_elems > 0 && !a.tail_part))
     return fail(nullptr, "dsb_op_head: hipMalloc failed");
-  float hsc[4] = {nv > 0 ? 1.f / nv : 0.f, 0.f, 0.f, 0.f};
-  OPCK(hipMemcpy(scal, hsc, sizeof(hsc), hipMemcpyHostToDevice));
-  if (n > 0) OPCK(hipMemcpy(dpred, pred.data(), n * sizeof(int32_t), hipMemcpyHostToDevice));
-  OPCK(hipMemset(err, 0, sizeof(int)));
+  a.tgt_logit = rows; a.lse = rows + NN; a.loss_row = rows + 2 * NN;
+  a.run_m = rows + 3 * NN; a.run_l = rows + 4 * NN; a.alpha = rows + 5 * NN;
   a.normed = (const bf16*)normed; a.ldh = ldh; a.W = (const bf16*)lm_w;
-  a.ids = ids; a.pred = dpred; a.err = err; a.n_dev = nullptr;
-  a.loss_out = scal + 1; a.inv_nvalid = scal; a.dH = dH;
+  a.ids = ids; a.pred = (const int*)ds; a.err = &dr->err; a.n_dev = nullptr;
+  a.loss_out = &dr->loss; a.inv_nvalid = &dr->inv_nvalid; a.dH = dH;
+  OPCK(hipMemcpyAsync(ds, hs, off + sizeof(Result), hipMemcpyHostToDevice, s));
   OPCK(head_fwd_bwd(a, s));
-  OPCK(hipStreamSynchronize(s));
-  int herr = 0;
-  OPCK(hipMemcpy(&herr, err, sizeof(int), hipMemcpyDeviceToHost));
-  if (herr) return fail(nullptr, "dsb_op_head: a target token id is outside [0, vocab)");
-  OPCK(hipMemcpy(hsc, scal, sizeof(hsc), hipMemcpyDeviceToHost));
-  if (loss) *loss = hsc[1];
+  OPCK(hipMemcpyAsync(hr, dr, sizeof(Result), hipMemcpyDeviceToHost, s));
+  OPCK(tmp.finish());
+  if (hr->err) return fail(nullptr, "dsb_op_head: a target token id is outside [0, vocab)");
+  if (loss) *loss = hr->loss;
   if (n_valid) *n_valid = nv;
   return 0;
 }
@@ -2272,16 +2266,16 @@ int dsb_op_lora_tn(const void* P, int64_t ldp, const void* X, int64_t ldx, int n
   if (C % 8 || ldx % 8 || rg <= 0 || (R + rg - 1) / rg > 3)
     return fail(nullptr, "dsb_op_lora_tn: C and ldx must be multiples of 8, at most 3 groups");
   hipStream_t s = (hipStream_t)stream;
-  TmpDev tmp;
+  Scratch tmp(s);
   const int ns = 8;
-  float* work = tmp.alloc<float>((size_t)ns * R * C);
+  float* work = tmp.dev<float>((size_t)ns * R * C);
   if (!work) return fail(nullptr, "dsb_op_lora_tn: hipMalloc failed");
   TnArgs a{};
   a.P = (const bf16*)P; a.ldp = ldp; a.X = (const bf16*)X; a.ldx = ldx; a.R = R; a.C = C; a.n = n;
   a.n_dev = nullptr; a.work = work; a.nsplit = ns; a.outs[0] = out0; a.outs[1] = out1;
   a.outs[2] = out2; a.rg = rg; a.transpose_out = transpose_out; a.scale = scale;
   OPCK(lora_tn(a, s));
-  OPCK(hipStreamSynchronize(s));
+  OPCK(tmp.finish());
   return 0;
 }
 
@@ -2290,16 +2284,15 @@ int dsb_op_lora_skinny(const void* X, int64_t ldx, const void* B, int64_t ldb, i
   if (K % 8 || ldx % 8 || ldb % 8) return fail(nullptr, "dsb_op_lora_skinny: K, ldx, ldb must be multiples of 8");
   hipStream_t s = (hipStream_t)stream;
   SkinnyArgs a{(const bf16*)X, ldx, (const bf16*)B, ldb, R, K, (bf16*)Z, ldz, n, nullptr};
-  // the K split the cycle takes for short token ranges, partials in a buffer
-  // allocated for the call
-  TmpDev tmp;
+  // the K split the cycle takes for short token ranges
+  Scratch tmp(s);
   a.part_elems = 8L * n * R;
   if (lora_skinny_split(a) > 1) {
-    a.part = tmp.alloc<float>((size_t)a.part_elems);
+    a.part = tmp.dev<float>((size_t)a.part_elems);
     if (!a.part) return fail(nullptr, "dsb_op_lora_skinny: hipMalloc failed");
   }
   OPCK(lora_skinny(a, s));
-  OPCK(hipStreamSynchronize(s));
+  OPCK(tmp.finish());
   return 0;
 }
 
@@ -2421,18 +2414,31 @@ int dsb_op_lora_dual(const dsb_dual_pass* passes, int count, int n, int n_alloc,
     return -1;
   if (n == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
-  TmpDev tmp;
-  float* work = tmp.alloc<float>((size_t)elems);
-  int* nd = tmp.alloc<int>(1);
-  if (!work || !nd) return fail(nullptr, "dsb_op_lora_dual: hipMalloc failed");
-  OPCK(hipMemcpy(nd, &n, sizeof(int), hipMemcpyHostToDevice));
+  Scratch tmp(s);
+  float* work = tmp.dev<float>((size_t)elems);
+  int* nd = tmp.dev<int>(1);
+  int* nh = tmp.host<int>(1);
+  if (!work || !nd || !nh) return fail(nullptr, "dsb_op_lora_dual: hipMalloc failed");
+  *nh = n;
+  OPCK(hipMemcpyAsync(nd, nh, sizeof(int), hipMemcpyHostToDevice, s));
   for (int i = 0; i < count; ++i) {
     a[i].work = work + reinterpret_cast<long>(a[i].work);
     a[i].n_dev = nd;
     a[i].n = n_alloc;  // grid sized for the capacity, live rows from the device
   }
   OPCK(lora_dual(a, count, s));
-  OPCK(hipStreamSynchronize(s));
+  OPCK(tmp.finish());
+  return 0;
+}
+
+int dsb_release_workspaces(void) {
+  pinned_pool().trim(0);
+  int cur = 0, n = 0;
+  if (hipGetDevice(&cur) != hipSuccess || hipGetDeviceCount(&n) != hipSuccess) {
+    (void)hipGetLastError();  // no device: nothing was ever kept on one
+    return 0;
+  }
+  for (int d = 0; d < std::min(n, kPoolDevices); ++d) device_pool(d).trim(0);
   return 0;
 }
 
@@ -2457,24 +2463,26 @@ int dsb_op_clip_adamw(float* const* w, float* const* g, float* const* m, float* 
   }
   for (int gidx = prev + 1; gidx < ngroups; ++gidx) lchunks[gidx] = int2{(int)chunks.size(), 0};
   hipStream_t s = (hipStream_t)stream;
-  TmpDev tmp;
-  OptTensor* dT = tmp.alloc<OptTensor>(T.size());
-  int2* dc = tmp.alloc<int2>(chunks.size() + 1);
-  int2* dl = tmp.alloc<int2>(lchunks.size());
-  float* part = tmp.alloc<float>(chunks.size() + 1);
-  float* sq = tmp.alloc<float>(ngroups);
-  OptHyper* hp = tmp.alloc<OptHyper>(1);
-  if (!dT || !dc || !dl || !part || !sq || !hp) return fail(nullptr, "dsb_op_clip_adamw: hipMalloc failed");
-  OptHyper hh{lr, beta1, beta2, eps, wd, (float)(1.0 - pow((double)beta1, (double)step)),
-              (float)(1.0 - pow((double)beta2, (double)step)), max_norm};
-  OPCK(hipMemcpy(dT, T.data(), T.size() * sizeof(OptTensor), hipMemcpyHostToDevice));
-  if (!chunks.empty())
-    OPCK(hipMemcpy(dc, chunks.data(), chunks.size() * sizeof(int2), hipMemcpyHostToDevice));
-  OPCK(hipMemcpy(dl, lchunks.data(), lchunks.size() * sizeof(int2), hipMemcpyHostToDevice));
-  OPCK(hipMemcpy(hp, &hh, sizeof(hh), hipMemcpyHostToDevice));
-  OPCK(hipMemset(sq, 0, ngroups * sizeof(float)));
-  OPCK(clip_adamw(dT, dc, (int)chunks.size(), dl, ngroups, part, sq, hp, do_clip, s));
-  OPCK(hipStreamSynchronize(s));
+  Scratch tmp(s);
+  // staged as one block: tensor table, chunk lists, hyperparameters
+  const size_t oc = T.size() * sizeof(OptTensor), ol = oc + chunks.size() * sizeof(int2),
+               oh = (ol + lchunks.size() * sizeof(int2) + 15) / 16 * 16,
+               total = oh + sizeof(OptHyper);
+  char* hs = tmp.host<char>(total);
+  char* ds = tmp.dev<char>(total);
+  float* part = tmp.dev<float>(chunks.size() + 1);
+  float* sq = tmp.dev<float>(ngroups);
+  if (!hs || !ds || !part || !sq) return fail(nullptr, "dsb_op_clip_adamw: hipMalloc failed");
+  const OptHyper hh{lr, beta1, beta2, eps, wd, (float)(1.0 - pow((double)beta1, (double)step)),
+                    (float)(1.0 - pow((double)beta2, (double)step)), max_norm};
+  memcpy(hs, T.data(), oc);
+  memcpy(hs + oc, chunks.data(), chunks.size() * sizeof(int2));
+  memcpy(hs + ol, lchunks.data(), lchunks.size() * sizeof(int2));
+  memcpy(hs + oh, &hh, sizeof(hh));
+  OPCK(hipMemcpyAsync(ds, hs, total, hipMemcpyHostToDevice, s));
+  OPCK(clip_adamw((const OptTensor*)ds, (const int2*)(ds + oc), (int)chunks.size(),
+                  (const int2*)(ds + ol), ngroups, part, sq, (const OptHyper*)(ds + oh), do_clip, s));
+  OPCK(tmp.finish());
   return 0;
 }
 

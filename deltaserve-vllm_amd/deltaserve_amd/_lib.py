@@ -109,6 +109,7 @@ _SIGS = {
                          POINTER(c_int32)]),
     "dsb_rope_inv_freq": (c_int, [c_int, c_float, c_int, c_float, c_float, c_float,
                                   c_float, POINTER(c_float)]),
+    "dsb_release_workspaces": (c_int, []),
     "dsb_op_gemm": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
                             c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p,
                             c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_int,

@@ -38,6 +38,12 @@ def _dev(*ts):
             raise ValueError("deltaserve_amd ops take CUDA (HIP) tensors")
 
 
+def release_workspaces():
+    """Free the scratch memory the ops keep between calls (the next call
+    allocates again)."""
+    L.check(L.load().dsb_release_workspaces(), what="dsb_release_workspaces")
+
+
 # ---------------------------------------------------------------- integer packing
 
 def pack(seq_lens):

@@ -254,15 +254,22 @@ int dsb_save_rows(const void* x, int64_t ldx, const void* r, int64_t ldr, int64_
 int dsb_save_ids(const int64_t* ids, int64_t ids_len, const int64_t* src, const int64_t* dst,
                  int count, int64_t* out, int64_t out_len, void* stream);
 
-/* ---- single-op entry points (parity tests; synchronous on `stream`) ---- */
+/* ---- single-op entry points (synchronous on `stream`) ----
+ *
+ * Their scratch memory comes from a pool per device that keeps up to 512 MiB
+ * between calls (and 16 MiB of pinned host memory in all); a block serves one
+ * call at a time. dsb_release_workspaces gives back what is kept and not in
+ * use by a running call. */
+int dsb_release_workspaces(void);
 
 /* C = A·Bᵀ (+ A2·B2ᵀ) [+ R]; out_f32 selects fp32 C (accumulate adds to C).
  * b_kn: B and B2 are stored [K, N] (a weight in its own [out, in] layout read
  * by the backward's C = dY·W; N a multiple of 8) instead of [N, K].
- * cfg: -1 tile by shape, 0/1/2 force 256/128/64-wide tiles, -2 split K over
- * the grid as the cycle does when the problem has too few 256-wide tiles,
- * -3 split K over the tiles of a partly filled last round of the device's
- * compute units, as the cycle does (plain launch when there is no such tail). */
+ * cfg: -1 (or -2) the tile and the K split the cycle would take for the shape
+ * (the least estimated time); 0/1/2 force 256/128/64-wide tiles, 3 a 256x128
+ * and 4 a 128x64 one, without a split; -3 256-wide tiles with K split over
+ * those of a partly filled last round of the device's compute units (plain
+ * launch when there is no such tail). */
 int dsb_op_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, const void* A2,
                 int64_t lda2, const void* B2, int64_t ldb2, int M, int N, int K1, int K2,
                 void* C, int64_t ldc, int out_f32, int accumulate, const void* R, int64_t ldr,
@@ -339,7 +346,7 @@ typedef struct dsb_dual_pass {
 /* 1 to 3 passes of rank r in {16, 32} over n rows in one launch (the cycle
  * batches q, k and v this way). The row count is read from device memory,
  * as in the cycle, and the token-split partials are laid out for n_alloc >= n
- * rows. Allocates its partial-sum workspace. */
+ * rows. */
 int dsb_op_lora_dual(const dsb_dual_pass* passes, int count, int n, int n_alloc, int r,
                      void* stream);
 /* dsb_op_lora_dual without any allocation, for callers that cannot call

@@ -520,3 +520,48 @@ def test_head_reference_moves(n, V, vchunk, std):
         assert cosine(dH, ref.float()) > 0.9999
     else:
         assert dH.abs().max().item() == 0.0
+
+
+@pytest.mark.parametrize("release", [False, True])
+def test_scratch_is_private_to_a_call(release):
+    """The ops' kept scratch memory: four threads on streams of their own run
+    ops of different sizes that need scratch (attention tables and dsum, head
+    buffers, split-K partials) over and over, some giving the kept blocks back
+    in between; every result equals the one of a lone call bit for bit."""
+    import threading
+
+    from deltaserve_amd import ops
+
+    def job(seed, lens, V):
+        n, Hq, Hkv = sum(lens), 4, 2
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16)  # noqa: E731
+        q, k, v, do = rnd(n, Hq * 128), rnd(n, Hkv * 128), rnd(n, Hkv * 128), rnd(n, Hq * 128)
+        W, ids = rnd(V, Hq * 128), torch.randint(0, V, (n,), generator=g, device=DEV)
+        torch.cuda.synchronize()
+
+        def run():
+            ctx, o32, lse = ops.attn_forward(q, k, v, lens, Hq, Hkv)
+            dq, dk, dv = ops.attn_backward(q, k, v, o32, lse, do, lens, Hq, Hkv)
+            _, _, dH = ops.head_backward(ctx, W, ids, lens)
+            return ctx, dq, dk, dv, dH, ops.gemm_nt(q, W, out_dtype=torch.float32)
+        return run
+
+    jobs = [job(i, lens, V) for i, (lens, V) in enumerate(
+        [([37, 128, 1], 700), ([300], 1500), ([64, 65], 332), ([5, 900, 20], 2000)])]
+    want = [j() for j in jobs]
+    bad = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for rep in range(6):
+                got = jobs[i]()
+                if release and rep % 2:
+                    ops.release_workspaces()
+                if not all(torch.equal(a, b) for a, b in zip(got, want[i])):
+                    bad.append((i, rep))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad, bad
