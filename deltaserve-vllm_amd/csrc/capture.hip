@@ -48,8 +48,37 @@ template <>
 DSB_DEV float round_to<DSB_DT_F32>(float v) { return v; }
 }  // namespace
 
-// One block per index slot; the block's threads cover the row's width.
+// 8 consecutive elements as floats (16-byte aligned: one 16-byte load, two for
+// fp32).
 template <int T>
+DSB_DEV void load8_as_float(const void* p, long i, float v[8]) {
+  if constexpr (T == DSB_DT_F32) {
+    const f32x4* q = reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(p) + i);
+    const f32x4 a = q[0], b = q[1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = a[e];
+      v[4 + e] = b[e];
+    }
+  } else if constexpr (T == DSB_DT_F16) {
+    typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+    const f16x8 a = *reinterpret_cast<const f16x8*>(reinterpret_cast<const _Float16*>(p) + i);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = (float)a[e];
+  } else {
+    unpack8(ldg128(reinterpret_cast<const bf16*>(p) + i), v);
+  }
+}
+
+// The grid's x is the index slot, its y a run of kSaveRun columns of the row;
+// a thread moves kSaveVec groups of 8 columns, loaded before the first is
+// stored. VEC: 16-byte accesses (rows, strides and width allow them), else
+// element by element. One block per row with one load in flight per thread,
+// and residual rows element by element, took 13.6 µs per launch for the
+// 256-row saves of a 5120-wide model (residual and 34816-wide rows, 34 µs of
+// them in 17 launches at copy rate); now 7.9 µs.
+constexpr int kSaveVec = 2, kSaveRun = 256 * 8 * kSaveVec;
+template <int T, bool VEC>
 __global__ __launch_bounds__(256) void save_rows_kernel(const void* __restrict__ x, long ldx,
                                                         const void* __restrict__ r, long ldr,
                                                         long x_rows,
@@ -57,23 +86,52 @@ __global__ __launch_bounds__(256) void save_rows_kernel(const void* __restrict__
                                                         const int64_t* __restrict__ dst, int width,
                                                         bf16* __restrict__ buf, long ldbuf,
                                                         long buf_rows) {
-  const long d = dst[blockIdx.x];
+  const long d = dst[blockIdx.x], s = src[blockIdx.x];
   if (d < 0 || d >= buf_rows - 1) return;  // the scratch row (and out of range): skipped
-  const long s = src[blockIdx.x];
   if (s < 0 || s >= x_rows) return;  // a source row outside x: skipped
   const long xo = s * ldx, ro = s * ldr, bo = d * ldbuf;
-  if (T == DSB_DT_BF16 && !r && (width & 7) == 0 && ((ldx | ldbuf) & 7) == 0 &&
-      (((unsigned long)x | (unsigned long)buf) & 15) == 0) {
-    // plain bf16 copy: 16 bytes per lane
-    const bf16* xs = reinterpret_cast<const bf16*>(x) + xo;
-    for (int c = threadIdx.x * 8; c < width; c += 256 * 8)
-      stg128(buf + bo + c, ldg128(xs + c));
-    return;
-  }
-  for (int c = threadIdx.x; c < width; c += 256) {
-    float v = load_as_float<T>(x, xo + c);
-    if (r) v = round_to<T>(v + load_as_float<T>(r, ro + c));
-    buf[bo + c] = (bf16)v;
+  const int c0 = blockIdx.y * kSaveRun;
+  if constexpr (VEC) {
+    if (T == DSB_DT_BF16 && !r) {  // a copy: the bits as they are, NaN payloads included
+      u32x4 v[kSaveVec];
+#pragma unroll
+      for (int i = 0; i < kSaveVec; ++i) {
+        const int c = c0 + (threadIdx.x + 256 * i) * 8;
+        if (c < width) v[i] = ldg128(reinterpret_cast<const bf16*>(x) + xo + c);
+      }
+#pragma unroll
+      for (int i = 0; i < kSaveVec; ++i) {
+        const int c = c0 + (threadIdx.x + 256 * i) * 8;
+        if (c < width) stg128(buf + bo + c, v[i]);
+      }
+      return;
+    }
+    float v[kSaveVec][8], w[kSaveVec][8];
+#pragma unroll
+    for (int i = 0; i < kSaveVec; ++i) {
+      const int c = c0 + (threadIdx.x + 256 * i) * 8;
+      if (c < width) {
+        load8_as_float<T>(x, xo + c, v[i]);
+        if (r) load8_as_float<T>(r, ro + c, w[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kSaveVec; ++i) {
+      const int c = c0 + (threadIdx.x + 256 * i) * 8;
+      if (c >= width) continue;
+      if (r) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[i][e] = round_to<T>(v[i][e] + w[i][e]);
+      }
+      stg128(buf + bo + c, pack8(v[i]));
+    }
+  } else {
+    const int end = min(width, c0 + kSaveRun);
+    for (int c = c0 + threadIdx.x; c < end; c += 256) {
+      float v = load_as_float<T>(x, xo + c);
+      if (r) v = round_to<T>(v + load_as_float<T>(r, ro + c));
+      buf[bo + c] = (bf16)v;
+    }
   }
 }
 
@@ -94,23 +152,26 @@ hipError_t save_rows(const void* x, long ldx, const void* r, long ldr, long x_ro
                      const int64_t* src, const int64_t* dst, int count, int width, bf16* buf,
                      long ldbuf, long buf_rows, hipStream_t s) {
   if (count <= 0 || width <= 0) return hipSuccess;
+  const long es = dtype == DSB_DT_F32 ? 4 : 2;
+  const bool vec = width % 8 == 0 && ldx * es % 16 == 0 && (!r || ldr * es % 16 == 0) &&
+                   ldbuf % 8 == 0 &&
+                   (((unsigned long)x | (unsigned long)r | (unsigned long)buf) & 15) == 0;
+  const dim3 grid(count, (width + kSaveRun - 1) / kSaveRun);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, x, ldx, r, ldr, x_rows, src, dst, width, buf,
+                       ldbuf, buf_rows);
+    return hipGetLastError();
+  };
   switch (dtype) {
     case DSB_DT_BF16:
-      hipLaunchKernelGGL(save_rows_kernel<DSB_DT_BF16>, dim3(count), dim3(256), 0, s, x, ldx, r,
-                         ldr, x_rows, src, dst, width, buf, ldbuf, buf_rows);
-      break;
+      return vec ? go(save_rows_kernel<DSB_DT_BF16, true>) : go(save_rows_kernel<DSB_DT_BF16, false>);
     case DSB_DT_F16:
-      hipLaunchKernelGGL(save_rows_kernel<DSB_DT_F16>, dim3(count), dim3(256), 0, s, x, ldx, r, ldr,
-                         x_rows, src, dst, width, buf, ldbuf, buf_rows);
-      break;
+      return vec ? go(save_rows_kernel<DSB_DT_F16, true>) : go(save_rows_kernel<DSB_DT_F16, false>);
     case DSB_DT_F32:
-      hipLaunchKernelGGL(save_rows_kernel<DSB_DT_F32>, dim3(count), dim3(256), 0, s, x, ldx, r, ldr,
-                         x_rows, src, dst, width, buf, ldbuf, buf_rows);
-      break;
+      return vec ? go(save_rows_kernel<DSB_DT_F32, true>) : go(save_rows_kernel<DSB_DT_F32, false>);
     default:
       return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
 
 hipError_t save_ids(const int64_t* ids, long ids_len, const int64_t* src, const int64_t* dst, int count,

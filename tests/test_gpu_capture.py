@@ -62,6 +62,34 @@ def test_save_rows_bit_exact_vs_oracle(xdt, width, ld_pad, resid):
     assert torch.equal(got[M], buf[M])  # the scratch row is not written
 
 
+@pytest.mark.parametrize("xdt", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("width,ld_pad", [(4104, 0), (8192, 0), (12304, 16), (4100, 0), (9001, 2)])
+@pytest.mark.parametrize("resid", [False, True])
+def test_save_rows_wide(xdt, width, ld_pad, resid):
+    """Rows of more than one 4096-column run (the grid's second axis): a whole
+    last run, 8 columns, a partial one, and widths off the 16-byte path; the
+    stored values are the bf16 of the same sums, so bit-exact, with infinities,
+    NaN and denormals among them (a plain bf16 save keeps NaN payloads)."""
+    C = _capture()
+    g = torch.Generator().manual_seed(width)
+    T, M = 20, 9
+    xf = (torch.randn(T, width + ld_pad, generator=g) * 4).to(xdt)
+    xf[3, 5:9] = torch.tensor([float("inf"), -float("inf"), 1e-40, -0.0]).to(xdt)
+    xf[3, 4100 - 1] = float("nan")
+    rf = (torch.randn(T, width + ld_pad, generator=g) * 4).to(xdt) if resid else None
+    pos = torch.tensor([3, 19, 0, 7, 11])
+    src, dst, n = O.capture_index(pos.tolist(), 5, 2, M)
+    buf = torch.randn(M + 1, width, generator=g).to(torch.bfloat16)
+    want = _oracle_save(xf[:, :width], None if rf is None else rf[:, :width], buf.clone(), src, dst)
+    gbuf, gx = buf.cuda(), xf.cuda()[:, :width]
+    C.save_rows(gx, None if rf is None else rf.cuda()[:, :width], gbuf, src.cuda(), dst.cuda())
+    torch.cuda.synchronize()
+    got = gbuf.cpu()[:M]
+    nan = torch.isnan(want[:M].float())
+    assert torch.equal(torch.isnan(got.float()), nan)
+    assert torch.equal(got.view(torch.int16)[~nan], want[:M].view(torch.int16)[~nan])
+
+
 def test_capture_follows_index_contents():
     """tests/test_ft_save_op.py:40-90 on the MI355X op: capture once, replay
     with other positions and offsets; a stateless capture records nothing."""
