@@ -688,9 +688,13 @@ const char* cfg_name(int cfg) {
 // One NT GEMM launch of the cycle (M = live tokens), timed under
 // "<tile>_<epilogue>". Algorithmic flops 2·n·N·(K1+K2); bytes: A, B once,
 // C once at `ob` bytes per element, plus `xrow` extra bytes per output row.
+// parts (optional): the caller takes a split product's K-slice partials itself
+// (*parts planes of p.M × p.N floats in h->part, 1: none, e holds the result)
+// instead of the reduction's output.
 template <class Epi>
 int gemm(dsb_handle* h, const char* epi, const GemmProblem& p, const Epi& e, hipStream_t st,
-         double ob, double xrow) {
+         double ob, double xrow, int* parts = nullptr) {
+  if (parts) *parts = 1;
   const double K = (double)p.K1 + p.K2;
   constexpr bool can_split = SplitPart<Epi>::enabled;
   GemmPlan pl = h->gemm_cfg >= 0
@@ -704,7 +708,12 @@ int gemm(dsb_handle* h, const char* epi, const GemmProblem& p, const Epi& e, hip
                 2.0 * K + ob * p.N + xrow, 0, 2.0 * p.N * K);
       GemmProblem q = p;
       q.part = h->part;
-      LK(launch_gemm_split(q, e, pl, st));
+      if (parts) {
+        *parts = pl.ks;
+        LK(launch_gemm(q, e, st, pl.cfg, pl.ks));
+      } else {
+        LK(launch_gemm_split(q, e, pl, st));
+      }
       return 0;
     }
     // a partly filled last round of tiles: split K over the tail tiles
@@ -1091,12 +1100,15 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
       if (rest_g) CKR(skinny(h, h->Ggu, 2L * I, ls.BTg, r, I, h->gZgu_b, 2 * r, st));
       if (rest_u) CKR(skinny(h, h->Ggu + I, 2L * I, ls.BTu, r, I, h->gZgu_b + r, 2 * r, st));
     }
+    // K slices of the FFN and attention input gradients the RMSNorm backward adds
+    int parts = 1;
+    const long plane = (long)N * D;
     {
       GemmProblem p{h->Ggu, 2L * I, wgu, (long)D, hg ? h->gZgu_b : nullptr, 2L * r,
                     hg ? ls.Agu : nullptr, (long)D, N, D, 2 * I, hg ? 2 * r : 0, nd};
       p.b_kn = 1;
       EpiF32 e{h->gxn2, (long)D, D, 0};
-      CKR(gemm(h, "dx32", p, e, st, 4.0, 0.0));
+      CKR(gemm(h, "dx32", p, e, st, 4.0, 0.0, &parts));
     }
     if (hg) {
       float* gAg = grad_a(h, ls, DSB_PROJ_GATE);
@@ -1110,9 +1122,9 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
                nullptr, nullptr, r, 1, h->s, st));
     }
     {
-      KScope ks(h, st, "rmsnorm_bwd", 0, 0, 0, 18.0 * D, 0, 2.0 * D);
-      LK(rmsnorm_bwd(rs, ldrs, h->gxn2, true, D, (const bf16*)ls.w.post_ln, nullptr, D,
-                     h->grm, D, N, nd, D, eps, st, g32, h->grm32));
+      KScope ks(h, st, "rmsnorm_bwd", 0, 0, 0, 14.0 * D + 4.0 * D * parts, 0, 2.0 * D);
+      LK(rmsnorm_bwd(rs, ldrs, parts > 1 ? h->part : h->gxn2, true, D, (const bf16*)ls.w.post_ln,
+                     nullptr, D, h->grm, D, N, nd, D, eps, st, g32, h->grm32, parts, plane));
     }
     int dual_o = 1;
     if (ho) {
@@ -1200,7 +1212,7 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
                     hq ? ls.Aqkv : nullptr, (long)D, N, D, W3, hq ? 3 * r : 0, nd};
       p.b_kn = 1;
       EpiF32 e{h->gxn1, (long)D, D, 0};
-      CKR(gemm(h, "dx32", p, e, st, 4.0, 0.0));
+      CKR(gemm(h, "dx32", p, e, st, 4.0, 0.0, &parts));
     }
     if (hq) {
       CKR(tn(h, h->gZqkv_b, 3 * r, h->xn1, D, 3 * r, D, grad_a(h, ls, DSB_PROJ_Q),
@@ -1216,9 +1228,9 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
                nullptr, nullptr, r, 1, h->s, st));
     }
     {
-      KScope ks(h, st, "rmsnorm_bwd", 0, 0, 0, 18.0 * D, 0, 2.0 * D);
-      LK(rmsnorm_bwd(x, ldx, h->gxn1, true, D, (const bf16*)ls.w.in_ln, nullptr, D, gnext, D,
-                     N, nd, D, eps, st, h->grm32, gnext32));
+      KScope ks(h, st, "rmsnorm_bwd", 0, 0, 0, 14.0 * D + 4.0 * D * parts, 0, 2.0 * D);
+      LK(rmsnorm_bwd(x, ldx, parts > 1 ? h->part : h->gxn1, true, D, (const bf16*)ls.w.in_ln,
+                     nullptr, D, gnext, D, N, nd, D, eps, st, h->grm32, gnext32, parts, plane));
     }
     CKR(tn_flush(h, st));
     return 0;

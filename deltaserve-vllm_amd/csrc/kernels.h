@@ -11,11 +11,13 @@ hipError_t rmsnorm_fwd(const bf16* x, long ldx, const bf16* w, bf16* y, long ldy
                        const int* rows_dev, int D, float eps, hipStream_t s);
 // out = bf16(o), o = rmsnorm_backward(x, g, w) + (resid | resid32), and the
 // fp32 o into out32 when set (resid and resid32 share the row stride ldr,
-// out and out32 the row stride ldo).
+// out and out32 the row stride ldo). An fp32 g may be gparts planes, gplane
+// elements apart, whose sum is the gradient.
 hipError_t rmsnorm_bwd(const bf16* x, long ldx, const void* g, bool g_f32, long ldg,
                        const bf16* w, const bf16* resid, long ldr, bf16* out, long ldo,
                        int rows, const int* rows_dev, int D, float eps, hipStream_t s,
-                       const float* resid32 = nullptr, float* out32 = nullptr);
+                       const float* resid32 = nullptr, float* out32 = nullptr, int gparts = 1,
+                       long gplane = 0);
 hipError_t rope_table(const int* pos, int n, const int* n_dev, const float* inv_freq,
                       int half, float* cosb, float* sinb, hipStream_t s);
 // q heads of a row at in / pre (row stride ldin / ldp); k heads at ink / prek

@@ -102,10 +102,15 @@ __global__ __launch_bounds__(256) void rmsnorm_fwd_wave_kernel(
 // o = rmsnorm_backward(x, g, w) + resid (g fp32 or bf16; resid bf16, fp32
 // resid32, or none) → out = bf16(o) and, when out32 is set, the fp32 o (the
 // residual-stream gradient the next layer adds to, kept unrounded).
+// With gparts > 1 an fp32 g is the sum, in order, of gparts planes (row stride
+// ldg, gplane elements apart): the K-slice partials of the product that made
+// it, added here instead of by a reduction launch that writes the sum for this
+// pass to read (nine passes and eight reductions of a 4-layer cycle: 256 rows
+// × 5120, 84 + 129 µs → 132; 2048 × 2048, 144 + 107 → 170).
 template <typename GT>
 __global__ __launch_bounds__(NORM_NT) void rmsnorm_bwd_kernel(
-    const bf16* __restrict__ x, long ldx, const GT* __restrict__ g, long ldg,
-    const bf16* __restrict__ w, const bf16* __restrict__ resid,
+    const bf16* __restrict__ x, long ldx, const GT* __restrict__ g, long ldg, int gparts,
+    long gplane, const bf16* __restrict__ w, const bf16* __restrict__ resid,
     const float* __restrict__ resid32, long ldr, bf16* __restrict__ out,
     float* __restrict__ out32, long ldo, int rows, const int* rows_dev, int D, float eps) {
   int R = rows;
@@ -126,8 +131,24 @@ __global__ __launch_bounds__(NORM_NT) void rmsnorm_bwd_kernel(
       float wf[8];
       unpack8(ldg128(w + c * 8), wf);
       if constexpr (sizeof(GT) == 4) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(gr + c * 8);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(gr + c * 8 + 4);
+        f32x4 a = *reinterpret_cast<const f32x4*>(gr + c * 8);
+        f32x4 b = *reinterpret_cast<const f32x4*>(gr + c * 8 + 4);
+        for (int z0 = 1; z0 < gparts; z0 += 4) {  // four planes' loads in flight
+          f32x4 pa[4], pb[4];
+#pragma unroll
+          for (int z = 0; z < 4; ++z)
+            if (z0 + z < gparts) {
+              const GT* p = gr + (z0 + z) * gplane + c * 8;
+              pa[z] = *reinterpret_cast<const f32x4*>(p);
+              pb[z] = *reinterpret_cast<const f32x4*>(p + 4);
+            }
+#pragma unroll
+          for (int z = 0; z < 4; ++z)
+            if (z0 + z < gparts) {
+              a += pa[z];
+              b += pb[z];
+            }
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) { gw[i][e] = a[e] * wf[e]; gw[i][e + 4] = b[e] * wf[e + 4]; }
       } else {
@@ -375,15 +396,15 @@ hipError_t rmsnorm_fwd(const bf16* x, long ldx, const bf16* w, bf16* y, long ldy
 hipError_t rmsnorm_bwd(const bf16* x, long ldx, const void* g, bool g_f32, long ldg,
                        const bf16* w, const bf16* resid, long ldr, bf16* out, long ldo,
                        int rows, const int* rows_dev, int D, float eps, hipStream_t s,
-                       const float* resid32, float* out32) {
+                       const float* resid32, float* out32, int gparts, long gplane) {
   if (rows <= 0) return hipSuccess;
   if (g_f32)
     hipLaunchKernelGGL(rmsnorm_bwd_kernel<float>, dim3(rows), dim3(NORM_NT), 0, s, x, ldx,
-                       (const float*)g, ldg, w, resid, resid32, ldr, out, out32, ldo, rows,
+                       (const float*)g, ldg, gparts, gplane, w, resid, resid32, ldr, out, out32, ldo, rows,
                        rows_dev, D, eps);
   else
     hipLaunchKernelGGL(rmsnorm_bwd_kernel<bf16>, dim3(rows), dim3(NORM_NT), 0, s, x, ldx,
-                       (const bf16*)g, ldg, w, resid, resid32, ldr, out, out32, ldo, rows,
+                       (const bf16*)g, ldg, 1, 0L, w, resid, resid32, ldr, out, out32, ldo, rows,
                        rows_dev, D, eps);
   return hipGetLastError();
 }

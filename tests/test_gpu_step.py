@@ -44,6 +44,17 @@ def test_cycle_parity_head_dim_64(family):
     assert_north_star(worst)
 
 
+@pytest.mark.parametrize("I,lens", [(1536, [70]), (4096, [3, 90, 1]), (8192, [130, 31])])
+def test_cycle_parity_split_input_gradients(I, lens):
+    """Few rows over a long reduction: the dX products of the FFN input run in
+    K slices (3 to 16 of them, none a multiple of four) whose partials the
+    RMSNorm backward adds, and the LM head's dH keeps one accumulator per
+    slice over three vocabulary chunks."""
+    meta = tiny_meta(L=2, I=I, V=1500, s_max=sum(lens) + 3, vocab_chunk=512)
+    worst = _run(meta, lens)
+    assert_north_star(worst)
+
+
 def test_cycle_parity_qkvo_only_llama3_rope_scaling():
     """The reference's own configuration: LoRA on q/k/v/o only, llama3 RoPE."""
     sc = {"rope_type": "llama3", "factor": 8.0, "low_freq_factor": 1.0,
