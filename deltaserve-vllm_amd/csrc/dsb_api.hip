@@ -184,8 +184,8 @@ struct dsb_handle {
   dsb_desc d{};
   int D, Hq, Hkv, hd, q, kv, W3, I, V, r, L, N, max_tiles, vchunk, nvc;
   HeadArgs head{};  // the LM head's plan (tiles, K slices, statistics layout)
-  // the adapter's rank (rv) and the rank the kernels run at (r: rv rounded up
-  // to a multiple of 8; the padded rows of A and columns of B are zeros in the
+  // the adapter's rank (rv) and the rank the kernels run at (r: rv rounded up,
+  // see dsb_create; the padded rows of A and columns of B are zeros in the
   // bf16 operands, so they add nothing, and their gradients are not stored)
   int rv;
   int gemm_cfg = -1;  // forced dense-product tile (GEMM_*), -1 by shape
@@ -1128,9 +1128,12 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
     }
     int dual_o = 1;
     if (ho) {
+      // a small operand: the skinny pass alone is on the layer's critical path
+      // (grad_B joins the layer's batched token reductions), 5 µs against 13
+      // for the fused pass and its reduction at 504 × 1024 to 256 × 5120
       const DualSpec d{h->grm, D, D, h->Zo_b, r, ls.BTo, h->gZo_b, r, ls.lora[DSB_PROJ_O].gB,
                        h->s, 1};
-      dual_o = dual(h, &d, 1, r, st);
+      dual_o = (long)N * D <= (4L << 20) ? 1 : dual(h, &d, 1, r, st);
       if (dual_o < 0) return -1;
       if (dual_o) CKR(skinny(h, h->grm, D, ls.BTo, r, D, h->gZo_b, r, st));
     }
@@ -1591,7 +1594,14 @@ int dsb_create(const dsb_desc* d, dsb_handle** out) {
   h->hd = d->head_dim;
   h->q = h->Hq * h->hd; h->kv = h->Hkv * h->hd; h->W3 = h->q + 2 * h->kv;
   h->I = d->intermediate; h->V = d->vocab; h->L = d->n_layers;
-  h->rv = d->lora_rank; h->r = (d->lora_rank + 7) / 8 * 8;
+  h->rv = d->lora_rank;
+  // The rank the kernels run at: a multiple of 8. Where the MLP's operands are
+  // large enough for the fused LoRA passes (ranks 16 and 32) to save more than
+  // their reductions cost, ranks below those go up to them: separate skinny
+  // and token-reduction passes would read h, d_gate and d_up twice (rank 8,
+  // 2048 × 8192: cycle 4634 → 4539 µs; 504 × 3072: 1623 → 1631, so not there).
+  h->r = (h->rv + 7) / 8 * 8;
+  if (h->r <= 32 && (long)d->s_max * d->intermediate > (4L << 20)) h->r = h->r <= 16 ? 16 : 32;
   h->N = d->s_max; h->s = d->lora_scaling; h->qwen = d->family == DSB_FAMILY_QWEN3;
   h->max_tiles = max_tiles_for(d->s_max, std::min(d->max_seqs, d->s_max));
   // LM-head vocab chunk: one pause point per chunk in each pass, and the

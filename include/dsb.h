@@ -45,7 +45,7 @@ typedef struct dsb_handle dsb_handle;
 /* Model and trainer constants: the backward `meta` dict of
  * deltaserve-plugin/deltaserve/ft_meta.py:131-213 plus the AdamW settings of
  * trainer.py:252-256. head_dim 128 or 64; lora_rank in [1, 64] (the rank-r
- * kernels run at the rank rounded up to a multiple of 8, on zero-padded bf16
+ * kernels run at the rank rounded up (a multiple of 8, 16 or 32), on zero-padded bf16
  * copies of A and B, and store the adapter's own r rows of each gradient);
  * hidden <= 8192. */
 typedef struct dsb_desc {
