@@ -1210,13 +1210,6 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
       if (rest_qkv[2])
         CKR(skinny(h, h->gqkv + q + kv, W3, ls.BTv, r, kv, h->gZqkv_b + 2 * r, 3 * r, st));
     }
-    {
-      GemmProblem p{h->gqkv, (long)W3, wqkv, (long)D, hq ? h->gZqkv_b : nullptr, 3L * r,
-                    hq ? ls.Aqkv : nullptr, (long)D, N, D, W3, hq ? 3 * r : 0, nd};
-      p.b_kn = 1;
-      EpiF32 e{h->gxn1, (long)D, D, 0};
-      CKR(gemm(h, "dx32", p, e, st, 4.0, 0.0, &parts));
-    }
     if (hq) {
       CKR(tn(h, h->gZqkv_b, 3 * r, h->xn1, D, 3 * r, D, grad_a(h, ls, DSB_PROJ_Q),
              grad_a(h, ls, DSB_PROJ_K), grad_a(h, ls, DSB_PROJ_V), r, 0, 1.f, st));
@@ -1230,12 +1223,34 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
         CKR(tn(h, h->Zqkv_b + 2 * r, 3 * r, h->gqkv + q + kv, W3, r, kv, grad_b(h, ls, DSB_PROJ_V),
                nullptr, nullptr, r, 1, h->s, st));
     }
+    // The layer's token reductions (grad_A, grad_B) read what is complete by
+    // now and nothing in the layer reads their outputs: on the second stream
+    // they run beside the last dX product and RMSNorm backward instead of after
+    // them. Only with the layer overlap: where the products fill every CU for
+    // several rounds the order makes no difference.
+    const bool tfork = h->overlap && !h->ktiming && !h->tn_pending.empty();
+    if (tfork) {
+      CK(hipEventRecord(h->ev_fork, st));
+      CK(hipStreamWaitEvent(h->hs2, h->ev_fork, 0));
+      CKR(tn_flush(h, h->hs2));
+      CK(hipEventRecord(h->ev_join, h->hs2));
+    }
+    {
+      GemmProblem p{h->gqkv, (long)W3, wqkv, (long)D, hq ? h->gZqkv_b : nullptr, 3L * r,
+                    hq ? ls.Aqkv : nullptr, (long)D, N, D, W3, hq ? 3 * r : 0, nd};
+      p.b_kn = 1;
+      EpiF32 e{h->gxn1, (long)D, D, 0};
+      CKR(gemm(h, "dx32", p, e, st, 4.0, 0.0, &parts));
+    }
     {
       KScope ks(h, st, "rmsnorm_bwd", 0, 0, 0, 14.0 * D + 4.0 * D * parts, 0, 2.0 * D);
       LK(rmsnorm_bwd(x, ldx, parts > 1 ? h->part : h->gxn1, true, D, (const bf16*)ls.w.in_ln,
                      nullptr, D, gnext, D, N, nd, D, eps, st, h->grm32, gnext32, parts, plane));
     }
-    CKR(tn_flush(h, st));
+    if (tfork)
+      CK(hipStreamWaitEvent(st, h->ev_join, 0));
+    else
+      CKR(tn_flush(h, st));
     return 0;
   }
   return 0;
