@@ -182,7 +182,7 @@ struct GraphSet {  // the cycle's graphs for one attention grid capacity
 
 struct dsb_handle {
   dsb_desc d{};
-  int D, Hq, Hkv, hd, q, kv, W3, I, V, r, L, N, max_tiles, vchunk, nvc;
+  int D, Hq, Hkv, hd, q, kv, W3, I, V, r, L, N, max_tiles, vchunk, nvc, vgroup;
   HeadArgs head{};  // the LM head's plan (tiles, K slices, statistics layout)
   // the adapter's rank (rv) and the rank the kernels run at (r: rv rounded up,
   // see dsb_create; the padded rows of A and columns of B are zeros in the
@@ -423,7 +423,7 @@ int finalize(dsb_handle* h) {
   CKR(dalloc(h, &h->run_m, NN));
   CKR(dalloc(h, &h->run_l, NN));
   CKR(dalloc(h, &h->alpha, NN));
-  CKR(dalloc(h, &h->dlog, NN * h->vchunk));
+  CKR(dalloc(h, &h->dlog, NN * h->head.vchunk));
   CKR(dalloc(h, &h->dH, NN * D));
   h->tn_work_elems = 32L << 20;
   CKR(dalloc(h, &h->tn_work, h->tn_work_elems));
@@ -446,7 +446,7 @@ int finalize(dsb_handle* h) {
     long need = head_part_elems(h->head);
     {
       int tail = 0;
-      const int kt = gemm_tail_split(N, D, h->vchunk, h->ncu, &tail);
+      const int kt = gemm_tail_split(N, D, h->head.vchunk, h->ncu, &tail);
       if (h->head.dh_ks == 1 && kt > 1) need = std::max(need, (long)kt * tail * 65536);
     }
     for (const auto& sh : shapes) {
@@ -1283,6 +1283,13 @@ int join_recompute(dsb_handle* h, hipStream_t st) {
   return 0;
 }
 
+// A head segment between its unit's two products (enqueue_segment).
+bool segment_is_empty(const dsb_handle* h, int seg) {
+  if (seg >= 2 * h->nvc) return false;
+  const int c = seg / 2;
+  return seg & 1 ? c % h->vgroup != h->vgroup - 1 && c != h->nvc - 1 : c % h->vgroup != 0;
+}
+
 int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
   const int N = h->N, D = h->D;
   const int* nd = &h->d_hdr->n;
@@ -1315,8 +1322,12 @@ int enqueue_segment(dsb_handle* h, int seg, hipStream_t st) {
         LK(head_init(ha, st));
       }
     }
-    const int c = seg / 2;
-    const int c0 = c * h->vchunk, Vc = std::min(h->vchunk, h->V - c0);
+    // A unit of vgroup chunks is computed as one: its logits in the segment of
+    // its first chunk, its dH product in that of its last; the segments
+    // between are pause points without work.
+    const int c = seg / 2, cu = c / h->vgroup * h->vgroup;
+    const int c0 = cu * h->vchunk, Vc = std::min(h->head.vchunk, h->V - c0);
+    if (segment_is_empty(h, seg)) return 0;
     if ((seg & 1) == 0) {
       {
         // 2·n·Vc·D of the head's algorithmic 4·M·D·V (the logits product)
@@ -1619,15 +1630,17 @@ int dsb_create(const dsb_desc* d, dsb_handle** out) {
   if (h->r <= 32 && (long)d->s_max * d->intermediate > (4L << 20)) h->r = h->r <= 16 ? 16 : 32;
   h->N = d->s_max; h->s = d->lora_scaling; h->qwen = d->family == DSB_FAMILY_QWEN3;
   h->max_tiles = max_tiles_for(d->s_max, std::min(d->max_seqs, d->s_max));
-  // LM-head vocab chunk: one pause point per chunk in each pass, and the
-  // width of the bf16 dlogits tile (16384 columns: 268 MB at 8192 rows)
+  // LM-head vocab chunk: one pause point per chunk in each pass; the bf16
+  // probability tile is vgroup chunks wide (16384 columns: 268 MB at 8192 rows)
   h->vchunk = d->vocab_chunk > 0 ? d->vocab_chunk : 16384;
   h->vchunk = (int)std::min<long>(h->vchunk, ((long)h->V + 255) / 256 * 256);
   h->nvc = (h->V + h->vchunk - 1) / h->vchunk;
   h->gemm_cfg = d->gemm_tile == 256 ? GEMM_BIG
               : d->gemm_tile == 128 ? GEMM_MID
               : d->gemm_tile == 64  ? GEMM_SKINNY : -1;
-  h->head.n = h->N; h->head.D = h->D; h->head.V = h->V; h->head.vchunk = h->vchunk;
+  h->head.n = h->N; h->head.D = h->D; h->head.V = h->V;
+  h->vgroup = d->vocab_chunk > 0 ? 1 : head_group(h->N, h->V, h->vchunk);
+  h->head.vchunk = h->vgroup * h->vchunk;
   head_plan(h->head, h->gemm_cfg, true);
   h->layers.resize(h->L);
   h->ktiming = (d->flags & DSB_FLAG_KTIMING) != 0;
@@ -1904,7 +1917,9 @@ int dsb_step_segment(dsb_handle* h, int seg, int run_ahead) {
   if (run_ahead < 0 || run_ahead > 64) return fail(h, "dsb_step_segment: run_ahead must be in [0, 64]");
   const int ns = num_segments(h);
   bool launched = false;
-  if ((h->d.flags & DSB_FLAG_GRAPH) && !h->graph_failed && !h->ktiming) {
+  if (segment_is_empty(h, seg)) {
+    launched = true;
+  } else if ((h->d.flags & DSB_FLAG_GRAPH) && !h->graph_failed && !h->ktiming) {
     GraphSet& gs = graph_set(h);
     if ((int)gs.seg_exec.size() != ns) {
       gs.seg_exec.assign(ns, nullptr);
@@ -2263,6 +2278,7 @@ int dsb_op_head(const void* normed, int64_t ldh, const void* lm_w, const int64_t
   HeadArgs a{};
   a.n = n; a.D = D; a.V = V;
   a.vchunk = std::min(vocab_chunk > 0 ? vocab_chunk : 16384, ((V + 255) / 256) * 256);
+  if (vocab_chunk == 0) a.vchunk *= head_group(n, V, a.vchunk);
   head_plan(a, -1, true);
   const long NN = n + 1;
   a.labels = tmp.dev<int>(NN);

@@ -1,6 +1,7 @@
 // Final-norm output → LM head → shifted cross-entropy → dH, streaming the
-// vocabulary in chunks: no [rows, vocab] logits, probabilities or dlogits
-// ever exist in memory, only a bf16 [rows, chunk] probability tile per chunk.
+// vocabulary in chunks: no [rows, vocab] logits or dlogits ever exist in
+// memory, only a bf16 [rows, chunk] probability tile per chunk (over few rows
+// several chunks, or all, are taken as one: head_group).
 //
 // Semantics: deltaserve-plugin/deltaserve/bwd_services/common/head.py:42-100
 //   loss = sum_rows CE(logits, target) / n_valid, dlogits = (softmax - onehot)/n_valid,
@@ -286,6 +287,26 @@ __global__ __launch_bounds__(1024) void ce_loss_kernel(const float* __restrict__
 }
 
 int head_num_chunks(const HeadArgs& a) { return (a.V + a.vchunk - 1) / a.vchunk; }
+
+int head_group(int n, int V, int vchunk) {
+  // A chunk's products over few rows are short: at 504 rows × 1024 the ten
+  // pairs of a 151936-word head took 25 + 31 µs each, launch gaps, half-filled
+  // last rounds and the accumulators' read and write included. Chunks are
+  // taken together while the probability tile stays within the 2^27 elements
+  // (268 MB) that 8192 rows have with one chunk, which also keeps the time
+  // between two pause points with work at that of such a cycle's chunk; the
+  // units are made equal. Cycles in µs by the bound 2^20 (one chunk each) /
+  // 2^25 / 2^26 / 2^27 / 2^28: 504 rows × 1024 × 151936: 1600 / 1442 / 1433 /
+  // 1399 / 1398; 256 × 5120 × 151936: 3540 / 3267 / 3104 / 3100 / 3109; 2048 ×
+  // 2048 × 128256: 4470 / 4470 / 4311 / 4231 / 4150 (the head alone 1880 /
+  // 1870 / 1814 / 1769 / 2021).
+  if (n <= 0) return 1;
+  const long kGroupElems = 1L << 27;
+  const long nch = ((long)V + vchunk - 1) / vchunk;
+  const long most = std::max(1L, kGroupElems / ((long)n * vchunk));
+  const long units = (nch + most - 1) / most;
+  return (int)((nch + units - 1) / units);
+}
 
 static GemmProblem chunk_logits_problem(const HeadArgs& a, int c0) {
   const int Vc = min(a.vchunk, a.V - c0);

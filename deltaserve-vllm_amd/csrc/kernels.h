@@ -184,8 +184,8 @@ struct HeadArgs {
   float* loss_row;                // [n_cap]
   float* loss_out;                // scalar: sum(loss_row)/n_valid
   const float* inv_nvalid;        // device scalar 1/n_valid (0 when none)
-  bf16* dlog; int vchunk;         // [n_cap, vchunk] bf16 probabilities of one vocab
-                                  // chunk; vchunk a multiple of 256
+  bf16* dlog; int vchunk;         // [n_cap, vchunk] bf16 probabilities of one product
+                                  // pair's columns; vchunk a multiple of 256
   float* dH;                      // [n, D] fp32
   // head_part_elems floats when dh_ks > 1: the dH product's accumulators, one
   // per K slice, live from the first chunk to the finalize
@@ -203,6 +203,8 @@ struct HeadArgs {
 void head_plan(HeadArgs& a, int gemm_cfg, bool can_split);
 long head_part_elems(const HeadArgs& a);
 int head_num_chunks(const HeadArgs& a);
+// Vocabulary chunks per logits / dH product pair where the chunk width is the default
+int head_group(int n, int V, int vchunk);
 hipError_t head_fwd_bwd(const HeadArgs& a, hipStream_t s);
 hipError_t head_init(const HeadArgs& a, hipStream_t s);
 hipError_t head_prob(const HeadArgs& a, int c0, hipStream_t s);

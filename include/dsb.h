@@ -170,7 +170,10 @@ int dsb_step(dsb_handle* h, const int32_t* seq_lens, int nseq, int n, float lr, 
  * reference calls once per vocab chunk in both LM-head passes (head.py:78-80,
  * :92-94) and at every layer boundary (llama3.py:342-344). With C =
  * ceil(vocab / vocab_chunk): segments 0 .. C-1 are the head's LSE pass, one
- * vocab chunk each; C .. 2C-1 its gradient pass; 2C .. 2C+L-1 the decoder
+ * vocab chunk each; C .. 2C-1 its gradient pass (the two products of a chunk
+ * run in segments 2c and 2c+1; with vocab_chunk = 0 and few rows, chunks are
+ * computed together, and the segments between a group's two products are
+ * pause points without work); 2C .. 2C+L-1 the decoder
  * layers from the last to the first; 2C+L (the last) the clip, AdamW and
  * publish. dsb_step_begin stages the
  * cycle (like dsb_step's first half); dsb_step_segment launches segment `seg`

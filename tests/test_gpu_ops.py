@@ -340,6 +340,36 @@ def test_head(V, vchunk):
     assert dH[last].abs().max().item() == 0.0  # rows that predict nothing
 
 
+@pytest.mark.parametrize("lens,V", [([5, 1, 30], 16384 * 3 + 77), ([700, 1200, 200], 16384 * 4 + 8)])
+def test_head_grouped_chunks(lens, V):
+    """The default chunk width over few rows: all chunks as one product pair,
+    and five as units of three and two (the last one short), against fp32 and
+    against the explicit width, which takes one chunk at a time. The two
+    differ only in the order of fp32 sums over the same bf16 operands."""
+    from deltaserve_amd import ops
+    n, D = sum(lens), 256
+    normed = _bf(_rnd(n, D, seed=44)).to(DEV)
+    W = _bf(_rnd(V, D, seed=45) * 0.05).to(DEV)
+    ids = torch.randint(0, V, (n,), generator=torch.Generator().manual_seed(46))
+    ids[1], ids[7] = 0, V - 1
+    loss, nv, dH = ops.head_backward(normed, W, ids.to(DEV), lens)
+    loss1, nv1, dH1 = ops.head_backward(normed, W, ids.to(DEV), lens, vocab_chunk=16384)
+    _, _, rows, tgt, n_valid = O.pack(lens)
+    logits = normed.float()[rows] @ W.float().t()
+    t = ids[tgt].to(DEV)
+    ref_loss = torch.nn.functional.cross_entropy(logits, t, reduction="sum").item() / n_valid
+    p = torch.softmax(logits, -1)
+    p[torch.arange(n_valid, device=DEV), t] -= 1
+    ref = torch.zeros(n, D, device=DEV)
+    ref[rows] = p @ W.float() / n_valid
+    assert nv == nv1 == n_valid
+    assert abs(loss - ref_loss) / ref_loss < 1e-4 and abs(loss - loss1) / ref_loss < 1e-5
+    assert max_rel(dH, ref) < 1e-2 and cosine(dH, ref) > 0.9999
+    assert max_rel(dH, dH1) < 1e-4
+    last = [sum(lens[:i + 1]) - 1 for i in range(len(lens))]
+    assert dH[last].abs().max().item() == 0.0
+
+
 @pytest.mark.parametrize("n,R,C", [(333, 24, 520), (8192, 16, 4096), (1000, 48, 1024), (17, 96, 256)])
 def test_lora_tn(n, R, C):
     from deltaserve_amd import ops

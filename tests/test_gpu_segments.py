@@ -124,6 +124,40 @@ def test_pause_points_per_vocab_chunk_and_layer():
         svc.close()
 
 
+def test_grouped_vocab_chunks_keep_their_segments():
+    """A vocabulary of three default chunks over few rows is computed as one
+    unit: the cycle still has a segment and a pause check per chunk and pass,
+    and equals the single graph bit for bit."""
+    from deltaserve_amd import _lib as L
+
+    meta = tiny_meta(L=2, V=40000)
+    model = O.make_model(meta, seed=6, w_std=0.05, b_std=0.02, norm_jitter=0.2)
+    n = sum(SEQ)
+    ids = torch.randint(0, 40000, (n,), generator=torch.Generator().manual_seed(6))
+    acts = bf16_round_acts(O.forward_capture(model, ids, SEQ))
+    gacts = gpu_activations(acts, meta["max_saved_finetuning_tokens"])
+    one = build_service(model, "llama3")
+    seg = build_service(model, "llama3")
+    seg.shared["meta"]["backward_pause_boundaries"] = True
+    seg.shared["meta"]["backward_run_ahead_boundaries"] = 2
+    calls = []
+    seg._maybe_pause = lambda: calls.append(1)
+    try:
+        for _ in range(3):
+            calls.clear()
+            out = [s.process_backward(gacts, SEQ, n, epoch=0) for s in (one, seg)]
+            assert out[0] == out[1]
+            assert L.load().dsb_num_segments(seg._h) == 2 * 3 + 2 + 1
+            assert len(calls) == 1 + 2 * 3 + 2
+            s1, s2 = _state(one), _state(seg)
+            for k in s1:
+                assert torch.equal(s1[k][0], s2[k][0]), ("master", k)
+                assert torch.equal(s1[k][1], s2[k][1]), ("grad", k)
+    finally:
+        one.close()
+        seg.close()
+
+
 def test_cleared_grant_holds_the_cycle_until_set():
     meta, model, gacts = _setup()
     n = sum(SEQ)
