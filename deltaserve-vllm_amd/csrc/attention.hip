@@ -894,7 +894,7 @@ hipError_t attn_bwd_dkdv(const AttnArgs& a, hipStream_t s) {
   // of its group and a second launch adds the heads' fp32 partials in order.
   const int hs = a.kv_part ? attn_dkdv_head_split(a) : 1;
   hipLaunchKernelGGL(attn_dkdv_kernel, dim3(a.max_tiles, a.Hkv, hs), dim3(256), 0, s, a);
-  if (hs == 1) return hipGetLastError();
+  if (hs == 1 || a.kv_defer) return hipGetLastError();
   const long tot = (long)a.n * (2L * a.Hkv * a.hd / 4);
   hipLaunchKernelGGL(dkdv_head_sum_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
                      a, hs);

@@ -735,16 +735,31 @@ int gemm(dsb_handle* h, const char* epi, const GemmProblem& p, const Epi& e, hip
 }
 
 // Rank-r product keeping tokens: Z = bf16(X·Bᵀ) (B [R, K]).
-int skinny(dsb_handle* h, const bf16* X, long ldx, const bf16* B, int R, int K, bf16* Z,
-           long ldz, hipStream_t s) {
+SkinnyArgs skinny_args(dsb_handle* h, const bf16* X, long ldx, const bf16* B, int R, int K,
+                       bf16* Z, long ldz) {
   SkinnyArgs a{X, ldx, B, (long)K, R, K, Z, ldz, h->N, &h->d_hdr->n};
   // K-split partials (short token ranges) in the TN workspace, which holds
   // nothing between the launches that use it
   a.part = h->tn_work;
   a.part_elems = h->tn_work_elems;
-  KScope ks(h, s, "lora_skinny", 2.0 * R * K, 0, 0, 2.0 * K + 2.0 * R, 0, 2.0 * R * K);
-  LK(lora_skinny(a, s));
+  return a;
+}
+
+// Independent products of one rank.
+int skinny(dsb_handle* h, const SkinnyArgs* a, int count, hipStream_t s) {
+  if (count <= 0) return 0;
+  double k = 0;
+  for (int i = 0; i < count; ++i) k += a[i].K;
+  const int R = a[0].R;
+  KScope ks(h, s, "lora_skinny", 2.0 * R * k, 0, 0, 2.0 * k + 2.0 * R * count, 0, 2.0 * R * k);
+  LK(lora_skinny(a, count, s));
   return 0;
+}
+
+int skinny(dsb_handle* h, const bf16* X, long ldx, const bf16* B, int R, int K, bf16* Z,
+           long ldz, hipStream_t s) {
+  const SkinnyArgs a = skinny_args(h, X, ldx, B, R, K, Z, ldz);
+  return skinny(h, &a, 1, s);
 }
 
 // A TN pass (grad_A = grad_Zᵀ·X or grad_B = s·Gᵀ·Z) of the layer being
@@ -922,7 +937,7 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
     at.hd = h->hd; at.scale = 1.f / std::sqrt((float)h->hd);
     // dK/dV head-split partials (short cycles) in the TN workspace, which
     // holds nothing while the attention passes run
-    at.kv_part = h->tn_work; at.kv_part_elems = h->tn_work_elems;
+    at.kv_part = h->tn_work; at.kv_part_elems = h->tn_work_elems; at.kv_defer = true;
     // one causal attention matmul = Hq·Hd·S flops (S = sum L(L+1), unmasked pairs ×2)
     const double au = (double)Hq * h->hd;
     const double arow = 2.0 * (q + 2.0 * kv);
@@ -1097,8 +1112,11 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
         if (tu) rest_u = dual(h, &d[1], 1, r, st);
       }
       if (rest_g < 0 || rest_u < 0) return -1;
-      if (rest_g) CKR(skinny(h, h->Ggu, 2L * I, ls.BTg, r, I, h->gZgu_b, 2 * r, st));
-      if (rest_u) CKR(skinny(h, h->Ggu + I, 2L * I, ls.BTu, r, I, h->gZgu_b + r, 2 * r, st));
+      SkinnyArgs z[2];
+      int nz = 0;
+      if (rest_g) z[nz++] = skinny_args(h, h->Ggu, 2L * I, ls.BTg, r, I, h->gZgu_b, 2 * r);
+      if (rest_u) z[nz++] = skinny_args(h, h->Ggu + I, 2L * I, ls.BTu, r, I, h->gZgu_b + r, 2 * r);
+      CKR(skinny(h, z, nz, st));
     }
     // K slices of the FFN and attention input gradients the RMSNorm backward adds
     int parts = 1;
@@ -1179,14 +1197,17 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
       }
     }
     {
-      KScope ks(h, st, "rope_bwd", 0, 0, 0, 4.0 * (q + kv) + 512.0, 0, 0);
+      const int hs = attn_dkdv_head_split(at);  // dK and dV as fp32 partials of its slices
+      KScope ks(h, st, "rope_bwd", 0, 0, 0,
+                4.0 * (q + kv) + 512.0 + (hs > 1 ? 8.0 * hs * kv : 0.0), 0, 0);
       // the q/k-norm backward (Qwen3) reads the pre-norm q/k: saved or recomputed
       if (sqkv && h->qwen)
         LK(rope_bwd(h->gqkv, W3, h->q_in[li], h->ld_q_in, h->cosb, h->sinb, N, nd, h->Hq,
-                    h->Hkv, h->hd, qnw, knw, eps, st, h->k_in[li], h->ld_k_in));
+                    h->Hkv, h->hd, qnw, knw, eps, st, h->k_in[li], h->ld_k_in, at.kv_part, hs));
       else
         LK(rope_bwd(h->gqkv, W3, h->qkv_pre, W3, h->cosb, h->sinb, N, nd, h->Hq, h->Hkv,
-                    h->hd, h->qwen ? qnw : nullptr, h->qwen ? knw : nullptr, eps, st));
+                    h->hd, h->qwen ? qnw : nullptr, h->qwen ? knw : nullptr, eps, st, nullptr, 0,
+                    at.kv_part, hs));
     }
     int rest_qkv[3] = {0, 0, 0};
     if (hq) {
@@ -1205,10 +1226,14 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
       const int rest = dual(h, d, cnt, r, st);
       if (rest < 0) return -1;
       for (int i = 0; i < cnt; ++i) rest_qkv[member[i]] = rest;
-      if (rest_qkv[0]) CKR(skinny(h, h->gqkv, W3, ls.BTq, r, q, h->gZqkv_b, 3 * r, st));
-      if (rest_qkv[1]) CKR(skinny(h, h->gqkv + q, W3, ls.BTk, r, kv, h->gZqkv_b + r, 3 * r, st));
+      SkinnyArgs z[3];
+      int nz = 0;
+      if (rest_qkv[0]) z[nz++] = skinny_args(h, h->gqkv, W3, ls.BTq, r, q, h->gZqkv_b, 3 * r);
+      if (rest_qkv[1])
+        z[nz++] = skinny_args(h, h->gqkv + q, W3, ls.BTk, r, kv, h->gZqkv_b + r, 3 * r);
       if (rest_qkv[2])
-        CKR(skinny(h, h->gqkv + q + kv, W3, ls.BTv, r, kv, h->gZqkv_b + 2 * r, 3 * r, st));
+        z[nz++] = skinny_args(h, h->gqkv + q + kv, W3, ls.BTv, r, kv, h->gZqkv_b + 2 * r, 3 * r);
+      CKR(skinny(h, z, nz, st));
     }
     if (hq) {
       CKR(tn(h, h->gZqkv_b, 3 * r, h->xn1, D, 3 * r, D, grad_a(h, ls, DSB_PROJ_Q),

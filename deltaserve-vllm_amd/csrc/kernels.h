@@ -30,7 +30,8 @@ hipError_t rope_fwd(const bf16* in, long ldin, bf16* out, long ldout, const floa
 hipError_t rope_bwd(bf16* g, long ldg, const bf16* pre, long ldp, const float* cosb,
                     const float* sinb, int n, const int* n_dev, int Hq, int Hkv, int hd,
                     const bf16* qn_w, const bf16* kn_w, float eps, hipStream_t s,
-                    const bf16* prek = nullptr, long ldpk = 0);
+                    const bf16* prek = nullptr, long ldpk = 0, const float* kv_part = nullptr,
+                    int hs = 1);
 hipError_t swiglu_h(const bf16* gu, long ldgu, bf16* h, long ldh, int n, const int* n_dev,
                     int I, hipStream_t s);
 
@@ -68,6 +69,7 @@ struct AttnArgs {
   // (Hq / Hkv) · n · 2 · Hkv·hd floats when the split applies
   float* kv_part = nullptr;
   long kv_part_elems = 0;
+  bool kv_defer = false;  // the caller adds a head split's partials (rope_bwd)
 };
 hipError_t attn_fwd(const AttnArgs& a, hipStream_t s);
 hipError_t attn_bwd(const AttnArgs& a, hipStream_t s);  // attn_dsum, dQ, dK/dV in order
@@ -107,6 +109,10 @@ struct SkinnyArgs {
 // takes the split when a.part is set
 int lora_skinny_split(const SkinnyArgs& a);
 hipError_t lora_skinny(const SkinnyArgs& a, hipStream_t s);
+// Up to kSkinnyBatch independent products of one n and R: one launch where they take the
+// same block shape and none splits K, else one after the other.
+constexpr int kSkinnyBatch = 3;
+hipError_t lora_skinny(const SkinnyArgs* a, int count, hipStream_t s);
 // out[j, c] (or out[c, j] when transposed) = scale · sum_t P[t, j] * X[t, c],
 // t < n. Output rows j are split into groups of `rg` written to outs[j / rg].
 struct TnArgs {

@@ -293,18 +293,22 @@ __global__ __launch_bounds__(256) void rope_fwd_kernel(
 
 // In-place RoPE backward on g[:, :(Hq+Hkv)*HD] (then the per-head RMSNorm
 // backward against the pre-norm projection output when norm weights are given);
-// same lane layout as the forward.
+// same lane layout as the forward. With hs > 1 dK and dV come as hs fp32
+// partials kv_part[z][t][m·Hkv·HD + column] (m = 0 dK, 1 dV) of the dK/dV
+// pass's head split: they are added in order and rounded to bf16 here (dK then
+// rotated, dV stored as it is) instead of in a launch of their own (504 × 8 kv
+// heads: that launch 4.2 µs plus its gap in each layer's chain).
 template <int HD>
 __global__ __launch_bounds__(256) void rope_bwd_kernel(
     bf16* __restrict__ g, long ldg, const bf16* __restrict__ pre, long ldp,
     const bf16* __restrict__ prek, long ldpk,
     const float* __restrict__ cosb, const float* __restrict__ sinb, int n,
     const int* n_dev, int Hq, int Hkv, const bf16* __restrict__ qn_w,
-    const bf16* __restrict__ kn_w, float eps) {
+    const bf16* __restrict__ kn_w, float eps, const float* __restrict__ kv_part, int hs) {
   constexpr int LPH = HD / 16, HPW = 64 / LPH, HALF = HD / 2;
   int N = n;
   if (n_dev) N = min(N, *n_dev);
-  const int H = Hq + Hkv, HG = (H + HPW - 1) / HPW;
+  const int H = Hq + (hs > 1 ? 2 : 1) * Hkv, HG = (H + HPW - 1) / HPW;
   const long item = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (item >= (long)N * HG) return;
   const int t = (int)(item / HG), l = threadIdx.x & 63, i = l % LPH;
@@ -313,8 +317,33 @@ __global__ __launch_bounds__(256) void rope_bwd_kernel(
   const int h = live ? hh : H - 1;
   bf16* gp = g + (long)t * ldg + h * HD + 8 * i;
   float g1[8], g2[8];
-  unpack8(ldg128(gp), g1);
-  unpack8(ldg128(gp + HALF), g2);
+  if (hs > 1 && h >= Hq) {
+    const long KV = (long)Hkv * HD, plane = (long)n * 2 * KV;
+    const float* src = kv_part + t * 2 * KV + (h - Hq) * HD + 8 * i;
+    f32x4 a[4] = {};
+#pragma unroll 4
+    for (int z = 0; z < hs; ++z)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        a[e] += *reinterpret_cast<const f32x4*>(src + z * plane + (e >> 1) * HALF + 4 * (e & 1));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      g1[e] = (float)(bf16)a[0][e];
+      g1[4 + e] = (float)(bf16)a[1][e];
+      g2[e] = (float)(bf16)a[2][e];
+      g2[4 + e] = (float)(bf16)a[3][e];
+    }
+    if (h >= Hq + Hkv) {  // a dV head
+      if (live) {
+        stg128(gp, pack8(g1));
+        stg128(gp + HALF, pack8(g2));
+      }
+      return;
+    }
+  } else {
+    unpack8(ldg128(gp), g1);
+    unpack8(ldg128(gp + HALF), g2);
+  }
   const f32x4* cp = reinterpret_cast<const f32x4*>(cosb + (long)t * HALF + 8 * i);
   const f32x4* sp = reinterpret_cast<const f32x4*>(sinb + (long)t * HALF + 8 * i);
   const f32x4 c0 = cp[0], c1 = cp[1], s0 = sp[0], s1 = sp[1];
@@ -443,10 +472,10 @@ hipError_t rope_fwd(const bf16* in, long ldin, bf16* out, long ldout, const floa
 hipError_t rope_bwd(bf16* g, long ldg, const bf16* pre, long ldp, const float* cosb,
                     const float* sinb, int n, const int* n_dev, int Hq, int Hkv, int hd,
                     const bf16* qn_w, const bf16* kn_w, float eps, hipStream_t s,
-                    const bf16* prek, long ldpk) {
+                    const bf16* prek, long ldpk, const float* kv_part, int hs) {
   if (hd != 128 && hd != 64) return hipErrorInvalidValue;
   const int hpw = 64 / (hd / 16);
-  const long items = (long)n * ((Hq + Hkv + hpw - 1) / hpw);
+  const long items = (long)n * ((Hq + (hs > 1 ? 2 : 1) * Hkv + hpw - 1) / hpw);
   if (items <= 0) return hipSuccess;
   if (!prek) {
     prek = pre + (long)Hq * hd;
@@ -455,10 +484,10 @@ hipError_t rope_bwd(bf16* g, long ldg, const bf16* pre, long ldp, const float* c
   const dim3 grid((unsigned)((items + 3) / 4));
   if (hd == 128)
     hipLaunchKernelGGL(rope_bwd_kernel<128>, grid, dim3(256), 0, s, g, ldg, pre, ldp, prek, ldpk,
-                       cosb, sinb, n, n_dev, Hq, Hkv, qn_w, kn_w, eps);
+                       cosb, sinb, n, n_dev, Hq, Hkv, qn_w, kn_w, eps, kv_part, hs);
   else
     hipLaunchKernelGGL(rope_bwd_kernel<64>, grid, dim3(256), 0, s, g, ldg, pre, ldp, prek, ldpk,
-                       cosb, sinb, n, n_dev, Hq, Hkv, qn_w, kn_w, eps);
+                       cosb, sinb, n, n_dev, Hq, Hkv, qn_w, kn_w, eps, kv_part, hs);
   return hipGetLastError();
 }
 

@@ -58,6 +58,18 @@ def test_cycle_parity_split_input_gradients(I, lens):
     assert_north_star(worst, direct_masters=False)
 
 
+@pytest.mark.parametrize("family,Hq,Hkv,Hd,r,lens", [
+    ("llama3", 5, 1, 128, 8, [1, 33]), ("qwen3", 6, 2, 64, 24, [64, 65, 2]),
+    ("qwen3", 10, 2, 128, 40, [257])])
+def test_cycle_parity_head_partials(family, Hq, Hkv, Hd, r, lens):
+    """Groups of 3 and 5 q-heads: dK and dV reach the RoPE backward as one
+    fp32 partial per head of the group (with an odd number of 64-wide heads
+    in a wave's run), and the group's grad_Z products run as one launch over
+    reductions of different lengths."""
+    meta = tiny_meta(family=family, L=2, Hq=Hq, Hkv=Hkv, Hd=Hd, D=384, I=640, r=r)
+    assert_north_star(_run(meta, lens))
+
+
 def test_cycle_parity_qkvo_only_llama3_rope_scaling():
     """The reference's own configuration: LoRA on q/k/v/o only, llama3 RoPE."""
     sc = {"rope_type": "llama3", "factor": 8.0, "low_freq_factor": 1.0,
