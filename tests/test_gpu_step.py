@@ -70,6 +70,19 @@ def test_cycle_parity_head_partials(family, Hq, Hkv, Hd, r, lens):
     assert_north_star(_run(meta, lens))
 
 
+@pytest.mark.parametrize("r", [3, 16, 17, 25])
+@pytest.mark.parametrize("s_max", [2048, 2049])
+def test_cycle_parity_rank_rule(r, s_max):
+    """Both sides of the line (s_max * intermediate = 2^22) past which ranks
+    below 16 and 32 run padded to them: gradients and masters keep the
+    adapter's own rank and the values of the unpadded product."""
+    meta = tiny_meta(L=1, I=2048, r=r, s_max=s_max)
+    worst = _run(meta, [65, 7])
+    # masters by the explained bar, as above: down_proj's A is bounded by
+    # 1/sqrt(I), where 2 steps of 2·lr are 4e-4·sqrt(2048) = 1.8e-2
+    assert_north_star(worst, direct_masters=False)
+
+
 def test_cycle_parity_qkvo_only_llama3_rope_scaling():
     """The reference's own configuration: LoRA on q/k/v/o only, llama3 RoPE."""
     sc = {"rope_type": "llama3", "factor": 8.0, "low_freq_factor": 1.0,
