@@ -7,10 +7,13 @@
 // registers, no atomics). Softmax statistics, P and dS stay fp32 in
 // registers; P and dS are rounded to bf16 only as MFMA operands.
 //
-// head_dim 64 runs the head_dim-128 kernels on heads zero-padded to 128 inside
-// the loads (dims past a.hd load as zeros, so they add nothing to Q·Kᵀ, dO·Vᵀ
-// or dsum, and come out of P·V, dS·K, dSᵀ·Q and Pᵀ·dO as zeros that the
-// stores skip), scaled by a.scale = 1/sqrt(head_dim).
+// The kernels are instantiated for both head widths (HW). A 64-wide head's
+// tiles keep the 128-column LDS layout, whose upper chunks are filled with
+// zeros that nothing reads; its products take half the MFMAs and fragment
+// reads. With the heads padded to 128 instead (half of every product zeros),
+// 32 heads over 8 kv heads, the same results bit for bit: forward 577 µs at
+// 12193 tokens in 2 sequences, 87 at 8192 in 32, 45 at 2048 in 8; now 451, 80
+// and 42; backward 1933, 196 and 116 µs; now 1307, 154 and 98.
 //
 // Semantics: deltaserve-plugin/deltaserve/bwd_services/common/attention.py
 //   attn_forward_core   :20-45   (scale 1/sqrt(Hd), causal mask, fp32 softmax)
@@ -46,9 +49,8 @@
 namespace dsb {
 
 namespace {
-constexpr int HD = 128;             // head width the kernels compute on
 constexpr int TR = 64;             // rows per streamed tile
-constexpr int TILE = TR * HD;      // elements per tile (16 KB)
+constexpr int TILE = TR * 128;     // elements per tile (16 KB), for either head width
 constexpr float kLog2e = 1.4426950408889634f;
 // OR-ed into the lane offset of a chunk past the head width: beyond any
 // descriptor (num_records < 2^31), so it loads zeros
@@ -103,14 +105,15 @@ DSB_DEV void load_first_two(const SeqTiles& tk, const SeqTiles& tv, int nt, int 
   }
 }
 
-// Row fragments of one global row (lane's row, 8 × 16 columns) straight to
-// registers; columns from hd on (and rows that are not ok) are zeros.
+// Row fragments of one global row (lane's row, KK × 16 columns) straight to
+// registers; rows that are not ok are zeros.
+template <int KK>
 DSB_DEV void load_row_frags(const bf16* base, long ld, long row, int col0, bool ok, int lh,
-                            int hd, bf16x8 (&f)[8]) {
+                            bf16x8 (&f)[KK]) {
   const bf16* p = base + (ok ? row * ld + col0 : 0L);
 #pragma unroll
-  for (int kk = 0; kk < 8; ++kk) {
-    f[kk] = kk * 16 < hd ? *reinterpret_cast<const bf16x8*>(p + kk * 16 + lh * 8) : bf16x8{};
+  for (int kk = 0; kk < KK; ++kk) {
+    f[kk] = *reinterpret_cast<const bf16x8*>(p + kk * 16 + lh * 8);
     if (!ok) f[kk] = bf16x8{};
   }
 }
@@ -177,32 +180,34 @@ DSB_DEV QBlock q_block(const AttnArgs& a, int w) {
 }
 
 // acc += mfma(a, b) with the accumulator held in AGPRs (inline asm): the
-// dK/dV pass keeps its 128 long-lived accumulators there, while this
+// dK/dV pass keeps its long-lived accumulators there, while this
 // translation unit is compiled with MFMA results in VGPRs
 // (-amdgpu-mfma-vgpr-form), so the S/dP scores the softmax reads need no
 // AGPR-to-VGPR copies. The leading s_nop gives the VALU writes of a and b
 // (the bf16 packs of P and dS) their wait states before the MFMA reads them;
-// accumulations into one register tuple are at least 8 MFMAs apart.
+// accumulations into one register tuple are at least 4 MFMAs apart.
 DSB_DEV void mfma32_acc(f32x16& acc, bf16x8 a, bf16x8 b) {
   asm volatile("s_nop 2\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
 }
 
-// Store a wave's 32 rows × 128 columns, held in the 32×32 accumulator layout
+// Store a wave's 32 rows × 32·DF columns, held in the 32×32 accumulator layout
 // (lane l: row l%32, columns 32·d4 + 8·(e/4) + 4·(l/32) + e%4 of acc[d4][e]),
 // as bf16(scale·x) through the wave's LDS region `buf` (32 rows at a pitch of
 // kRowPitch elements): the lanes write their pieces there, then read back 16
-// contiguous bytes each and store whole 256-byte rows, four rows per store
-// instruction (storing the 8-byte pieces directly scatters every instruction
-// over 32 rows). Rows r >= nvalid and columns from ncol on are not stored.
+// contiguous bytes each and store whole rows of a head, four or eight per
+// store instruction (storing the 8-byte pieces directly scatters every instruction
+// over 32 rows). Rows r >= nvalid are not stored.
 // With `res`, the bf16 rounding residual bf16(x − bf16(x)) goes to res (same
 // row stride) after.
 constexpr int kRowPitch = 136;  // 272 bytes: rows 16 apart share LDS banks, at most 2-way
-DSB_DEV void store_rows32(const f32x16 (&acc)[4], float scale, bf16* buf, bf16* out, long ld,
-                          int nvalid, int ncol, int lane, bf16* res = nullptr) {
+template <int DF>
+DSB_DEV void store_rows32(const f32x16 (&acc)[DF], float scale, bf16* buf, bf16* out, long ld,
+                          int nvalid, int lane, bf16* res = nullptr) {
+  constexpr int CPR = 4 * DF;  // 16-byte chunks of a row
   const int lr = lane & 31, lh = lane >> 5;
   for (int pass = 0; pass < (res ? 2 : 1); ++pass) {
 #pragma unroll
-    for (int d4 = 0; d4 < 4; ++d4)
+    for (int d4 = 0; d4 < DF; ++d4)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         bf16x4 v;
@@ -216,10 +221,10 @@ DSB_DEV void store_rows32(const f32x16 (&acc)[4], float scale, bf16* buf, bf16* 
       }
     bf16* dst = pass == 0 ? out : res;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const int c = lane + 64 * i, r = c >> 4, col = (c & 15) * 8;
+    for (int i = 0; i < CPR / 2; ++i) {
+      const int c = lane + 64 * i, r = c / CPR, col = (c % CPR) * 8;
       const bf16x8 v = *reinterpret_cast<const bf16x8*>(buf + r * kRowPitch + col);
-      if (r < nvalid && col < ncol) *reinterpret_cast<bf16x8*>(dst + (long)r * ld + col) = v;
+      if (r < nvalid) *reinterpret_cast<bf16x8*>(dst + (long)r * ld + col) = v;
     }
   }
 }
@@ -231,12 +236,12 @@ DSB_DEV void store_rows32(const f32x16 (&acc)[4], float scale, bf16* buf, bf16* 
 // packed tokens and 32 heads; now 89.)
 constexpr int kRowPitchF = 36;
 static_assert(32 * kRowPitchF * 4 <= 32 * kRowPitch * 2, "fp32 rows fit the wave's region");
-DSB_DEV void store_rows32_f32(const f32x16 (&acc)[4], float scale, float* buf, float* out, long ld,
-                              int nvalid, int ncol, int lane) {
+template <int DF>
+DSB_DEV void store_rows32_f32(const f32x16 (&acc)[DF], float scale, float* buf, float* out, long ld,
+                              int nvalid, int lane) {
   const int lr = lane & 31, lh = lane >> 5;
 #pragma unroll
-  for (int d4 = 0; d4 < 4; ++d4) {
-    if (d4 * 32 >= ncol) break;
+  for (int d4 = 0; d4 < DF; ++d4) {
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       f32x4 v;
@@ -265,7 +270,9 @@ DSB_DEV bf16x8 pack_chunk(const f32x16& s, int c) {
 // Block: 4 waves × 32 queries (q_block layout) of one kv head's q-heads;
 // streams the kv head's K/V tiles. LDS: 2 stages × (K tile + V tile) = 64 KB
 // → 2 blocks per CU.
+template <int HW>
 __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
+  constexpr int hd = HW, KK = HW / 16, DF = HW / 32;
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const QBlock qb = q_block(a, w);
@@ -275,13 +282,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
   const int qpos = qb.q0 + lr;
   const bool qok = qpos < L;
 
-  const int hd = a.hd;
-  bf16x8 qf[8];
-  load_row_frags(a.q, a.ldq, st + qpos, h * hd, qok, lh, hd, qf);
+  bf16x8 qf[KK];
+  load_row_frags(a.q, a.ldq, st + qpos, h * hd, qok, lh, qf);
 
-  f32x16 o[4];
+  f32x16 o[DF];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < DF; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o[i][r] = 0.f;
   float m_i = -INFINITY, l_i = 0.f;
@@ -318,13 +324,13 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
     // under the MFMAs.
     f32x16 s[2] = {};
     {
-      bf16x8 kfr[16];
+      bf16x8 kfr[2 * KK];
 #pragma unroll
       for (int i = 0; i < 4; ++i) kfr[i] = row_frag(sK, fo, (i & 1) * 32, i >> 1);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
+      for (int i = 0; i < 2 * KK; ++i) {
         __builtin_amdgcn_sched_barrier(0);
-        if (i + 4 < 16) kfr[i + 4] = row_frag(sK, fo, ((i + 4) & 1) * 32, (i + 4) >> 1);
+        if (i + 4 < 2 * KK) kfr[i + 4] = row_frag(sK, fo, ((i + 4) & 1) * 32, (i + 4) >> 1);
         __builtin_amdgcn_sched_barrier(0);
         s[i & 1] = mfma32(kfr[i], qf[i >> 1], s[i & 1]);
       }
@@ -357,7 +363,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
       const float alpha = m_i == -INFINITY ? 0.f : fast_exp2(m_i - m_new);
       l_i *= alpha;
 #pragma unroll
-      for (int df = 0; df < 4; ++df)
+      for (int df = 0; df < DF; ++df)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[df][r] *= alpha;
       m_i = m_new;
@@ -377,12 +383,12 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
     l_i += rs;
 #pragma unroll
     for (int kc = 0; kc < 4; ++kc) {
-      bf16x8 vfr[4];
+      bf16x8 vfr[DF];
 #pragma unroll
-      for (int df = 0; df < 4; ++df) vfr[df] = tr_frag(sV, fo, kc * 16, df);
+      for (int df = 0; df < DF; ++df) vfr[df] = tr_frag(sV, fo, kc * 16, df);
       const bf16x8 pb = pack_chunk(s[kc >> 1], kc & 1);
 #pragma unroll
-      for (int df = 0; df < 4; ++df) o[df] = mfma32(vfr[df], pb, o[df]);
+      for (int df = 0; df < DF; ++df) o[df] = mfma32(vfr[df], pb, o[df]);
     }
   }
   for (int t = nt_w; t < nt; ++t) advance(t);
@@ -393,11 +399,11 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(AttnArgs a) {
   if (nt_w > 0) {
     const float inv_l = 1.f / l_i;
     const long r0 = (long)(st + qb.q0) * a.ldc + h * hd;
-    store_rows32(o, inv_l, smem + w * 32 * kRowPitch, a.ctx + r0, a.ldc, L - qb.q0, hd, lane,
+    store_rows32(o, inv_l, smem + w * 32 * kRowPitch, a.ctx + r0, a.ldc, L - qb.q0, lane,
                  a.ores ? a.ores + r0 : nullptr);
     if (a.o32)
       store_rows32_f32(o, inv_l, reinterpret_cast<float*>(smem + w * 32 * kRowPitch),
-                       a.o32 + (long)(st + qb.q0) * a.ldo32 + h * hd, a.ldo32, L - qb.q0, hd, lane);
+                       a.o32 + (long)(st + qb.q0) * a.ldo32 + h * hd, a.ldo32, L - qb.q0, lane);
   }
   if (qok && lh == 0) a.lse[(long)h * a.ld_stat + st + qpos] = m_i + log2f(l_i);
 }
@@ -462,7 +468,9 @@ __global__ __launch_bounds__(256) void attn_dsum_kernel(AttnArgs a) {
 // ---------------------------------------------------------------- dQ
 // Block: 4 waves × 32 queries (q_block layout) of one kv head's q-heads;
 // streams the kv head's K/V tiles. dQ = scale · dS·K.
+template <int HW>
 __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnArgs a) {
+  constexpr int hd = HW, KK = HW / 16, DF = HW / 32;
   const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, lh = lane >> 5;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const QBlock qb = q_block(a, w);
@@ -472,10 +480,9 @@ __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnArgs a) {
   const int qpos = qb.q0 + lr;
   const bool qok = qpos < L;
 
-  const int hd = a.hd;
-  bf16x8 qf[8], df_[8];
-  load_row_frags(a.q, a.ldq, st + qpos, h * hd, qok, lh, hd, qf);
-  load_row_frags(a.dout, a.lddo, st + qpos, h * hd, qok, lh, hd, df_);
+  bf16x8 qf[KK], df_[KK];
+  load_row_frags(a.q, a.ldq, st + qpos, h * hd, qok, lh, qf);
+  load_row_frags(a.dout, a.lddo, st + qpos, h * hd, qok, lh, df_);
   const float lse2 = qok ? a.lse[(long)h * a.ld_stat + st + qpos] : 0.f;
   const float dsum = qok ? a.dsum[(long)h * a.ld_stat + st + qpos] : 0.f;
   const FragOffs fo(lane);
@@ -483,9 +490,9 @@ __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnArgs a) {
   const unsigned lds0 = lds_addr(smem);
   load_first_two(tk, tv, qb.nt, kvh * hd, lds0, w);
 
-  f32x16 dq[4];
+  f32x16 dq[DF];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < DF; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) dq[i][r] = 0.f;
   const float sl2 = a.scale * kLog2e;
@@ -516,16 +523,16 @@ __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnArgs a) {
     f32x16 s[2] = {}, dp[2] = {};
 #pragma unroll
     for (int kf = 0; kf < 2; ++kf) {
-      bf16x8 kfr[8], vfr[8];
+      bf16x8 kfr[KK], vfr[KK];
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         kfr[kk] = row_frag(sK, fo, kf * 32, kk);
         vfr[kk] = row_frag(sV, fo, kf * 32, kk);
       }
 #pragma unroll
-      for (int kk = 0; kk < 8; ++kk) {
+      for (int kk = 0; kk < KK; ++kk) {
         __builtin_amdgcn_sched_barrier(0);
-        if (kk + 2 < 8) {
+        if (kk + 2 < KK) {
           kfr[kk + 2] = row_frag(sK, fo, kf * 32, kk + 2);
           vfr[kk + 2] = row_frag(sV, fo, kf * 32, kk + 2);
         }
@@ -555,12 +562,12 @@ __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnArgs a) {
       for (int r = 0; r < 16; ++r) s[kf][r] *= dp[kf][r] - dsum;
 #pragma unroll
     for (int kc = 0; kc < 4; ++kc) {
-      bf16x8 kt[4];
+      bf16x8 kt[DF];
 #pragma unroll
-      for (int d4 = 0; d4 < 4; ++d4) kt[d4] = tr_frag(sK, fo, kc * 16, d4);
+      for (int d4 = 0; d4 < DF; ++d4) kt[d4] = tr_frag(sK, fo, kc * 16, d4);
       const bf16x8 sb = pack_chunk(s[kc >> 1], kc & 1);
 #pragma unroll
-      for (int d4 = 0; d4 < 4; ++d4) dq[d4] = mfma32(kt[d4], sb, dq[d4]);
+      for (int d4 = 0; d4 < DF; ++d4) dq[d4] = mfma32(kt[d4], sb, dq[d4]);
     }
   }
   for (int t = nt_w; t < nt; ++t) advance(t);
@@ -569,14 +576,21 @@ __global__ __launch_bounds__(256, 2) void attn_dq_kernel(AttnArgs a) {
   __syncthreads();
   if (nt_w > 0)
     store_rows32(dq, a.scale, smem + w * 32 * kRowPitch, a.dq + (long)(st + qb.q0) * a.lddq + h * hd,
-                 a.lddq, L - qb.q0, hd, lane);
+                 a.lddq, L - qb.q0, lane);
 }
 
 // ---------------------------------------------------------------- dK / dV
 // Block: 128 keys (4 waves × 32) of kv-head kvh; streams Q/dO tiles of every
 // q head of the group over the queries at or after the block's first key.
 // LDS: 2 stages × (Q tile + dO tile + lse/dsum rows) ≈ 65 KB.
+// One wave per SIMD at either head width: a 64-wide head's registers could be
+// held to 256 for two blocks per CU (128 VGPRs, 39 of the 103 AGPRs copies),
+// which took the backward 2.3-4 % longer (1338 against 1307 µs at 12193 tokens,
+// 102 against 98 at 2048).
+template <int HW>
 __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
+  constexpr int hd = HW, KK = HW / 16, DF = HW / 32;
+  constexpr int SE = 8 / KK;  // softmax elements after each MFMA of phases B and C
   const XcdPos xp = xcd_pos(a.Hkv);
   const int tile = xp.x;
   if (tile >= *a.ntiles_dev) return;
@@ -591,14 +605,13 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
   const bool kok = key < L;
   const int wk_first = k0 + w * 32;  // wave-uniform
 
-  const int hd = a.hd;
-  bf16x8 kf_[8], vf_[8];
-  load_row_frags(a.k, a.ldk, st + key, kvh * hd, kok, lh, hd, kf_);
-  load_row_frags(a.v, a.ldv, st + key, kvh * hd, kok, lh, hd, vf_);
+  bf16x8 kf_[KK], vf_[KK];
+  load_row_frags(a.k, a.ldk, st + key, kvh * hd, kok, lh, kf_);
+  load_row_frags(a.v, a.ldv, st + key, kvh * hd, kok, lh, vf_);
 
-  f32x16 dk[4], dv[4];
+  f32x16 dk[DF], dv[DF];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < DF; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dk[i][r] = 0.f; dv[i][r] = 0.f; }
   const float sl2 = a.scale * kLog2e;
@@ -721,7 +734,7 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
             sb[qf][r >> 3] = b;
           }
         };
-        bf16x8 qf_[8], of_[8];
+        bf16x8 qf_[KK], of_[KK];
         // Phase A: S/dP of half 0, fragment reads two chunks ahead; the last
         // two steps read the first chunks of half 1
 #pragma unroll
@@ -731,9 +744,9 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
         }
         stats(0, 0, 0);
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
+        for (int kk = 0; kk < KK; ++kk) {
           __builtin_amdgcn_sched_barrier(0);
-          const int nk = (kk + 2) & 7, nr = kk + 2 < 8 ? 0 : 32;
+          const int nk = (kk + 2) % KK, nr = kk + 2 < KK ? 0 : 32;
           qf_[nk] = row_frag(cQ, fo, nr, nk);
           of_[nk] = row_frag(cO, fo, nr, nk);
           __builtin_amdgcn_sched_barrier(0);
@@ -753,19 +766,21 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
         };
         mask(s0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        // Phase B: S/dP of half 1; P, dS of half 0 one element after each MFMA
+        // Phase B: S/dP of half 1; P, dS of half 0 in order after its MFMAs
 #pragma unroll
-        for (int kk = 0; kk < 8; ++kk) {
+        for (int kk = 0; kk < KK; ++kk) {
           __builtin_amdgcn_sched_barrier(0);
-          if (kk + 2 < 8) {
+          if (kk + 2 < KK) {
             qf_[kk + 2] = row_frag(cQ, fo, 32, kk + 2);
             of_[kk + 2] = row_frag(cO, fo, 32, kk + 2);
           }
           s1 = mfma32(qf_[kk], kf_[kk], s1);
-          soft(s0, d0, 0, 2 * kk);
+#pragma unroll
+          for (int e = 0; e < SE; ++e) soft(s0, d0, 0, 2 * kk * SE + e);
           __builtin_amdgcn_sched_barrier(0);
           d1 = mfma32(of_[kk], vf_[kk], d1);
-          soft(s0, d0, 0, 2 * kk + 1);
+#pragma unroll
+          for (int e = 0; e < SE; ++e) soft(s0, d0, 0, (2 * kk + 1) * SE + e);
           __builtin_amdgcn_sched_barrier(0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -777,11 +792,11 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
         ot[0] = tr_frag(cO, fo, 0, 0);
         qt[0] = tr_frag(cQ, fo, 0, 0);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int c = i >> 2, d4 = i & 3;
+        for (int i = 0; i < 2 * DF; ++i) {
+          const int c = i / DF, d4 = i % DF;
           __builtin_amdgcn_sched_barrier(0);
-          if (i + 1 < 8) {
-            const int c1 = (i + 1) >> 2, e1 = (i + 1) & 3;
+          if (i + 1 < 2 * DF) {
+            const int c1 = (i + 1) / DF, e1 = (i + 1) % DF;
             ot[(i + 1) & 1] = tr_frag(cO, fo, c1 * 16, e1);
             qt[(i + 1) & 1] = tr_frag(cQ, fo, c1 * 16, e1);
           } else {
@@ -789,19 +804,21 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
             qt[0] = tr_frag(cQ, fo, 32, 0);
           }
           mfma32_acc(dv[d4], ot[i & 1], pb[0][c]);
-          soft(s1, d1, 1, 2 * i);
+#pragma unroll
+          for (int e = 0; e < SE; ++e) soft(s1, d1, 1, 2 * i * SE + e);
           __builtin_amdgcn_sched_barrier(0);
           mfma32_acc(dk[d4], qt[i & 1], sb[0][c]);
-          soft(s1, d1, 1, 2 * i + 1);
+#pragma unroll
+          for (int e = 0; e < SE; ++e) soft(s1, d1, 1, (2 * i + 1) * SE + e);
           __builtin_amdgcn_sched_barrier(0);
         }
         // Phase D: dV/dK of half 1
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const int c = i >> 2, d4 = i & 3;
+        for (int i = 0; i < 2 * DF; ++i) {
+          const int c = i / DF, d4 = i % DF;
           __builtin_amdgcn_sched_barrier(0);
-          if (i + 1 < 8) {
-            const int c1 = (i + 1) >> 2, e1 = (i + 1) & 3;
+          if (i + 1 < 2 * DF) {
+            const int c1 = (i + 1) / DF, e1 = (i + 1) % DF;
             ot[(i + 1) & 1] = tr_frag(cO, fo, 32 + c1 * 16, e1);
             qt[(i + 1) & 1] = tr_frag(cQ, fo, 32 + c1 * 16, e1);
           }
@@ -822,17 +839,16 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
   // checks) complete before their AGPRs are read
   asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
   if (hs > 1) {
-    // fp32 partials: kv_part[z][row][m·KV + kvh·128 + dim], m = 0 dK, 1 dV;
+    // fp32 partials: kv_part[z][row][m·KV + kvh·hd + dim], m = 0 dK, 1 dV;
     // the lane holds key row `key`, dims d4·32 + 8g + 4·lh .. +3
     if (kok) {
       const long KV = (long)a.Hkv * hd;
       float* pr = a.kv_part + ((long)blockIdx.z * a.n + st + key) * 2 * KV + kvh * hd + 4 * lh;
       const float ks = a.scale;
 #pragma unroll
-      for (int d4 = 0; d4 < 4; ++d4)
+      for (int d4 = 0; d4 < DF; ++d4)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          if (d4 * 32 + 8 * g >= hd) continue;
           const f32x4 k4 = {dk[d4][4 * g] * ks, dk[d4][4 * g + 1] * ks, dk[d4][4 * g + 2] * ks,
                             dk[d4][4 * g + 3] * ks};
           const f32x4 v4 = {dv[d4][4 * g], dv[d4][4 * g + 1], dv[d4][4 * g + 2], dv[d4][4 * g + 3]};
@@ -848,9 +864,8 @@ __global__ __launch_bounds__(256, 1) void attn_dkdv_kernel(AttnArgs a) {
   if (wk_first < L) {
     bf16* buf = smem + w * 32 * kRowPitch;
     const long row0 = st + wk_first;
-    store_rows32(dk, a.scale, buf, a.dk + row0 * a.lddk + kvh * hd, a.lddk, L - wk_first, hd,
-                 lane);
-    store_rows32(dv, 1.f, buf, a.dv + row0 * a.lddv + kvh * hd, a.lddv, L - wk_first, hd, lane);
+    store_rows32(dk, a.scale, buf, a.dk + row0 * a.lddk + kvh * hd, a.lddk, L - wk_first, lane);
+    store_rows32(dv, 1.f, buf, a.dv + row0 * a.lddv + kvh * hd, a.lddv, L - wk_first, lane);
   }
 }
 
@@ -876,8 +891,8 @@ __global__ __launch_bounds__(256) void dkdv_head_sum_kernel(AttnArgs a, int hs) 
 
 hipError_t attn_fwd(const AttnArgs& a, hipStream_t s) {
   if (a.max_tiles <= 0) return hipSuccess;
-  hipLaunchKernelGGL(attn_fwd_kernel, dim3(a.max_tiles * (a.Hq / a.Hkv), a.Hkv), dim3(256), 0, s,
-                     a);
+  hipLaunchKernelGGL(a.hd == 64 ? attn_fwd_kernel<64> : attn_fwd_kernel<128>,
+                     dim3(a.max_tiles * (a.Hq / a.Hkv), a.Hkv), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -893,7 +908,8 @@ hipError_t attn_bwd_dkdv(const AttnArgs& a, hipStream_t s) {
   // and kv head, far fewer than the CUs; each block then takes one q-head
   // of its group and a second launch adds the heads' fp32 partials in order.
   const int hs = a.kv_part ? attn_dkdv_head_split(a) : 1;
-  hipLaunchKernelGGL(attn_dkdv_kernel, dim3(a.max_tiles, a.Hkv, hs), dim3(256), 0, s, a);
+  hipLaunchKernelGGL(a.hd == 64 ? attn_dkdv_kernel<64> : attn_dkdv_kernel<128>,
+                     dim3(a.max_tiles, a.Hkv, hs), dim3(256), 0, s, a);
   if (hs == 1 || a.kv_defer) return hipGetLastError();
   const long tot = (long)a.n * (2L * a.Hkv * a.hd / 4);
   hipLaunchKernelGGL(dkdv_head_sum_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, s,
@@ -903,8 +919,8 @@ hipError_t attn_bwd_dkdv(const AttnArgs& a, hipStream_t s) {
 
 hipError_t attn_bwd_dq(const AttnArgs& a, hipStream_t s) {
   if (a.max_tiles <= 0) return hipSuccess;
-  hipLaunchKernelGGL(attn_dq_kernel, dim3(a.max_tiles * (a.Hq / a.Hkv), a.Hkv), dim3(256), 0, s,
-                     a);
+  hipLaunchKernelGGL(a.hd == 64 ? attn_dq_kernel<64> : attn_dq_kernel<128>,
+                     dim3(a.max_tiles * (a.Hq / a.Hkv), a.Hkv), dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
