@@ -243,7 +243,7 @@ def test_rope_fwd_bwd(qk_norm, hd):
 
 # group sizes Hq/Hkv 1..8: forward and dQ blocks take four (32-query subtile,
 # q-head) pairs of one kv head, so G = 3 and 5 mix subtiles within a block
-# head_dim 64 (last three cases): heads zero-padded to 128 inside the kernels
+# head_dim 64 (last three cases): the kernels' 64-wide instantiation
 @pytest.mark.parametrize("seq_lens,Hq,Hkv,hd", [([37, 128, 1, 200, 64], 4, 2, 128),
                                                 ([300], 8, 2, 128), ([5, 129, 256], 2, 1, 128),
                                                 ([1, 1, 2], 4, 4, 128),

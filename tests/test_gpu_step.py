@@ -37,7 +37,7 @@ def test_cycle_parity_7proj(family):
 @pytest.mark.parametrize("family", ["llama3", "qwen3"])
 def test_cycle_parity_head_dim_64(family):
     """head_dim 64 (Llama-3.2-1B's): RoPE over 32-wide halves, the q/k norm
-    over 64 dims (Qwen3), attention on heads zero-padded to 128 with scale
+    over 64 dims (Qwen3), attention on 64-wide heads with scale
     1/8, and the qkv / o widths of 64-dim heads; GQA group of 4."""
     meta = tiny_meta(family=family, L=2, D=512, Hq=8, Hkv=2, Hd=64, I=768)
     worst = _run(meta, [37, 128, 1, 200, 64])
