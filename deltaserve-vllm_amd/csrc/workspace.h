@@ -2,7 +2,7 @@
 // staging kept between calls, because hipMalloc, hipFree (which waits for the
 // whole device) and a synchronous copy each cost more than most of the ops'
 // kernels (attention forward, 8192 packed tokens: 164 µs per call with them,
-// 130 without; its kernel is 105).
+// 130 without; its kernel took 105 of them then).
 //
 // A block belongs to one call at a time: a Scratch takes it from the pool of
 // its device under the pool's lock and gives it back only once the call's
