@@ -12,18 +12,26 @@
 // reference M that is known before the first product:
 //   ce_init: M = the row's target logit (a dot of the row with W[target]);
 //   per chunk c: logits = H·W_cᵀ (GEMM; its epilogue writes P = bf16(exp(logit
-//     − M)) and, per wave-wide run of vocabulary columns, Σ exp(logit − M).
-//     Any reference within a few tens of the row maximum serves: bf16 and
-//     fp32 keep their relative precision over that range. Only where a sum
-//     passes 2^57 (a logit more than about 40 above M) does the run take its
-//     own maximum m_t as its reference instead);
+//     − M)) and, per wave-wide run of vocabulary columns, Σ exp(logit − M),
+//     both over the columns other than the target's, whose logit x_t goes out
+//     by itself. Any reference within a few tens of the row maximum serves:
+//     bf16 and fp32 keep their relative precision over that range. Only where
+//     a sum passes 2^57 (a logit more than about 40 above M) does the run take
+//     its own maximum m_t as its reference instead);
 //   ce_rescale: per row L += Σ_t s_t·e^(m_t − M) and, on the rows where some
 //     m_t differs from M, M' = max_t m_t, α = e^(M − M') and P scaled in place
 //     to M';
 //   dH = dH·α + P·W_c (GEMM, fp32 accumulate with the per-row α);
-//   after the last chunk: dH = (dH/L − W[target]) / n_valid (the onehot term
-//   exactly, in fp32), LSE = M + ln L, loss_row = LSE − target logit, and a
+//   after the last chunk, with e_t = exp(x_t − M): loss_row = ln(1 + L/e_t),
+//   dH = (dH − L·W[target]) / (e_t + L) / n_valid, LSE = M + ln(e_t + L), and a
 //   single-block deterministic sum gives the cycle loss.
+// The target's term stays out of the sums because softmax − onehot cancels
+// there: with p_t near 1 the row's loss and its coefficient of W[target],
+// p_t − 1, are L/e_t and −L/(e_t + L), full precision in L, while e_t + L
+// rounds L away and M, the dot, differs from x_t by the order of its sum. At
+// 1 − p_t = 5e-5 on average (298 rows, target logits near 18, 4096 wide, 2000
+// words) sums over all columns gave each row's dH an error of 29 % on average
+// and the loss one of 1 %; now 6e-5 and 6e-7.
 // With the tile maxima as references (every row of the first chunk rescaled,
 // later ones where the row maximum lay in the chunk) the rescale took 48 µs
 // per chunk at 8192 rows and 14 µs at 504, whose rows' serial passes over P
@@ -50,9 +58,12 @@ constexpr float kSumLimit = 0x1p57f;
 // Per run of TN vocabulary columns (a wave tile's width) of chunk [c0, c0 + Vc)
 // and row: (reference m_t, Σ exp(logit − m_t)) into stats[m, (c0 + column) / TN]
 // and P[m, j] = bf16(exp(logit[m, c0 + j] − m_t)) for the chunk's columns
-// j < Vc; columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are written as zero so the
-// dH product runs its K loop over whole 16-byte chunks. m_t is run_m[m] unless
-// the run's sum passes kSumLimit (or is NaN), then the run's maximum.
+// j < Vc; the row's target column counts as zero in both, its logit goes to
+// tgt_logit[m]. Columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are written as zero so
+// the dH product runs its K loop over whole 16-byte chunks. m_t is run_m[m]
+// unless the run's sum passes kSumLimit (or is NaN), then the run's maximum.
+// Runs that hold a target (one in V / TN of a row's) or pass the limit take the
+// exponentials a second time; the others test neither per element.
 // A lane holds 4·FN values of a row, so the exponentials and the row sums are
 // taken in the accumulator layout (two shuffles per row) and only bf16 values
 // are staged for the row-contiguous stores; no barrier, each wave its own
@@ -69,6 +80,8 @@ struct EpiCEProb {
   long ldp;
   int c0, Vc, Nc8;
   const float* run_m;
+  const int* labels;
+  float* tgt_logit;
   template <int FM, int FN, int WM, int WN>
   DSB_DEV void run(const f32x4 (&acc)[FM][FN], int mw, int nw, int M, int lane, int wave,
                    void* smem) const {
@@ -78,11 +91,16 @@ struct EpiCEProb {
     const bool whole = nw + TN <= Vc;
     const int run = (c0 + nw) / TN;
     bf16* buf = reinterpret_cast<bf16*>(smem) + wave * 32 * PITCH;
-    // the rows' references, all loaded before the first is used (rows past M
-    // read row M − 1 and are not stored)
+    // the rows' references and target columns, all loaded before the first is
+    // used (rows past M read row M − 1 and are not stored)
     float ref0[FM];
+    int tcol[FM];  // within the run; outside [0, TN): not in it (label −1: negative)
 #pragma unroll
-    for (int fm = 0; fm < FM; ++fm) ref0[fm] = run_m[min(mw + fm * 16 + l16, M - 1)];
+    for (int fm = 0; fm < FM; ++fm) {
+      const int m = min(mw + fm * 16 + l16, M - 1);
+      ref0[fm] = run_m[m];
+      tcol[fm] = labels[m] - (c0 + nw);
+    }
 #pragma unroll
     for (int b = 0; b < FM / 2; ++b) {
       if (mw + b * 32 >= M) break;  // uniform: the rest of the wave tile is past M
@@ -90,8 +108,11 @@ struct EpiCEProb {
       for (int h = 0; h < 2; ++h) {
         const int fm = 2 * b + h;
         bf16x4 pk[FN];
-        // lane: row l16, columns 16·fn + 4·lq + i
-        auto take = [&](float ref) {
+        // lane: row l16, columns 16·fn + 4·lq + i; with `skips` column 4·lq + tl
+        // counts as zero (a factor min(|column − target|, 1): as per-element
+        // tests the masks of 128 columns spill)
+        const float tl = (float)(tcol[fm] - 4 * lq);
+        auto take = [&](float ref, auto skips) {
           float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
@@ -99,6 +120,7 @@ struct EpiCEProb {
             for (int i = 0; i < 4; ++i) {
               float e = __expf(acc[fm][fn][i] - ref);
               if (!whole) e = nw + fn * 16 + 4 * lq + i < Vc ? e : 0.f;
+              if (decltype(skips)::value) e *= fminf(fabsf((float)(fn * 16 + i) - tl), 1.f);
               part[i] += e;
               pk[fn][i] = (bf16)e;
             }
@@ -106,25 +128,32 @@ struct EpiCEProb {
           v += __shfl_xor(v, 16, 64);
           return v + __shfl_xor(v, 32, 64);
         };
+        const int m = mw + fm * 16 + l16;
         float ref = ref0[fm];
-        float sum = take(ref);
-        if (__any(!(sum <= kSumLimit))) {
-          // rare: the rows past the limit against their run's own maximum
-          float v = -INFINITY;
+        float sum = take(ref, std::false_type{});
+        if (__any(!(sum <= kSumLimit) || (unsigned)tcol[fm] < (unsigned)TN)) {
+          // rare: rows with their target in this run, without it; rows past
+          // the limit, against their run's own maximum
+          float v = -INFINITY, xt = 0.f;
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-              v = whole || nw + fn * 16 + 4 * lq + i < Vc ? fmaxf(v, acc[fm][fn][i]) : v;
+            {
+              const float x = acc[fm][fn][i];
+              v = whole || nw + fn * 16 + 4 * lq + i < Vc ? fmaxf(v, x) : v;
+              xt = (float)(fn * 16 + i) == tl ? x : xt;
+            }
+          const int tc = tcol[fm];
+          if ((unsigned)tc < (unsigned)TN && ((tc >> 2) & 3) == lq && m < M) tgt_logit[m] = xt;
           v = fmaxf(v, __shfl_xor(v, 16, 64));
           v = fmaxf(v, __shfl_xor(v, 32, 64));
           ref = sum <= kSumLimit ? ref : fmaxf(ref, v);
-          sum = take(ref);
+          sum = take(ref, std::true_type{});
         }
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn)
           *reinterpret_cast<bf16x4*>(buf + (16 * h + l16) * PITCH + fn * 16 + 4 * lq) = pk[fn];
-        const int m = mw + fm * 16 + l16;
         if (lq == 0 && m < M) stats[(long)m * ntn + run] = make_float2(ref, sum);
       }
 #pragma unroll
@@ -146,8 +175,8 @@ constexpr int ce_run(int cfg) {
 }  // namespace
 
 // One wave per live row: the label (ids[t + 1] where row t predicts, −1
-// elsewhere; an id outside [0, V) raises err bit 1), the target logit, which is
-// also the row's first softmax reference (0 for rows without a target), and
+// elsewhere; an id outside [0, V) raises err bit 1), the row's first softmax
+// reference, a dot of the row with W[target] (0 for rows without a target), and
 // L = 0, α = 1.
 __global__ __launch_bounds__(256) void ce_init_kernel(HeadArgs a) {
   int N = a.n;
@@ -176,7 +205,6 @@ __global__ __launch_bounds__(256) void ce_init_kernel(HeadArgs a) {
   }
   if (l == 0) {
     a.labels[m] = lab;
-    a.tgt_logit[m] = dot;
     a.run_m[m] = dot;
     a.run_l[m] = 0.f;
     a.alpha[m] = 1.f;
@@ -228,10 +256,12 @@ __global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0) {
   }
 }
 
-// After the last chunk, one wave per live row: LSE = M + ln L, loss_row =
-// LSE − target logit, dH = (dH/L − W[target]) / n_valid, with dH the sum in
-// order of the `ks` accumulated K-slice partials when the product was split;
-// rows without a target get dH = 0 and no loss.
+// After the last chunk, one wave per live row: with e_t = exp(x_t − M) and the
+// other columns' sum L, loss_row = ln(1 + L/e_t) (where x_t lies far below M as
+// ln(e_t + L) − (x_t − M)), LSE = x_t + loss_row and dH = (dH − L·W[target]) /
+// (e_t + L) / n_valid, with dH the sum in order of the `ks` accumulated K-slice
+// partials when the product was split; rows without a target get dH = 0 and no
+// loss.
 __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
   int N = a.n;
   if (a.n_dev) N = min(N, *a.n_dev);
@@ -245,12 +275,15 @@ __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
     if (l == 0) a.loss_row[m] = 0.f;
     return;
   }
-  const float L = a.run_l[m], lse = a.run_m[m] + __logf(L);
+  const float L = a.run_l[m], xt = a.tgt_logit[m], d = xt - a.run_m[m], et = __expf(d);
   if (l == 0) {
-    a.lse[m] = lse;
-    a.loss_row[m] = lse - a.tgt_logit[m];
+    // M is at least the dot that x_t differs from by rounding: d is about 0, or
+    // negative where the reference moved (or NaN)
+    const float loss = d > -1.f ? log1pf(L / et) : logf(et + L) - d;
+    a.lse[m] = xt + loss;
+    a.loss_row[m] = loss;
   }
-  const float inv = 1.f / L, sc = *a.inv_nvalid;
+  const float inv = 1.f / (et + L), ct = L * inv, sc = *a.inv_nvalid;
   const bf16* w = a.W + (long)t * a.D;
   const float* src = ks > 1 ? a.part + (long)m * a.D : dr;
   const long plane = (long)a.n * a.D;
@@ -265,10 +298,10 @@ __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
       x1 += *reinterpret_cast<const f32x4*>(src + z * plane + 8 * k + 4);
     }
     f32x4* d = reinterpret_cast<f32x4*>(dr + 8 * k);
-    d[0] = f32x4{(x0[0] * inv - wf[0]) * sc, (x0[1] * inv - wf[1]) * sc,
-                 (x0[2] * inv - wf[2]) * sc, (x0[3] * inv - wf[3]) * sc};
-    d[1] = f32x4{(x1[0] * inv - wf[4]) * sc, (x1[1] * inv - wf[5]) * sc,
-                 (x1[2] * inv - wf[6]) * sc, (x1[3] * inv - wf[7]) * sc};
+    d[0] = f32x4{(x0[0] * inv - wf[0] * ct) * sc, (x0[1] * inv - wf[1] * ct) * sc,
+                 (x0[2] * inv - wf[2] * ct) * sc, (x0[3] * inv - wf[3] * ct) * sc};
+    d[1] = f32x4{(x1[0] * inv - wf[4] * ct) * sc, (x1[1] * inv - wf[5] * ct) * sc,
+                 (x1[2] * inv - wf[6] * ct) * sc, (x1[3] * inv - wf[7] * ct) * sc};
   }
 }
 
@@ -375,7 +408,8 @@ hipError_t head_init(const HeadArgs& a, hipStream_t s) {
 hipError_t head_prob(const HeadArgs& a, int c0, hipStream_t s) {
   if (a.n <= 0) return hipSuccess;
   const int Vc = min(a.vchunk, a.V - c0), Nc8 = (Vc + 7) / 8 * 8;
-  EpiCEProb epi{a.stats, a.ntn, a.dlog, (long)a.vchunk, c0, Vc, Nc8, a.run_m};
+  EpiCEProb epi{a.stats, a.ntn,   a.dlog,  (long)a.vchunk, c0,
+                Vc,      Nc8,     a.run_m, a.labels,       a.tgt_logit};
   const GemmProblem p = chunk_logits_problem(a, c0);
   switch (a.ce_cfg) {
     case GEMM_BIG: return launch_gemm_cfg<256, 256, 2, 2, 2, 3>(p, epi, s);

@@ -178,14 +178,16 @@ struct HeadArgs {
   int* labels;                    // [n] target id or -1 (head_init)
   int n; const int* n_dev;
   int D, V;
-  float2* stats;                  // [n_cap, ntn] per run of ce_bn columns (reference, sum exp)
+  // [n_cap, ntn] per run of ce_bn columns (reference, sum exp), without the
+  // row's target column
+  float2* stats;
   int ntn;                        // ceil(V / ce_bn)
   int ce_bn, ce_cfg;              // run width and tile of the logits product (head_plan)
   int dh_cfg, dh_ks;              // tile and K slices of the dH product (head_plan)
-  float* tgt_logit;               // [n_cap]
+  float* tgt_logit;               // [n_cap] from the logits product
   float* lse;                     // [n_cap] row LSE (natural log), after the last chunk
   float* run_m;                   // [n_cap] the row's softmax reference M
-  float* run_l;                   // [n_cap] running Σ exp(logit − run_m)
+  float* run_l;                   // [n_cap] running Σ exp(logit − run_m), target left out
   float* alpha;                   // [n_cap] the dH accumulator's factor for the chunk
   float* loss_row;                // [n_cap]
   float* loss_out;                // scalar: sum(loss_row)/n_valid

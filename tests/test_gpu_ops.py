@@ -552,6 +552,52 @@ def test_head_reference_moves(n, V, vchunk, std):
         assert dH.abs().max().item() == 0.0
 
 
+def _peaked_rows(n, V, D, gain, seed):
+    """Rows x = gain·W[peak] + noise: logit about 10·gain at `peak` (D = 4096),
+    N(0, 1) elsewhere."""
+    W = _bf(_rnd(V, D, seed=seed) * 0.05)
+    peak = torch.randint(0, V, (n,), generator=torch.Generator().manual_seed(seed + 1))
+    x = _bf(gain * W[peak].float() + _rnd(n, D, seed=seed + 2) * 0.3)
+    return x, W, peak
+
+
+def _row_errors(x, W, ids, seq_lens, dH):
+    """fp64 loss, and per predicting row the 2-norm error of dH relative to the row."""
+    _, _, rows, tgt, n_valid = O.pack(seq_lens)
+    logits = x.double()[rows] @ W.double().t()
+    t = ids[tgt]
+    i = torch.arange(n_valid)
+    rest = logits - logits[i, t][:, None]
+    rest[i, t] = -math.inf
+    s = rest.exp().sum(1)                      # (1 − p_t) / p_t
+    p = rest.exp() / (1 + s)[:, None]
+    ref = (p @ W.double() - (s / (1 + s))[:, None] * W.double()[t]) / n_valid
+    err = (dH.cpu().double()[rows] - ref).norm(dim=1) / ref.norm(dim=1)
+    return torch.log1p(s).mean().item(), err
+
+
+@pytest.mark.parametrize("gain", [1.0, 1.8, 3.0])
+@pytest.mark.parametrize("vchunk", [0, 512])
+def test_head_confident_rows(vchunk, gain):
+    """Rows whose target already has almost all the probability (1 − p_t about
+    0.2, 1e-4 and 1e-9): softmax − onehot cancels, so each row's dH is compared
+    by itself, 2-norm against fp64. The other columns' probabilities are bf16,
+    each within 2^-9 of itself, and so is their sum: 2^-8. The loss is a sum of
+    exp(logit − target logit), both logits fp32 sums of 4096 terms whose
+    partial sums stay below 32: off by 2^-24·32·sqrt(4096) = 1.2e-4 at most."""
+    from deltaserve_amd import ops
+    seq_lens, V = [200, 100], 2000
+    x, W, peak = _peaked_rows(sum(seq_lens), V, 4096, gain, seed=91)
+    ids = torch.roll(peak, 1)                  # row t's target is ids[t + 1]
+    loss, nv, dH = ops.head_backward(x.to(DEV), W.to(DEV), ids.to(DEV), seq_lens, vocab_chunk=vchunk)
+    want, err = _row_errors(x, W, ids, seq_lens, dH)
+    print(f"[confident rows] loss {loss:.6e} ({want:.6e}), dH error max {err.max():.2e} "
+          f"mean {err.mean():.2e}", flush=True)
+    assert nv == 298 and loss >= 0.0
+    assert abs(loss - want) < 1.2e-4 * want
+    assert err.max() < 2 ** -8
+
+
 @pytest.mark.parametrize("release", [False, True])
 def test_scratch_is_private_to_a_call(release):
     """The ops' kept scratch memory: four threads on streams of their own run
