@@ -246,8 +246,8 @@ struct dsb_handle {
   float *g32[2], *grm32;
   bf16* ores;  // bf16 rounding residual of the attention output: rowsum(dO∘O) from ctx + ores
   bf16 *normed, *dlog;
-  float2* stats;
-  float *tgt_logit, *lse_h, *loss_row, *dH, *run_m, *run_l, *alpha;
+  CEStat* stats;
+  float *tgt_logit, *lse_h, *loss_row, *dH, *run_m, *run_l, *run_r, *alpha;
   float* tn_work;
   long tn_work_elems;
   float* part = nullptr;  // split-K partials of the products with too few 256×256 tiles
@@ -422,6 +422,7 @@ int finalize(dsb_handle* h) {
   CKR(dalloc(h, &h->loss_row, NN));
   CKR(dalloc(h, &h->run_m, NN));
   CKR(dalloc(h, &h->run_l, NN));
+  CKR(dalloc(h, &h->run_r, NN));
   CKR(dalloc(h, &h->alpha, NN));
   CKR(dalloc(h, &h->dlog, NN * h->head.vchunk));
   CKR(dalloc(h, &h->dH, NN * D));
@@ -886,7 +887,7 @@ HeadArgs head_args(dsb_handle* h) {
   ha.labels = h->labels;
   ha.n_dev = &h->d_hdr->n; ha.stats = h->stats;
   ha.tgt_logit = h->tgt_logit; ha.lse = h->lse_h; ha.loss_row = h->loss_row;
-  ha.run_m = h->run_m; ha.run_l = h->run_l; ha.alpha = h->alpha;
+  ha.run_m = h->run_m; ha.run_l = h->run_l; ha.run_r = h->run_r; ha.alpha = h->alpha;
   ha.loss_out = &h->d_hdr->loss; ha.inv_nvalid = &h->d_hdr->inv_nvalid;
   ha.dlog = h->dlog; ha.dH = h->dH;
   ha.part = ha.tail_part = h->part;
@@ -2307,8 +2308,8 @@ int dsb_op_head(const void* normed, int64_t ldh, const void* lm_w, const int64_t
   head_plan(a, -1, true);
   const long NN = n + 1;
   a.labels = tmp.dev<int>(NN);
-  a.stats = tmp.dev<float2>(NN * a.ntn);
-  float* rows = tmp.dev<float>(6 * NN);
+  a.stats = tmp.dev<CEStat>(NN * a.ntn);
+  float* rows = tmp.dev<float>(7 * NN);
   a.dlog = tmp.dev<bf16>(NN * a.vchunk);
   int tail = 0;
   if (a.dh_ks == 1 && a.dh_cfg == GEMM_BIG) {
@@ -2325,6 +2326,7 @@ int dsb_op_head(const void* normed, int64_t ldh, const void* lm_w, const int64_t
     return fail(nullptr, "dsb_op_head: hipMalloc failed");
   a.tgt_logit = rows; a.lse = rows + NN; a.loss_row = rows + 2 * NN;
   a.run_m = rows + 3 * NN; a.run_l = rows + 4 * NN; a.alpha = rows + 5 * NN;
+  a.run_r = rows + 6 * NN;
   a.normed = (const bf16*)normed; a.ldh = ldh; a.W = (const bf16*)lm_w;
   a.ids = ids; a.pred = (const int*)ds; a.err = &dr->err; a.n_dev = nullptr;
   a.loss_out = &dr->loss; a.inv_nvalid = &dr->inv_nvalid; a.dH = dH;

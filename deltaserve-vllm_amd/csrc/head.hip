@@ -14,17 +14,24 @@
 //   per chunk c: logits = H·W_cᵀ (GEMM; its epilogue writes P = bf16(exp(logit
 //     − M)) and, per wave-wide run of vocabulary columns, Σ exp(logit − M),
 //     both over the columns other than the target's, whose logit x_t goes out
-//     by itself. Any reference within a few tens of the row maximum serves:
-//     bf16 and fp32 keep their relative precision over that range. Only where
+//     by itself, and the sum of the rounded P beside it. Any reference within
+//     a few tens of the row maximum serves: bf16 and fp32 keep their relative
+//     precision over that range. Only where
 //     a sum passes 2^57 (a logit more than about 40 above M) does the run take
 //     its own maximum m_t as its reference instead);
-//   ce_rescale: per row L += Σ_t s_t·e^(m_t − M) and, on the rows where some
-//     m_t differs from M, M' = max_t m_t, α = e^(M − M') and P scaled in place
-//     to M';
+//   ce_rescale: per row L += Σ_t s_t·e^(m_t − M), the rounded sum R likewise,
+//     and, on the rows where some m_t differs from M, M' = max_t m_t, α =
+//     e^(M − M') and P scaled in place to M';
 //   dH = dH·α + P·W_c (GEMM, fp32 accumulate with the per-row α);
 //   after the last chunk, with e_t = exp(x_t − M): loss_row = ln(1 + L/e_t),
-//   dH = (dH − L·W[target]) / (e_t + L) / n_valid, LSE = M + ln(e_t + L), and a
-//   single-block deterministic sum gives the cycle loss.
+//   dH = (dH·L/R − L·W[target]) / (e_t + L) / n_valid, LSE = M + ln(e_t + L),
+//   and a single-block deterministic sum gives the cycle loss.
+// L/R takes the common part of P's rounding out of dH: one column that
+// dominates the others' sum is rounded by up to 2^-9 (its exponential is 1 only
+// against a reference that is its own), and L/R restores it to fp32. 300 rows
+// with one column 17 above the sum of 2000 others: dH off by up to 2.5e-3 without
+// it, 1e-7 with. It costs a dot product with ones per two values (the head of
+// 2048 rows × 2048: 1802 and 1799 µs without and with it).
 // The target's term stays out of the sums because softmax − onehot cancels
 // there: with p_t near 1 the row's loss and its coefficient of W[target],
 // p_t − 1, are L/e_t and −L/(e_t + L), full precision in L, while e_t + L
@@ -56,9 +63,9 @@ namespace {
 constexpr float kSumLimit = 0x1p57f;
 
 // Per run of TN vocabulary columns (a wave tile's width) of chunk [c0, c0 + Vc)
-// and row: (reference m_t, Σ exp(logit − m_t)) into stats[m, (c0 + column) / TN]
-// and P[m, j] = bf16(exp(logit[m, c0 + j] − m_t)) for the chunk's columns
-// j < Vc; the row's target column counts as zero in both, its logit goes to
+// and row: (reference m_t, Σ exp(logit − m_t), Σ of those values as P holds
+// them) into stats[m, (c0 + column) / TN] and P[m, j] = bf16(exp(logit[m, c0 + j] − m_t)) for the chunk's columns
+// j < Vc; the row's target column counts as zero in all, its logit goes to
 // tgt_logit[m]. Columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are written as zero so
 // the dH product runs its K loop over whole 16-byte chunks. m_t is run_m[m]
 // unless the run's sum passes kSumLimit (or is NaN), then the run's maximum.
@@ -74,7 +81,7 @@ constexpr float kSumLimit = 0x1p57f;
 // 798 µs in the same two runs), 147 → 116 µs at 2048 × 2048 and 30.5 → 25.3 µs
 // at 504 × 1024.
 struct EpiCEProb {
-  float2* stats;
+  CEStat* stats;
   int ntn;
   bf16* P;
   long ldp;
@@ -113,7 +120,7 @@ struct EpiCEProb {
         // tests the masks of 128 columns spill)
         const float tl = (float)(tcol[fm] - 4 * lq);
         auto take = [&](float ref, auto skips) {
-          float part[4] = {0.f, 0.f, 0.f, 0.f};
+          float part[4] = {0.f, 0.f, 0.f, 0.f}, rpart[2] = {0.f, 0.f};
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
@@ -123,15 +130,20 @@ struct EpiCEProb {
               if (decltype(skips)::value) e *= fminf(fabsf((float)(fn * 16 + i) - tl), 1.f);
               part[i] += e;
               pk[fn][i] = (bf16)e;
+              if (i & 1) {  // two rounded values per instruction: their dot with ones
+                const bf16x2 two = {pk[fn][i - 1], pk[fn][i]}, ones = {(bf16)1.f, (bf16)1.f};
+                rpart[i >> 1] = __builtin_amdgcn_fdot2_f32_bf16(two, ones, rpart[i >> 1], false);
+              }
             }
           float v = (part[0] + part[1]) + (part[2] + part[3]);
+          float r = rpart[0] + rpart[1];
           v += __shfl_xor(v, 16, 64);
-          return v + __shfl_xor(v, 32, 64);
+          r += __shfl_xor(r, 16, 64);
+          return CEStat{ref, v + __shfl_xor(v, 32, 64), r + __shfl_xor(r, 32, 64)};
         };
         const int m = mw + fm * 16 + l16;
-        float ref = ref0[fm];
-        float sum = take(ref, std::false_type{});
-        if (__any(!(sum <= kSumLimit) || (unsigned)tcol[fm] < (unsigned)TN)) {
+        CEStat st = take(ref0[fm], std::false_type{});
+        if (__any(!(st.sum <= kSumLimit) || (unsigned)tcol[fm] < (unsigned)TN)) {
           // rare: rows with their target in this run, without it; rows past
           // the limit, against their run's own maximum
           float v = -INFINITY, xt = 0.f;
@@ -148,13 +160,12 @@ struct EpiCEProb {
           if ((unsigned)tc < (unsigned)TN && ((tc >> 2) & 3) == lq && m < M) tgt_logit[m] = xt;
           v = fmaxf(v, __shfl_xor(v, 16, 64));
           v = fmaxf(v, __shfl_xor(v, 32, 64));
-          ref = sum <= kSumLimit ? ref : fmaxf(ref, v);
-          sum = take(ref, std::true_type{});
+          st = take(st.sum <= kSumLimit ? st.ref : fmaxf(st.ref, v), std::true_type{});
         }
 #pragma unroll
         for (int fn = 0; fn < FN; ++fn)
           *reinterpret_cast<bf16x4*>(buf + (16 * h + l16) * PITCH + fn * 16 + 4 * lq) = pk[fn];
-        if (lq == 0 && m < M) stats[(long)m * ntn + run] = make_float2(ref, sum);
+        if (lq == 0 && m < M) stats[(long)m * ntn + run] = st;
       }
 #pragma unroll
       for (int it = 0; it < 32 * CG / 64; ++it) {
@@ -177,7 +188,7 @@ constexpr int ce_run(int cfg) {
 // One wave per live row: the label (ids[t + 1] where row t predicts, −1
 // elsewhere; an id outside [0, V) raises err bit 1), the row's first softmax
 // reference, a dot of the row with W[target] (0 for rows without a target), and
-// L = 0, α = 1.
+// L = R = 0, α = 1.
 __global__ __launch_bounds__(256) void ce_init_kernel(HeadArgs a) {
   int N = a.n;
   if (a.n_dev) N = min(N, *a.n_dev);
@@ -206,16 +217,16 @@ __global__ __launch_bounds__(256) void ce_init_kernel(HeadArgs a) {
   if (l == 0) {
     a.labels[m] = lab;
     a.run_m[m] = dot;
-    a.run_l[m] = 0.f;
+    a.run_l[m] = a.run_r[m] = 0.f;
     a.alpha[m] = 1.f;
   }
 }
 
 // Chunk [c0, c0 + Vc) after its logits product, one wave per live row: the
-// runs' largest reference M_c, the row's reference M and sum L moved to
+// runs' largest reference M_c, the row's reference M and sums L and R moved to
 // M' = max(M, M_c), α = e^(M − M') for the dH accumulator, and, on rows where
 // some run's reference is not M', P scaled in place by e^(m_t − M') so that
-// P = bf16(exp(logit − M')). Rows without a target keep their P: the finalize
+// P = bf16(exp(logit − M')), R then taking the sum of the rounded products. Rows without a target keep their P: the finalize
 // sets their dH to zero whatever the product accumulated.
 __global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0) {
   int N = a.n;
@@ -224,42 +235,56 @@ __global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0) {
   if (m >= N) return;
   const int bn = a.ce_bn, Vc = min(a.vchunk, a.V - c0), Nc8 = (Vc + 7) / 8 * 8;
   const int nt = (Vc + bn - 1) / bn;
-  const float2* st = a.stats + (long)m * a.ntn + c0 / bn;
+  const CEStat* st = a.stats + (long)m * a.ntn + c0 / bn;
   const float mo = a.run_m[m];
   float mc = -INFINITY;
-  for (int j = l; j < nt; j += 64) mc = fmaxf(mc, st[j].x);
+  for (int j = l; j < nt; j += 64) mc = fmaxf(mc, st[j].ref);
   mc = wave_max(mc);
   const float mn = fmaxf(mo, mc);
-  float sc = 0.f;
-  for (int j = l; j < nt; j += 64) sc += st[j].y * __expf(st[j].x - mn);
+  float sc = 0.f, rs = 0.f;
+  bool scaled = false;
+  for (int j = l; j < nt; j += 64) {
+    const CEStat s = st[j];
+    sc += s.sum * __expf(s.ref - mn);
+    rs += s.rsum;
+    scaled |= s.ref != mn;
+  }
   sc = wave_sum(sc);
+  rs = wave_sum(rs);
+  const float al = __expf(mo - mn);
   if (l == 0) {
-    const float al = __expf(mo - mn);
     a.run_m[m] = mn;
     a.run_l[m] = a.run_l[m] * al + sc;
     a.alpha[m] = al;
   }
   if (a.labels[m] < 0) return;
-  bool scaled = false;
-  for (int j = l; j < nt; j += 64) scaled |= st[j].x != mn;
-  if (!__any(scaled)) return;
+  if (!__any(scaled)) {
+    if (l == 0) a.run_r[m] = a.run_r[m] * al + rs;
+    return;
+  }
+  rs = 0.f;
   bf16* pr = a.dlog + (long)m * a.vchunk;
 #pragma unroll 4
   for (int k = l; k < Nc8 / 8; k += 64) {
     u32x4* q = reinterpret_cast<u32x4*>(pr + 8 * k);
-    const float f = __expf(st[(8 * k) / bn].x - mn);
+    const float f = __expf(st[(8 * k) / bn].ref - mn);
     float v[8];
     unpack8(*q, v);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] *= f;
+    for (int e = 0; e < 8; ++e) {
+      v[e] = (float)(bf16)(v[e] * f);
+      rs += v[e];
+    }
     *q = pack8(v);
   }
+  rs = wave_sum(rs);
+  if (l == 0) a.run_r[m] = a.run_r[m] * al + rs;
 }
 
 // After the last chunk, one wave per live row: with e_t = exp(x_t − M) and the
 // other columns' sum L, loss_row = ln(1 + L/e_t) (where x_t lies far below M as
-// ln(e_t + L) − (x_t − M)), LSE = x_t + loss_row and dH = (dH − L·W[target]) /
-// (e_t + L) / n_valid, with dH the sum in order of the `ks` accumulated K-slice
+// ln(e_t + L) − (x_t − M)), LSE = x_t + loss_row and dH = (dH·L/R −
+// L·W[target]) / (e_t + L) / n_valid (R: the sum of P), with dH the sum in order of the `ks` accumulated K-slice
 // partials when the product was split; rows without a target get dH = 0 and no
 // loss.
 __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
@@ -283,7 +308,8 @@ __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
     a.lse[m] = xt + loss;
     a.loss_row[m] = loss;
   }
-  const float inv = 1.f / (et + L), ct = L * inv, sc = *a.inv_nvalid;
+  const float R = a.run_r[m], sc = *a.inv_nvalid;
+  const float ct = L / (et + L), inv = R > 0.f ? ct / R : ct;  // R = 0: P is all zeros
   const bf16* w = a.W + (long)t * a.D;
   const float* src = ks > 1 ? a.part + (long)m * a.D : dr;
   const long plane = (long)a.n * a.D;

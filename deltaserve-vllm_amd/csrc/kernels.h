@@ -169,6 +169,11 @@ hipError_t lora_dual(const DualArgs* a, int count, hipStream_t s);
 bool lora_dual_supported(int R1, int R2, int C);
 
 // ---- head.hip
+// Of a run of vocabulary columns of one row, the target column left out: the
+// softmax reference, Σ exp(logit − ref) and the same sum of bf16-rounded terms.
+struct CEStat {
+  float ref, sum, rsum;
+};
 struct HeadArgs {
   const bf16* normed; long ldh;   // [n, D]
   const bf16* W;                  // [V, D]
@@ -178,9 +183,7 @@ struct HeadArgs {
   int* labels;                    // [n] target id or -1 (head_init)
   int n; const int* n_dev;
   int D, V;
-  // [n_cap, ntn] per run of ce_bn columns (reference, sum exp), without the
-  // row's target column
-  float2* stats;
+  CEStat* stats;                  // [n_cap, ntn] per run of ce_bn columns
   int ntn;                        // ceil(V / ce_bn)
   int ce_bn, ce_cfg;              // run width and tile of the logits product (head_plan)
   int dh_cfg, dh_ks;              // tile and K slices of the dH product (head_plan)
@@ -188,6 +191,7 @@ struct HeadArgs {
   float* lse;                     // [n_cap] row LSE (natural log), after the last chunk
   float* run_m;                   // [n_cap] the row's softmax reference M
   float* run_l;                   // [n_cap] running Σ exp(logit − run_m), target left out
+  float* run_r;                   // [n_cap] the same sum of P as stored (bf16)
   float* alpha;                   // [n_cap] the dH accumulator's factor for the chunk
   float* loss_row;                // [n_cap]
   float* loss_out;                // scalar: sum(loss_row)/n_valid

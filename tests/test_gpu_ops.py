@@ -598,6 +598,29 @@ def test_head_confident_rows(vchunk, gain):
     assert err.max() < 2 ** -8
 
 
+@pytest.mark.parametrize("gain", [2.5, 3.3, 6.0])
+@pytest.mark.parametrize("vchunk", [0, 512])
+def test_head_dominating_column(vchunk, gain):
+    """Rows where one column other than the target has almost all the
+    probability, below and past the softmax reference's limit (25, 33 and 61
+    above the target): dH is W[column] − W[target] to fp32, whatever bf16 makes
+    of that column's exponential (up to 2^-9 of itself). Per row, 2-norm against
+    fp64: the other columns hold at most 5e-7 of the probability and the logits
+    are fp32 sums (error 1.2e-4 at most, times p(1 − p)), so 1e-5."""
+    from deltaserve_amd import ops
+    seq_lens, V = [200, 100], 2000
+    x, W, peak = _peaked_rows(sum(seq_lens), V, 4096, gain, seed=91)
+    ids = (torch.roll(peak, 1) + 1 + torch.arange(300) % (V - 1)) % V
+    assert not (ids == torch.roll(peak, 1)).any()
+    loss, nv, dH = ops.head_backward(x.to(DEV), W.to(DEV), ids.to(DEV), seq_lens, vocab_chunk=vchunk)
+    want, err = _row_errors(x, W, ids, seq_lens, dH)
+    print(f"[dominating column] loss {loss:.7f} ({want:.7f}), dH error max {err.max():.2e} "
+          f"mean {err.mean():.2e}", flush=True)
+    assert nv == 298
+    assert abs(loss - want) < 1e-5 * want
+    assert err.max() < 1e-5
+
+
 @pytest.mark.parametrize("release", [False, True])
 def test_scratch_is_private_to_a_call(release):
     """The ops' kept scratch memory: four threads on streams of their own run
