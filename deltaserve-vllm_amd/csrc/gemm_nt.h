@@ -9,20 +9,22 @@
 //
 // Main loop. BK = 64: each K tile is a 128-byte run of every operand row,
 // fetched by direct-to-LDS buffer loads (buffer_load_dwordx4 ... lds; 8 lanes
-// cover one row, so every request is a whole 128-byte line) into a ring of
-// LDS stages. Each wave owns a (BM/WM)×(BN/WN) sub-tile of
+// cover one row, so every request is a whole 128-byte line) into a ring of NA
+// LDS slots for A tiles and NB for B tiles. Each wave owns a (BM/WM)×(BN/WN) sub-tile of
 // v_mfma_f32_16x16x32_bf16 accumulators, tied to their AGPRs by inline-asm
 // MFMAs (with the builtin the compiler gave each MFMA's result registers
 // other than its accumulator's and moved every accumulator back at the end
 // of each iteration: 400 moves per K step). A K step is two 32-deep slices:
 // the first half of slice 0's MFMAs carries the fragment reads of slice 1
-// (one after each MFMA); then every wave's reads of stage kt have returned
-// and its loads of stage kt+1 have landed, so one barrier publishes stage
-// kt+1 and frees stage kt's slot; the rest of the step's MFMAs carry the
-// loads of stage kt+2 into that slot (one after every other MFMA) and, in
-// slice 1, the reads of slice 0 of stage kt+1. Loads get about one step of
-// latency budget. Past the end of K the loads zero-fill the slot without
-// touching memory, so the waits are constants.
+// (one after each MFMA); then every wave's reads of tile kt have returned and
+// its loads of tile kt+1 have landed (the wait leaves in flight the loads
+// issued after them), so one barrier publishes tile kt+1 and frees tile kt's
+// slots; the rest of the step's MFMAs carry the loads of A tile kt+NA and B
+// tile kt+NB into them (one after every third MFMA) and, in slice 1, the reads
+// of slice 0 of tile kt+1. Loads have NA − 1 (A) and NB − 1 (B) steps of
+// latency budget. A block's last steps, with nothing left to load, wait for
+// what is still in flight; a block of fewer K tiles than slots fills the rest
+// of them from the zero page.
 //
 // LDS layout per stage and operand: rows of 128 B (64 bf16) as eight 16-byte
 // chunks; chunk c of row r sits in slot c ^ f(r), f(r) = ((r>>1)&7) ^ ((r&1)<<2),
@@ -30,8 +32,10 @@
 // quarter-wave) conflict-free. The loads write LDS linearly (lane i of a load
 // lands at byte 16·i of its 1 KB segment = 8 rows), so the swizzle is applied
 // on the global side: the lane filling slot s of row r fetches chunk s ^ f(r).
-// Out-of-range rows (past M or N) and chunks past K are fetched from an offset
-// outside the buffer descriptor and land as zeros.
+// Chunks past K, and rows past M or N in an 8-row block that has some before,
+// are fetched from an offset outside the buffer descriptor and land as zeros; a
+// load with nothing of its own to fetch takes rows that exist or the zero page
+// (gemm_ring.h).
 //
 // Block ids are remapped so each XCD (round-robin dispatch over 8 XCDs) gets a
 // contiguous run of tiles, grouped 4 deep along M for L2 reuse.
@@ -42,6 +46,7 @@
 #include <type_traits>
 
 #include "dsb_common.h"
+#include "gemm_ring.h"
 
 namespace dsb {
 
@@ -122,9 +127,9 @@ DSB_DEV void mfma_drain() { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop
 // issue no other instruction that reads M0 (checked on their assembly), so
 // the save/restore around each load is not needed. In the main loop the M0
 // write (set_m0) goes before the MFMA that precedes its load (dma16_m0), which
-// covers the wait state between them; elsewhere lds_dma16_m0 does both.
-// (clang warns on every use that M0 is reserved; the warning is silenced for
-// these two helpers only.)
+// covers the wait state between them; elsewhere an s_nop does. (clang warns on
+// every use that M0 is reserved; the warning is silenced for these two helpers
+// only.)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 DSB_DEV void set_m0(unsigned lds_addr) {
@@ -132,15 +137,6 @@ DSB_DEV void set_m0(unsigned lds_addr) {
 }
 DSB_DEV void dma16_m0(u32x4 rsrc, int voff) {
   asm volatile("buffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(voff), "s"(rsrc) : "memory");
-}
-DSB_DEV void lds_dma16_m0(u32x4 rsrc, int voff, unsigned lds_addr) {
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "buffer_load_dwordx4 %0, %1, 0 offen lds"
-      :
-      : "v"(voff), "s"(rsrc), "s"(lds_addr)
-      : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
@@ -329,6 +325,20 @@ DSB_DEV int fkn(int k) {
   return ((2 * (k & 3)) ^ (((k >> 3) & 1) << 3)) & (CPR - 1);
 }
 
+// A fill of one A and one B slot of the ring. EDGE: either tile may lie past the
+// block's K range or be the last of a segment.
+template <bool EDGE>
+struct GemmFill {
+  static constexpr bool kEdge = EDGE;
+  u32x4 dA, dB;
+  int voA, voB;
+  int stA, lastA;    // bytes per 8·NW rows of A, of the wave's last row block
+  bool s1B;          // of the first K segment
+  int pastA, pastB;  // −1: past the block's range, the zero page; 0 (EDGE only)
+  int liveB;         // rows of a [K, N] B tile (EDGE only)
+  unsigned dstA, dstB;
+};
+
 template <int BM, int BN, int WM, int WN, class Epi, bool KN = false, int NA = 2, int NB = 3>
 __global__ __launch_bounds__(WM* WN * 64)
 __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel(GemmProblem p, Epi epi) {
@@ -410,16 +420,18 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     return make_rsrc((s1 ? p.B : p.B2) + n0 + (long)k0 * ld,
                      (int)(((long)(rows - 1) * ld + rowsB) * 2));
   };
-  // lane byte offset of its first row; A load j adds j·8·NW rows, B load j
-  // starts at row brow0(j) of the descriptor (uniform)
-  const int rw = 8 * wave + lrow;
+  // lane byte offset of its first row; A load j adds j·8·NW rows, up to the
+  // wave's last row block, B load j starts at row brow0(j) of the descriptor
+  // (uniform)
+  const int rw = ring_row_block(8 * wave, rowsA) + lrow;
   const int voA1 = (rw * (int)p.lda + lch * 8) * 2, voB1 = (lrow * (int)p.ldb + lch * 8) * 2;
   const int voA2 = (rw * (int)p.lda2 + lch * 8) * 2, voB2 = (lrow * (int)p.ldb2 + lch * 8) * 2;
   const int stA1 = 16 * NW * (int)p.lda;  // bytes per 8·NW rows
   const int stA2 = 16 * NW * (int)p.lda2;
+  const int jlast = ring_last_block(8 * wave, 8 * NW, rowsA);
   auto brow0 = [&](int jb) {
     const int r = 8 * (wave + jb * NW);  // LDS row of the block
-    if (!glu) return r;
+    if (!glu) return ring_row_block(r, rowsB);
     constexpr int HF = TN / 2;                // features per wave column
     const int wcol = r / TN, c = r % TN;      // wave column, column within it
     const int f = pn * (BN / 2) + wcol * HF + (c % HF);
@@ -450,74 +462,84 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   }
   const unsigned lds0 = lds_addr(smem);
 
-  // Loads of K tile kt into stage slot `slot`, issued one at a time by
-  // issue_one(j) so they can be spread over a run of MFMAs. Tiles past this
-  // block's range (kt >= kt1) get an empty descriptor: their loads fill the
-  // slot with zeros without touching memory, and loads complete in issue
-  // order all the same, so the waits' counts are constants.
-  // A fill of K tile ktA into A slot sa and of K tile ktB into B slot sb;
-  // dstB is biased by −SA elements, so B row offsets keep the SA of the
-  // fragment-read layout (brow, btr).
-  struct Fill {
-    u32x4 dA, dB;
-    int voA, voB, stA;
-    bool s1B;
-    unsigned dstA, dstB;
+  // Loads of K tile ktA into A slot sa and of K tile ktB into B slot sb, issued
+  // one at a time by issue_one(j) so they can be spread over a run of MFMAs.
+  // Tiles past this block's range (kt >= kt1) load from the zero page, so the
+  // waits' counts are constants and every load touches memory. dstB is biased
+  // by −SA elements, so B row offsets keep the SA of the fragment-read layout
+  // (brow, btr).
+  const u32x4 zs = zero_rsrc();
+  // a ? x : y by a scalar mask (−1 or 0): as selects on one uniform condition
+  // the compiler moves descriptors that a vector select shares it with out of
+  // the scalar registers
+  auto mask = [](bool c) { return __builtin_amdgcn_readfirstlane(c ? -1 : 0); };
+  auto pick = [](int a, int x, int y) { return (x & a) | (y & ~a); };
+  auto pick_rsrc = [&](int a, const u32x4& x, const u32x4& y) {
+    u32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = (unsigned)pick(a, (int)x[i], (int)y[i]);
+    return r;
   };
   auto a_slot = [&](int sa) { return lds0 + (unsigned)(sa * SA * 2) + (unsigned)(8 * wave * BK * 2); };
   auto b_slot = [&](int sb) {
     return lds0 + (unsigned)(((NA - 1) * SA + sb * SB) * 2) + (unsigned)(8 * wave * BK * 2);
   };
   auto make_fill = [&](int ktA, int sa, int ktB, int sb) {
-    Fill f;
+    GemmFill<true> f;
     {
       const bool s1 = ktA < nk1;
       const int k0 = s1 ? ktA * BK : (ktA - nk1) * BK;
       const int kb = (k0 * 2) | ((k0 + lch * 8 < (s1 ? p.K1 : K2)) ? 0 : OOB);
-      f.dA = s1 ? dA1 : dA2;
-      f.dA[2] = ktA < kt1 ? f.dA[2] : 0u;
-      f.voA = (s1 ? voA1 : voA2) + kb;
-      f.stA = s1 ? stA1 : stA2;
+      f.pastA = mask(ktA >= kt1);
+      f.dA = pick_rsrc(f.pastA, zs, s1 ? dA1 : dA2);
+      f.voA = pick(f.pastA, lane * 16, (s1 ? voA1 : voA2) + kb);
+      f.stA = pick(f.pastA, 0, s1 ? stA1 : stA2);
+      f.lastA = jlast * f.stA;
     }
     {
       const bool s1 = ktB < nk1;
       const int k0 = s1 ? ktB * BK : (ktB - nk1) * BK;
       const int kb = (k0 * 2) | ((k0 + lch * 8 < (s1 ? p.K1 : K2)) ? 0 : OOB);
-      if constexpr (KN)
-        f.dB = kn_rsrc(s1, k0);
-      else
-        f.dB = s1 ? dB1 : dB2;
-      f.dB[2] = ktB < kt1 ? f.dB[2] : 0u;
-      f.voB = (s1 ? voB1 : voB2) + kb;
+      f.pastB = mask(ktB >= kt1);
       f.s1B = s1;
+      if constexpr (KN) {
+        f.dB = kn_rsrc(s1, k0);
+        f.liveB = pick(f.pastB, 0, (s1 ? kbr1 : K2) - k0);
+      } else {
+        f.dB = pick_rsrc(f.pastB, zs, s1 ? dB1 : dB2);
+        f.voB = pick(f.pastB, lane * 16, (s1 ? voB1 : voB2) + kb);
+      }
     }
     f.dstA = a_slot(sa);
     f.dstB = b_slot(sb);
     return f;
   };
-  auto issue_one = [&](const Fill& f, int j) {
-    if (j < IA) {
-      lds_dma16_m0(f.dA, f.voA + j * f.stA, f.dstA + j * 8 * NW * BK * 2);
-    } else if constexpr (KN) {
-      set_m0(f.dstB + (SA + (j - IA) * 8 * NW * BK) * 2);
-      asm volatile("s_nop 0" ::: "memory");
-      dma16_m0(f.dB, f.s1B ? vkn1[j - IA] : vkn2[j - IA]);
-    } else {
-      lds_dma16_m0(f.dB, f.voB + (f.s1B ? boff1[j - IA] : boff2[j - IA]),
-                   f.dstB + (SA + (j - IA) * 8 * NW * BK) * 2);
-    }
-  };
-  // the same load split around an MFMA: M0 before it, the load after it
-  auto pre_one = [&](const Fill& f, int j) {
+  // load j of fill f: M0 (its LDS address), and the load itself, which in a run
+  // of MFMAs go before and after one of them
+  auto pre_one = [&](const auto& f, int j) __attribute__((always_inline)) {
     set_m0(j < IA ? f.dstA + j * 8 * NW * BK * 2 : f.dstB + (SA + (j - IA) * 8 * NW * BK) * 2);
   };
-  auto go_one = [&](const Fill& f, int j) {
-    if (j < IA)
-      dma16_m0(f.dA, f.voA + j * f.stA);
-    else if constexpr (KN)
-      dma16_m0(f.dB, f.s1B ? vkn1[j - IA] : vkn2[j - IA]);
-    else
-      dma16_m0(f.dB, f.voB + (f.s1B ? boff1[j - IA] : boff2[j - IA]));
+  auto go_one = [&](const auto& f, int j) __attribute__((always_inline)) {
+    constexpr bool EDGE = std::decay_t<decltype(f)>::kEdge;
+    if (j < IA) {
+      dma16_m0(f.dA, j == 0 ? f.voA : f.voA + min(j * f.stA, f.lastA));
+    } else if constexpr (KN) {
+      const int off = f.s1B ? vkn1[j - IA] : vkn2[j - IA];
+      if constexpr (EDGE) {
+        const int none = mask(!ring_kn_live(RPL * (wave + (j - IA) * NW), f.liveB));
+        dma16_m0(pick_rsrc(none, zs, f.dB), pick(none, lane * 16, off));
+      } else {
+        dma16_m0(f.dB, off);
+      }
+    } else {
+      const int off = f.s1B ? boff1[j - IA] : boff2[j - IA];
+      dma16_m0(f.dB, f.voB + (EDGE ? pick(f.pastB, 0, off) : off));
+    }
+  };
+  auto issue_one = [&](const auto& f, int j) __attribute__((always_inline)) {
+    pre_one(f, j);
+    asm volatile("s_nop 0" ::: "memory");
+    go_one(f, j);
   };
 
   f32x4 acc[FM][FN];
@@ -586,7 +608,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   // of other instructions between MFMAs would leave the matrix pipe idle
   // (loads after every MFMA, or every other one, measured slower).
   auto mma = [&](int buf, int t0, int t1, const bf16* nba, const bf16* nbb, int ns, int nbuf,
-                 int nr, const Fill& f, int j0, int nj) {
+                 int nr, const auto& f, int j0, int nj) __attribute__((always_inline)) {
     int r = 0, j = 0;
 #pragma unroll
     for (int t = t0; t < t1; ++t) {
@@ -615,10 +637,10 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     for (int jj = 0; jj < IAB; ++jj)
       if (jj >= j && jj < nj) issue_one(f, j0 + jj);
   };
-  // Loads of K tiles ktA, ktB (both < nk1, first segment): the descriptors
-  // and row offsets are the loop-invariant ones of segment 1.
+  // Loads of K tiles ktA, ktB (both of the first segment, whole): the
+  // descriptors and row offsets are the loop-invariant ones of segment 1.
   auto make_fill1 = [&](int ktA, int sa, int ktB, int sb) {
-    Fill f;
+    GemmFill<false> f;
     const int k0a = ktA * BK, k0b = ktB * BK;
     f.dA = dA1;
     if constexpr (KN)
@@ -628,6 +650,7 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     f.voA = voA1 + ((k0a * 2) | ((k0a + lch * 8 < p.K1) ? 0 : OOB));
     f.voB = voB1 + ((k0b * 2) | ((k0b + lch * 8 < p.K1) ? 0 : OOB));
     f.stA = stA1;
+    f.lastA = jlast * stA1;
     f.s1B = true;
     f.dstA = a_slot(sa);
     f.dstB = b_slot(sb);
@@ -637,19 +660,24 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   // Prologue: every slot's tile requested at once (one latency, not one for
   // the first tile and another for the next), then the first tile awaited and
   // published and slice 0 of it read.
-  {
-    const Fill f = make_fill(kt0, 0, kt0, 0);
+  const int whole = ring_whole_tiles(KN, nk1, kbr1);
+  auto prologue = [&](auto&& mk) __attribute__((always_inline)) {
     if constexpr (NB > NA) {
+      const auto f = mk(kt0, 0, kt0, 0);
 #pragma unroll
       for (int j = IA; j < IAB; ++j) issue_one(f, j);
     }
 #pragma unroll
     for (int t = 0; t < NA; ++t) {
-      const Fill g = make_fill(kt0 + t, t, kt0 + t + NB - NA, t + NB - NA);
+      const auto g = mk(kt0 + t, t, kt0 + t + NB - NA, t + NB - NA);
 #pragma unroll
       for (int j = 0; j < IAB; ++j) issue_one(g, j);
     }
-  }
+  };
+  if (kt0 + NB <= min(kt1, whole))
+    prologue(make_fill1);
+  else
+    prologue(make_fill);
   wait_vm<WPRO>();
   lds_barrier();
 #pragma unroll
@@ -659,33 +687,51 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   // (fragments of slice 0 already in buffer 0). Its mid-step wait leaves in
   // flight the loads issued after those of tile kt+1. After that barrier tile
   // kt's slots are free, and it issues A of tile kt+NA and then B of tile
-  // kt+NB into them.
+  // kt+NB into them (mk: their fill; loads 0 .. `loads` − 1 of it: IA for A
+  // alone, 0 where nothing is left to load).
   int ca = 0, cb = 0;
-  auto step = [&](int kt, auto&& mk) {
+  auto step = [&](int kt, auto&& mk, auto loads, auto&& wait) __attribute__((always_inline)) {
+    constexpr int NL = decltype(loads)::value, NL1 = NL < H1 ? NL : H1;
     const bf16* ba = a_base(ca);
     const bf16* bb = b_base(cb);
-    const Fill next = mk(kt + NA, ca, kt + NB, cb);
+    const auto next = mk(kt + NA, ca, kt + NB, cb);
     ca = ca + 1 == NA ? 0 : ca + 1;
     cb = cb + 1 == NB ? 0 : cb + 1;
     __builtin_amdgcn_sched_barrier(0);
     mma(0, 0, NM / 2, ba, bb, 1, 1, NR, next, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
     wait_lgkm0();
-    wait_vm<WSTEP>();
+    wait();
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    mma(0, NM / 2, NM, ba, bb, 1, 1, 0, next, 0, H1);
+    mma(0, NM / 2, NM, ba, bb, 1, 1, 0, next, 0, NL1);
     __builtin_amdgcn_sched_barrier(0);
-    mma(1, 0, NM, a_base(ca), b_base(cb), 0, 0, NR, next, H1, IAB - H1);
+    mma(1, 0, NM, a_base(ca), b_base(cb), 0, 0, NR, next, NL1, NL - NL1);
     __builtin_amdgcn_sched_barrier(0);
   };
   // Steps whose prefetches (A tile kt+NA, B tile kt+NB) stay in segment 1 use
-  // the invariant segment-1 fill; the last few steps select the segment per
-  // tile, and load nothing past this block's range.
-  const int nfast = max(kt0, min(kt1, nk1) - NB);
+  // the invariant segment-1 fill; the next ones, up to the block's last tiles,
+  // select the segment, and what there is to load of it, per tile; the last NA
+  // load nothing and wait for less and less. (With loads of the zero page in
+  // them instead, which keep the waits' counts constant, the epilogue waits for
+  // those loads: the 8192-token 4096-wide cycle took 1 % longer.)
+  constexpr std::integral_constant<int, IAB> both{};
+  constexpr std::integral_constant<int, IA> a_only{};
+  constexpr std::integral_constant<int, 0> none{};
+  const auto full = [] { wait_vm<WSTEP>(); };
+  const int nfast = ring_fast_end(kt0, kt1, whole, NB);
   int kt = kt0;
-  for (; kt < nfast; ++kt) step(kt, make_fill1);
-  for (; kt < kt1; ++kt) step(kt, make_fill);
+  for (; kt < nfast; ++kt) step(kt, make_fill1, both, full);
+  for (; kt < kt1 - NB; ++kt) step(kt, make_fill, both, full);
+  if (NB > NA && kt < kt1 - NA) step(kt++, make_fill, a_only, full);
+  for (; kt < kt1; ++kt)
+    step(kt, [](int, int, int, int) { return GemmFill<false>{}; }, none, [&] {
+      const int left = kt1 - kt;  // tiles that may be in flight: those from kt + 2 on
+      if (left >= NB) wait_vm<WSTEP>();
+      else if (NA > 4 && left == 4) wait_vm<2 * IAB>();
+      else if (NA > 3 && left == 3) wait_vm<IAB>();
+      else wait_vm<0>();
+    });
   mfma_drain();
   // the last step's loads land before the epilogue reuses the LDS
   wait_vm<0>();
