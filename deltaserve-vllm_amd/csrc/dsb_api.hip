@@ -320,7 +320,7 @@ template <class T>
 int dalloc(dsb_handle* h, T** p, size_t count) {
   void* v = nullptr;
   const size_t bytes = count * sizeof(T) + 256;
-  hipError_t e = hipMalloc(&v, bytes);
+  hipError_t e = device_malloc(&v, bytes);
   if (e != hipSuccess) {
     set_error("hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     h->err = get_error();
@@ -1484,9 +1484,9 @@ int rebuild_publish(dsb_handle* h) {
   h->npub_chunks = 0;
   h->pub_elems = elems;
   if (!jobs.empty()) {
-    CK(hipMalloc(&h->d_pub_jobs, jobs.size() * sizeof(CastJob)));
+    CK(device_malloc((void**)&h->d_pub_jobs, jobs.size() * sizeof(CastJob)));
     CK(hipMemcpy(h->d_pub_jobs, jobs.data(), jobs.size() * sizeof(CastJob), hipMemcpyHostToDevice));
-    CK(hipMalloc(&h->d_pub_chunks, chunks.size() * sizeof(int2)));
+    CK(device_malloc((void**)&h->d_pub_chunks, chunks.size() * sizeof(int2)));
     CK(hipMemcpy(h->d_pub_chunks, chunks.data(), chunks.size() * sizeof(int2),
                  hipMemcpyHostToDevice));
     h->npub_chunks = (int)chunks.size();

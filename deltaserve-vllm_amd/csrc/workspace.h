@@ -10,7 +10,8 @@
 // and no kernel of an earlier call can still use it. The pool is bounded
 // (kPoolBytes per device for what it keeps; a larger block is freed at the end
 // of its call, the longest unused ones make room), emptied when an allocation
-// fails, and released on request (dsb_release_workspaces).
+// of this library on its device fails, and released on request
+// (dsb_release_workspaces).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -66,27 +67,42 @@ class BlockPool {
       release(b);
       return;
     }
-    trim(limit_ - b.bytes);
-    std::lock_guard<std::mutex> lk(mu_);
-    kept_.push_back(b);
-    held_ += b.bytes;
+    std::vector<Block> out;
+    {
+      // kept and the oldest evicted under one lock, so that calls returning
+      // blocks together stay within the limit
+      std::lock_guard<std::mutex> lk(mu_);
+      kept_.push_back(b);
+      held_ += b.bytes;
+      evict(limit_, out);
+    }
+    for (const Block& v : out) release(v);
   }
   // Frees kept blocks, the longest kept first, down to `bytes`.
   void trim(size_t bytes) {
     std::vector<Block> out;
     {
       std::lock_guard<std::mutex> lk(mu_);
-      while (held_ > bytes && !kept_.empty()) {
-        out.push_back(kept_.front());
-        held_ -= kept_.front().bytes;
-        kept_.pop_front();
-      }
+      evict(bytes, out);
     }
     for (const Block& b : out) release(b);
+  }
+  // Bytes kept.
+  size_t held() {
+    std::lock_guard<std::mutex> lk(mu_);
+    return held_;
   }
   void release(const Block& b) { (void)(pinned_ ? hipHostFree(b.p) : hipFree(b.p)); }
 
  private:
+  // under mu_: takes the longest kept blocks out until at most `bytes` stay
+  void evict(size_t bytes, std::vector<Block>& out) {
+    while (held_ > bytes && !kept_.empty()) {
+      out.push_back(kept_.front());
+      held_ -= kept_.front().bytes;
+      kept_.pop_front();
+    }
+  }
   static size_t round_up(size_t bytes) {
     size_t r = 4096;
     while (r < bytes && r < (1u << 20)) r *= 2;
@@ -115,6 +131,17 @@ inline BlockPool& device_pool(int dev) {
 inline BlockPool& pinned_pool() {
   static BlockPool* p = new BlockPool(true, kPinnedBytes);
   return *p;
+}
+
+// hipMalloc on the current device for memory that is not the pool's; what the
+// pool keeps there makes room if it fails.
+inline hipError_t device_malloc(void** p, size_t bytes) {
+  const hipError_t e = hipMalloc(p, bytes);
+  int dev = 0;
+  if (e == hipSuccess || hipGetDevice(&dev) != hipSuccess || dev >= kPoolDevices) return e;
+  (void)hipGetLastError();
+  device_pool(dev).trim(0);
+  return hipMalloc(p, bytes);
 }
 
 // One call's scratch memory on stream s.
