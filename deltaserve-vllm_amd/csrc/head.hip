@@ -24,7 +24,7 @@
 //     e^(M − M') and P scaled in place to M';
 //   dH = dH·α + P·W_c (GEMM, fp32 accumulate with the per-row α);
 //   after the last chunk, with e_t = exp(x_t − M): loss_row = ln(1 + L/e_t),
-//   dH = (dH·L/R − L·W[target]) / (e_t + L) / n_valid, LSE = M + ln(e_t + L),
+//   dH = (dH − R·W[target]) · L/R / (e_t + L) / n_valid, LSE = M + ln(e_t + L),
 //   and a single-block deterministic sum gives the cycle loss.
 // L/R takes the common part of P's rounding out of dH: one column that
 // dominates the others' sum is rounded by up to 2^-9 (its exponential is 1 only
@@ -283,8 +283,8 @@ __global__ __launch_bounds__(256) void ce_rescale_kernel(HeadArgs a, int c0) {
 
 // After the last chunk, one wave per live row: with e_t = exp(x_t − M) and the
 // other columns' sum L, loss_row = ln(1 + L/e_t) (where x_t lies far below M as
-// ln(e_t + L) − (x_t − M)), LSE = x_t + loss_row and dH = (dH·L/R −
-// L·W[target]) / (e_t + L) / n_valid (R: the sum of P), with dH the sum in order of the `ks` accumulated K-slice
+// ln(e_t + L) − (x_t − M)), LSE = x_t + loss_row and dH = (dH −
+// R·W[target]) · L/R / (e_t + L) / n_valid (R: the sum of P), with dH the sum in order of the `ks` accumulated K-slice
 // partials when the product was split; rows without a target get dH = 0 and no
 // loss.
 __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
@@ -308,8 +308,8 @@ __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
     a.lse[m] = xt + loss;
     a.loss_row[m] = loss;
   }
-  const float R = a.run_r[m], sc = *a.inv_nvalid;
-  const float ct = L / (et + L), inv = R > 0.f ? ct / R : ct;  // R = 0: P is all zeros
+  // R = 0: P is all zeros
+  const float R = a.run_r[m], f = R == 0.f ? 0.f : L / (et + L) / R * *a.inv_nvalid;
   const bf16* w = a.W + (long)t * a.D;
   const float* src = ks > 1 ? a.part + (long)m * a.D : dr;
   const long plane = (long)a.n * a.D;
@@ -324,10 +324,10 @@ __global__ __launch_bounds__(256) void ce_finalize_kernel(HeadArgs a, int ks) {
       x1 += *reinterpret_cast<const f32x4*>(src + z * plane + 8 * k + 4);
     }
     f32x4* d = reinterpret_cast<f32x4*>(dr + 8 * k);
-    d[0] = f32x4{(x0[0] * inv - wf[0] * ct) * sc, (x0[1] * inv - wf[1] * ct) * sc,
-                 (x0[2] * inv - wf[2] * ct) * sc, (x0[3] * inv - wf[3] * ct) * sc};
-    d[1] = f32x4{(x1[0] * inv - wf[4] * ct) * sc, (x1[1] * inv - wf[5] * ct) * sc,
-                 (x1[2] * inv - wf[6] * ct) * sc, (x1[3] * inv - wf[7] * ct) * sc};
+    d[0] = f32x4{(x0[0] - wf[0] * R) * f, (x0[1] - wf[1] * R) * f,
+                 (x0[2] - wf[2] * R) * f, (x0[3] - wf[3] * R) * f};
+    d[1] = f32x4{(x1[0] - wf[4] * R) * f, (x1[1] - wf[5] * R) * f,
+                 (x1[2] - wf[6] * R) * f, (x1[3] - wf[7] * R) * f};
   }
 }
 
