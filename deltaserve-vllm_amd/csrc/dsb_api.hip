@@ -2116,6 +2116,39 @@ int dsb_op_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, const vo
   return 0;
 }
 
+int dsb_op_gemm_split(const void* A, int64_t lda, const void* B, int64_t ldb, const void* A2,
+                      int64_t lda2, const void* B2, int64_t ldb2, int M, int N, int K1, int K2,
+                      void* C, int64_t ldc, int out_f32, int accumulate, const void* R, int64_t ldr,
+                      int b_kn, int tile, int slices, void* stream) {
+  if (K1 % 8 || K2 % 8 || lda % 8 || ldb % 8 || (K2 && (lda2 % 8 || ldb2 % 8)) || ldc % 4 || N % 8)
+    return fail(nullptr, "dsb_op_gemm_split: N, K and leading dims must be multiples of 8 (ldc of 4)");
+  if (tile < 0 || tile >= kGemmCfgs || slices < 2 || slices > 16 || M < 0 || N < 0)
+    return fail(nullptr, "dsb_op_gemm_split: tile in [0, 4], slices in [2, 16]");
+  hipStream_t s = (hipStream_t)stream;
+  GemmProblem p{(const bf16*)A, lda, (const bf16*)B, ldb, (const bf16*)A2, lda2,
+                (const bf16*)B2, ldb2, M, N, K1, K2, nullptr};
+  p.b_kn = b_kn ? 1 : 0;
+  const GemmPlan pl{tile, slices};
+  Scratch tmp(s);
+  p.part = tmp.dev<float>(gemm_part_elems(M, N, slices));
+  if (!p.part) return fail(nullptr, "dsb_op_gemm_split: hipMalloc failed");
+  if (out_f32)
+    OPCK(launch_gemm_split(p, EpiF32{(float*)C, ldc, N, accumulate}, pl, s));
+  else
+    OPCK(launch_gemm_split(p, EpiBF16{(bf16*)C, ldc, N, (const bf16*)R, ldr}, pl, s));
+  OPCK(tmp.finish());
+  return 0;
+}
+
+int dsb_gemm_plan(int M, int N, int K, double out_bytes, int* tile, int* slices) {
+  if (M <= 0 || N <= 0 || K <= 0 || !tile || !slices)
+    return fail(nullptr, "dsb_gemm_plan: bad arguments");
+  const GemmPlan pl = gemm_plan(M, N, K, out_bytes, true);
+  *tile = pl.cfg;
+  *slices = pl.ks;
+  return 0;
+}
+
 int dsb_op_gemm_glu(const void* A, int64_t lda, const void* B, int64_t ldb, const void* A2,
                     int64_t lda2, const void* B2, int64_t ldb2, int M, int I, int K1, int K2,
                     void* GU, int64_t ldgu, void* H, int64_t ldh, void* stream) {

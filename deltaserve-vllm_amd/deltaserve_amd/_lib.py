@@ -114,6 +114,11 @@ _SIGS = {
                             c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p,
                             c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_int,
                             c_void_p]),
+    "dsb_gemm_plan": (c_int, [c_int, c_int, c_int, c_double, POINTER(c_int), POINTER(c_int)]),
+    "dsb_op_gemm_split": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
+                                  c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p,
+                                  c_int64, c_int, c_int, c_void_p, c_int64, c_int, c_int,
+                                  c_int, c_void_p]),
     "dsb_op_gemm_glu": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_int64,
                                 c_void_p, c_int64, c_int, c_int, c_int, c_int, c_void_p, c_int64,
                                 c_void_p, c_int64, c_void_p]),

@@ -77,11 +77,21 @@ def rope_inv_freq(head_dim, theta, rope_scaling=None):
 
 # ---------------------------------------------------------------- dense products
 
+def gemm_plan(M, N, K, out_bytes):
+    """(tile, K slices) that a product takes by the cost model; ``out_bytes``
+    read and written per output element."""
+    tile, slices = c_int(), c_int()
+    L.check(L.load().dsb_gemm_plan(M, N, K, float(out_bytes), byref(tile), byref(slices)),
+            what="dsb_gemm_plan")
+    return tile.value, slices.value
+
+
 def gemm_nt(A, B, A2=None, B2=None, out_dtype=BF16, R=None, out=None, accumulate=False, cfg=-1,
-            b_kn=False):
+            b_kn=False, slices=0):
     """C = A·Bᵀ (+ A2·B2ᵀ) (+ R) — the projection products of ops.py:103-146.
     b_kn: B [K1, N] and B2 [K2, N] (C = A·B + A2·B2, the backward's dY·W with W
-    in its own layout)."""
+    in its own layout). ``slices`` 2 to 16: tile ``cfg`` (0 to 4) in that many K
+    slices instead of the cost model's choice."""
     _dev(A, B, A2, B2, R)
     M, K1 = A.shape
     N = B.shape[1] if b_kn else B.shape[0]
@@ -89,12 +99,14 @@ def gemm_nt(A, B, A2=None, B2=None, out_dtype=BF16, R=None, out=None, accumulate
     f32 = out_dtype == torch.float32
     if out is None:
         out = torch.empty(M, N, dtype=out_dtype, device=A.device)
-    L.check(L.load().dsb_op_gemm(_p(A), _ld(A), _p(B), _ld(B), _p(A2), 0 if A2 is None else _ld(A2),
-                                 _p(B2), 0 if B2 is None else _ld(B2), M, N, K1, K2, _p(out),
-                                 _ld(out), int(f32), int(accumulate), _p(R),
-                                 0 if R is None else _ld(R), int(bool(b_kn)), int(cfg),
-                                 _stream()),
-            what="dsb_op_gemm")
+    args = (_p(A), _ld(A), _p(B), _ld(B), _p(A2), 0 if A2 is None else _ld(A2),
+            _p(B2), 0 if B2 is None else _ld(B2), M, N, K1, K2, _p(out),
+            _ld(out), int(f32), int(accumulate), _p(R),
+            0 if R is None else _ld(R), int(bool(b_kn)), int(cfg))
+    if slices:
+        L.check(L.load().dsb_op_gemm_split(*args, int(slices), _stream()), what="dsb_op_gemm_split")
+    else:
+        L.check(L.load().dsb_op_gemm(*args, _stream()), what="dsb_op_gemm")
     return out
 
 

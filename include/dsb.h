@@ -277,6 +277,15 @@ int dsb_op_gemm(const void* A, int64_t lda, const void* B, int64_t ldb, const vo
                 int64_t lda2, const void* B2, int64_t ldb2, int M, int N, int K1, int K2,
                 void* C, int64_t ldc, int out_f32, int accumulate, const void* R, int64_t ldr,
                 int b_kn, int cfg, void* stream);
+/* dsb_gemm_plan (host only): the tile (cfg 0 to 4) and the number of K slices
+ * that a product M × N × K with `out_bytes` read and written per output element
+ * takes where it may split. dsb_op_gemm_split: dsb_op_gemm with the tile (0 to
+ * 4) and 2 to 16 K slices of it given; N a multiple of 8. */
+int dsb_gemm_plan(int M, int N, int K, double out_bytes, int* tile, int* slices);
+int dsb_op_gemm_split(const void* A, int64_t lda, const void* B, int64_t ldb, const void* A2,
+                      int64_t lda2, const void* B2, int64_t ldb2, int M, int N, int K1, int K2,
+                      void* C, int64_t ldc, int out_f32, int accumulate, const void* R, int64_t ldr,
+                      int b_kn, int tile, int slices, void* stream);
 /* Gate‖up product with the SwiGLU forward in its epilogue (the recompute of
  * ffn.py:25-26, frozen gate_up_proj plus its LoRA term; silu as ffn.py:40-41): GU[m, :] = bf16(A·Bᵀ + A2·B2ᵀ)
  * with B [2I, K1] = gate rows then up rows (GU = [gate | up], ld ldgu), and,

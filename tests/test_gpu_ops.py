@@ -51,9 +51,10 @@ def _b_operand(B, kn):
                                       (1, 8, 8, 8), (513, 264, 1024, 16), (200, 1024, 4096, 64),
                                       (1, 8, 512, 8)])
 def test_gemm_nt(cfg, M, N, K, K2, kn):
-    """cfg -2 splits K (the last three shapes: 4, 8 and 2 K slices, the
-    slices crossing into the second K segment) and sums the fp32 partials.
-    kn: B and B2 stored [K, N] (N a multiple of 8 there)."""
+    """The 256-, 128- and 64-wide tiles, and the tile and K split of the cost
+    model (cfg -2; of these shapes only 200 × 1024 splits: test_gemm_split has
+    every tile in slices). kn: B and B2 stored [K, N] (N a multiple of 8
+    there)."""
     from deltaserve_amd import ops
     if kn and N % 8:
         pytest.skip("a [K, N] B needs N a multiple of 8 (test_gemm_kn_refuses_ragged_n)")
@@ -82,8 +83,8 @@ def test_gemm_nt(cfg, M, N, K, K2, kn):
 def test_gemm_kn_equals_nt(M, N, K, K2):
     """The [K, N] operand path gives the [N, K] path's product bit for bit:
     the same MFMA fragments in the same order, only the B staging differs
-    (cycle-sized shapes: 256-wide tiles with ragged M and K, a LoRA segment,
-    N not a multiple of the tile)."""
+    (cycle-sized shapes at the cost model's tiles, 256 × 256 and 256 × 128:
+    ragged M and K, a LoRA segment, N not a multiple of the tile)."""
     from deltaserve_amd import ops
     A = _bf(_rnd(M, K, seed=21)).to(DEV)
     B = _bf(_rnd(N, K, seed=22))
@@ -494,6 +495,52 @@ def test_gemm_tiles(cfg, M, N, K, K2, kn):
     got = ops.gemm_nt(A.to(DEV), _b_operand(B, kn), None if A2 is None else A2.to(DEV),
                       _b_operand(B2, kn), out_dtype=torch.float32, cfg=cfg, b_kn=kn)
     assert max_rel(got, ref) < 1e-5
+
+
+@pytest.mark.parametrize("kn", [False, True])
+@pytest.mark.parametrize("tile", [0, 1, 2, 3, 4])
+@pytest.mark.parametrize("M,N,K,K2,slices", [(257, 136, 328, 48, 2), (257, 136, 328, 48, 5),
+                                             (1, 8, 512, 8, 3), (130, 1032, 1024, 24, 16),
+                                             (200, 264, 4096, 64, 7), (513, 520, 192, 0, 3)])
+def test_gemm_split(tile, M, N, K, K2, slices, kn):
+    """Every tile with K in slices: slices of different lengths (7 K tiles as
+    4 + 3; 9 as 3 + 3 + 3; 65 as 6 × 10 + 5), empty last ones (7 K tiles in 5
+    slices: 2, 2, 2, 1, 0; 17 in 16: nine used), one-tile slices, shorter than
+    the load ring, slices that cross into the second K segment, rows and
+    columns past a tile. fp32 (bound as in test_gemm_tiles), bf16 with a
+    residual, and accumulated fp32 outputs."""
+    from deltaserve_amd import ops
+    A, B = _bf(_rnd(M, K, seed=65)), _bf(_rnd(N, K, seed=66))
+    A2 = _bf(_rnd(M, K2, seed=67)) if K2 else None
+    B2 = _bf(_rnd(N, K2, seed=68)) if K2 else None
+    ref = A.float() @ B.float().t()
+    if K2:
+        ref += A2.float() @ B2.float().t()
+    dA, dB = A.to(DEV), _b_operand(B, kn)
+    dA2, dB2 = None if A2 is None else A2.to(DEV), _b_operand(B2, kn)
+    kw = dict(cfg=tile, slices=slices, b_kn=kn)
+    c32 = ops.gemm_nt(dA, dB, dA2, dB2, out_dtype=torch.float32, **kw)
+    assert max_rel(c32, ref) < 1e-5
+    R = _bf(_rnd(M, N, seed=69))
+    c16 = ops.gemm_nt(dA, dB, dA2, dB2, R=R.to(DEV), **kw)
+    assert max_rel(c16, ref + R.float()) < 8e-3
+    # the same fp32 sums, the residual added and rounded to bf16 once
+    assert torch.equal(c16, (c32 + R.to(DEV).float()).to(torch.bfloat16))
+    acc = c32.clone()
+    ops.gemm_nt(dA, dB, dA2, dB2, out_dtype=torch.float32, out=acc, accumulate=True, **kw)
+    assert torch.equal(acc, c32 + c32)
+
+
+def test_gemm_split_refuses():
+    from deltaserve_amd import _lib as L
+    from deltaserve_amd import ops
+    A = torch.zeros(16, 64, dtype=torch.bfloat16, device=DEV)
+    B = torch.zeros(32, 64, dtype=torch.bfloat16, device=DEV)
+    for rows, kw in ((28, dict(cfg=0, slices=2)), (32, dict(cfg=5, slices=2)),
+                     (32, dict(cfg=-1, slices=2)), (32, dict(cfg=0, slices=1)),
+                     (32, dict(cfg=0, slices=17))):
+        with pytest.raises(L.DsbError, match="dsb_op_gemm_split"):
+            ops.gemm_nt(A, B[:rows], **kw)
 
 
 @pytest.mark.parametrize("M,I,K,K2", [(96, 192, 256, 16), (130, 3072, 1024, 32), (256, 14336, 256, 16),
