@@ -2186,6 +2186,19 @@ int dsb_op_rmsnorm_bwd(const void* x, int64_t ldx, const void* g, int g_f32, int
   return 0;
 }
 
+int dsb_op_rmsnorm_bwd_parts(const void* x, int64_t ldx, const float* g, int64_t ldg, int parts,
+                             int64_t plane, const void* w, const void* resid, int64_t ldr, void* out,
+                             int64_t ldo, int rows, int D, float eps, void* stream) {
+  if (D % 8 || D > 8192 || ldg % 4 || plane % 4 || parts < 1)
+    return fail(nullptr, "dsb_op_rmsnorm_bwd_parts: D must be a multiple of 8, <= 8192, the "
+                         "gradient's strides of 4");
+  hipStream_t s = (hipStream_t)stream;
+  OPCK(rmsnorm_bwd((const bf16*)x, ldx, g, true, ldg, (const bf16*)w, (const bf16*)resid, ldr,
+                   (bf16*)out, ldo, rows, nullptr, D, eps, s, nullptr, nullptr, parts, plane));
+  OPCK(hipStreamSynchronize(s));
+  return 0;
+}
+
 int dsb_op_rope_table(const int32_t* pos, int n, const float* inv_freq, int half, float* cos_out,
                       float* sin_out, void* stream) {
   hipStream_t s = (hipStream_t)stream;

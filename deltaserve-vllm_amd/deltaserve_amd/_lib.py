@@ -127,6 +127,9 @@ _SIGS = {
     "dsb_op_rmsnorm_bwd": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int64, c_void_p,
                                    c_void_p, c_int64, c_void_p, c_int64, c_int, c_int,
                                    c_float, c_void_p]),
+    "dsb_op_rmsnorm_bwd_parts": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int64,
+                                         c_void_p, c_void_p, c_int64, c_void_p, c_int64, c_int,
+                                         c_int, c_float, c_void_p]),
     "dsb_op_rope_table": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_void_p,
                                   c_void_p]),
     "dsb_op_rope": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_void_p, c_void_p, c_int,

@@ -140,9 +140,17 @@ def rmsnorm(x, w, eps):
 
 
 def rmsnorm_backward(x, g, w, eps, resid=None):
-    """ops.py:91-100 (+ bf16 residual add, llama3.py:205); bf16 out."""
+    """ops.py:91-100 (+ bf16 residual add, llama3.py:205); bf16 out. An fp32 g
+    [parts, n, D] is added up in order first."""
     _dev(x, g, w, resid)
     out = torch.empty(x.shape, dtype=BF16, device=x.device)
+    if g.dim() == 3:
+        assert g.dtype == torch.float32 and g.stride(2) == 1
+        L.check(L.load().dsb_op_rmsnorm_bwd_parts(
+            _p(x), _ld(x), _p(g), g.stride(1), g.shape[0], g.stride(0), _p(w), _p(resid),
+            0 if resid is None else _ld(resid), _p(out), _ld(out), x.shape[0], x.shape[1],
+            float(eps), _stream()), what="dsb_op_rmsnorm_bwd_parts")
+        return out
     L.check(L.load().dsb_op_rmsnorm_bwd(_p(x), _ld(x), _p(g), int(g.dtype == torch.float32),
                                         _ld(g), _p(w), _p(resid), 0 if resid is None else _ld(resid),
                                         _p(out), _ld(out), x.shape[0], x.shape[1], float(eps),

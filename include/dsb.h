@@ -301,6 +301,11 @@ int dsb_op_rmsnorm(const void* x, int64_t ldx, const void* w, void* y, int64_t l
 int dsb_op_rmsnorm_bwd(const void* x, int64_t ldx, const void* g, int g_f32, int64_t ldg,
                        const void* w, const void* resid, int64_t ldr, void* out, int64_t ldo,
                        int rows, int D, float eps, void* stream);
+/* The same with the gradient as `parts` fp32 planes, `plane` elements apart,
+ * added in order (the K slices of the product that made it). */
+int dsb_op_rmsnorm_bwd_parts(const void* x, int64_t ldx, const float* g, int64_t ldg, int parts,
+                             int64_t plane, const void* w, const void* resid, int64_t ldr, void* out,
+                             int64_t ldo, int rows, int D, float eps, void* stream);
 /* ops.py:60-65 cos/sin table [n, head_dim/2] fp32 from int32 positions. */
 int dsb_op_rope_table(const int32_t* pos, int n, const float* inv_freq, int half, float* cos_out,
                       float* sin_out, void* stream);

@@ -192,6 +192,24 @@ def test_rmsnorm_fwd_bwd():
     assert max_rel(dxb, O.rmsnorm_backward(x.float(), _bf(g32).float(), w.float(), eps)) < 8e-3
 
 
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 7, 8, 16])
+@pytest.mark.parametrize("rows,D", [(77, 1024), (1, 8), (5, 2056), (3, 8192)])
+def test_rmsnorm_bwd_parts(rows, D, parts):
+    """The gradient as the K slices of the product before: the planes added in
+    order, four loads in flight, whole groups of four and every remainder, the
+    same bits as the pass over their sum."""
+    from deltaserve_amd import ops
+    x, r = _bf(_rnd(rows, D, seed=15) * 3).to(DEV), _bf(_rnd(rows, D, seed=16)).to(DEV)
+    w = _bf(1 + _rnd(D, seed=17).abs() * 0.1).to(DEV)
+    g = _rnd(parts, rows, D, seed=18).to(DEV)
+    total = g[0].clone()
+    for p in g[1:]:
+        total += p
+    for resid in (None, r):
+        got = ops.rmsnorm_backward(x, g, w, 1e-5, resid=resid)
+        assert torch.equal(got, ops.rmsnorm_backward(x, total, w, 1e-5, resid=resid))
+
+
 @pytest.mark.parametrize("scaling", [None, {"rope_type": "llama3", "factor": 8.0,
                                             "low_freq_factor": 1.0, "high_freq_factor": 4.0,
                                             "original_max_position_embeddings": 8192.0}])

@@ -47,10 +47,14 @@ def test_cycle_parity_head_dim_64(family):
 @pytest.mark.parametrize("I,lens", [(1536, [70]), (4096, [3, 90, 1]), (8192, [130, 31])])
 def test_cycle_parity_split_input_gradients(I, lens):
     """Few rows over a long reduction: the dX products of the FFN input run in
-    K slices (3 to 16 of them, none a multiple of four) whose partials the
-    RMSNorm backward adds, and the LM head's dH keeps one accumulator per
-    slice over three vocabulary chunks."""
+    K slices (as many as the cost model gives; test_rmsnorm_bwd_parts has the
+    counts one by one) whose partials the RMSNorm backward adds, and the LM
+    head's dH keeps one accumulator per slice over three vocabulary chunks."""
+    from deltaserve_amd import ops
     meta = tiny_meta(L=2, I=I, V=1500, s_max=sum(lens) + 3, vocab_chunk=512)
+    r = meta["lora_rank"]
+    _, slices = ops.gemm_plan(sum(lens) + 3, meta["hidden_size"], 2 * I + 2 * r, 4.0)
+    assert slices > 1, "the cost model no longer splits this product"
     worst = _run(meta, lens)
     # down_proj's A is bounded by 1/sqrt(I), so an element whose reference
     # gradient is within rounding of zero may be off by 2 steps of 2·lr, 4e-4·
