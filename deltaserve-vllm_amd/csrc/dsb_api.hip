@@ -185,7 +185,7 @@ struct dsb_handle {
   int D, Hq, Hkv, hd, q, kv, W3, I, V, r, L, N, max_tiles, vchunk, nvc, vgroup;
   HeadArgs head{};  // the LM head's plan (tiles, K slices, statistics layout)
   // the adapter's rank (rv) and the rank the kernels run at (r: rv rounded up,
-  // see dsb_create; the padded rows of A and columns of B are zeros in the
+  // see run_rank; the padded rows of A and columns of B are zeros in the
   // bf16 operands, so they add nothing, and their gradients are not stored)
   int rv;
   int gemm_cfg = -1;  // forced dense-product tile (GEMM_*), -1 by shape
@@ -371,6 +371,26 @@ float* grad_b(dsb_handle*, const LayerState& ls, int p) {
   return ls.has[p] ? ls.lora[p].gB : nullptr;
 }
 
+// The rank the kernels run at: a multiple of 8. Where the MLP has adapters and
+// operands large enough for the fused LoRA passes (ranks 16 and 32) to save
+// more than their reductions cost, ranks below those go up to them: separate
+// skinny and token-reduction passes would read h, d_gate and d_up twice.
+// Cycles of 3 to 4 layers padded against not, in % of the time saved: 8192
+// wide, rank 8 at 1024, 2048 and 4096 rows 3.5, 2.1 and 2.9, rank 24 at 2048
+// 4.1; 14336 wide, rank 4 or 8 at 300, 600, 1200 and 8192 rows 4.0, 1.0, −0.2
+// and 2.0; 17408 wide at 256 and 600 rows 0.5 and 1.5; but 3072 wide (1024
+// hidden) at 504, 1400, 3000, 6000 and 8192 rows −0.5, −2.5, −1.6, −1.4 and
+// −0.8, whose projections are too narrow to fill the fused passes. Adapters on
+// q, k, v and o alone: −1.6 at 2048 × 2048, within 0.4 either way at 4096 and
+// 5120 hidden.
+int run_rank(const dsb_handle* h) {
+  const int r = (h->rv + 7) / 8 * 8;
+  bool mlp = false;
+  for (const LayerState& ls : h->layers) mlp |= has_gu(ls) || ls.has[DSB_PROJ_DOWN];
+  if (!mlp || r > 32 || h->I < 8192 || (long)h->N * h->I <= (4L << 20)) return r;
+  return r <= 16 ? 16 : 32;
+}
+
 int finalize(dsb_handle* h) {
   if (h->finalized) return 0;
   for (int i = 0; i < h->L; ++i)
@@ -382,6 +402,7 @@ int finalize(dsb_handle* h) {
   if (!h->lm_w || !h->norm_w) return fail(h, "LM head / final norm not bound");
   if (!h->final_in || !h->ids || (int)h->layer_in.size() != h->L)
     return fail(h, "activations not bound");
+  h->r = run_rank(h);
   const int N = h->N, D = h->D, q = h->q, kv = h->kv, W3 = h->W3, I = h->I, r = h->r;
   const int rv = h->rv;
   const long NN = N + 1;
@@ -1646,14 +1667,7 @@ int dsb_create(const dsb_desc* d, dsb_handle** out) {
   h->hd = d->head_dim;
   h->q = h->Hq * h->hd; h->kv = h->Hkv * h->hd; h->W3 = h->q + 2 * h->kv;
   h->I = d->intermediate; h->V = d->vocab; h->L = d->n_layers;
-  h->rv = d->lora_rank;
-  // The rank the kernels run at: a multiple of 8. Where the MLP's operands are
-  // large enough for the fused LoRA passes (ranks 16 and 32) to save more than
-  // their reductions cost, ranks below those go up to them: separate skinny
-  // and token-reduction passes would read h, d_gate and d_up twice (rank 8,
-  // 2048 × 8192: cycle 4634 → 4539 µs; 504 × 3072: 1623 → 1631, so not there).
-  h->r = (h->rv + 7) / 8 * 8;
-  if (h->r <= 32 && (long)d->s_max * d->intermediate > (4L << 20)) h->r = h->r <= 16 ? 16 : 32;
+  h->rv = h->r = d->lora_rank;  // r: run_rank, once the adapters are bound
   h->N = d->s_max; h->s = d->lora_scaling; h->qwen = d->family == DSB_FAMILY_QWEN3;
   h->max_tiles = max_tiles_for(d->s_max, std::min(d->max_seqs, d->s_max));
   // LM-head vocab chunk: one pause point per chunk in each pass; the bf16

@@ -75,15 +75,19 @@ def test_cycle_parity_head_partials(family, Hq, Hkv, Hd, r, lens):
 
 
 @pytest.mark.parametrize("r", [3, 16, 17, 25])
-@pytest.mark.parametrize("s_max", [2048, 2049])
-def test_cycle_parity_rank_rule(r, s_max):
-    """Both sides of the line (s_max * intermediate = 2^22) past which ranks
-    below 16 and 32 run padded to them: gradients and masters keep the
-    adapter's own rank and the values of the unpadded product."""
-    meta = tiny_meta(L=1, I=2048, r=r, s_max=s_max)
-    worst = _run(meta, [65, 7])
+@pytest.mark.parametrize("I,s_max,projs", [(2048, 2048, O.PROJS), (2048, 2049, O.PROJS),
+                                           (8192, 512, O.PROJS), (8192, 513, O.PROJS),
+                                           (8192, 513, ("q", "k", "v", "o")),
+                                           (8192, 513, ("o", "down"))])
+def test_cycle_parity_rank_rule(r, I, s_max, projs):
+    """Both sides of the lines (intermediate = 8192, s_max * intermediate =
+    2^22, an adapter in the MLP) past which ranks below 16 and 32 run padded to
+    them: gradients and masters keep the adapter's own rank and the values of
+    the unpadded product."""
+    meta = tiny_meta(L=1, I=I, r=r, s_max=s_max)
+    worst = _run(meta, [65, 7], projs=projs)
     # masters by the explained bar, as above: down_proj's A is bounded by
-    # 1/sqrt(I), where 2 steps of 2·lr are 4e-4·sqrt(2048) = 1.8e-2
+    # 1/sqrt(I), where 2 steps of 2·lr are 4e-4·sqrt(I) = 1.8e-2 and 3.6e-2
     assert_north_star(worst, direct_masters=False)
 
 
