@@ -1170,10 +1170,16 @@ int enqueue_layer(dsb_handle* h, int li, int lo, hipStream_t st, bool rec, bool 
     if (ho) {
       // a small operand: the skinny pass alone is on the layer's critical path
       // (grad_B joins the layer's batched token reductions), 5 µs against 13
-      // for the fused pass and its reduction at 504 × 1024 to 256 × 5120
+      // for the fused pass and its reduction at 504 × 1024 to 256 × 5120; its
+      // own chain grows with the width. Cycles of 3 to 4 layers, rank 16, in %
+      // saved by the skinny pass: 1024 wide at 1000, 2000, 4000 and 8000 rows
+      // 3.1, 3.6, 0.8 and 0.8; 2048 wide at 1000, 2000 and 4000 2.8, 1.5 and
+      // −1.5; 4096 wide at 1000, 2000 and 4000 −0.8, −0.2 and 0.3; 5120 wide at
+      // 512, 800 and 1600 0.0, −0.6 and −0.2
+      const long small_o = (D <= 2048 ? 8L : 5L) << 19;
       const DualSpec d{h->grm, D, D, h->Zo_b, r, ls.BTo, h->gZo_b, r, ls.lora[DSB_PROJ_O].gB,
                        h->s, 1};
-      dual_o = (long)N * D <= (4L << 20) ? 1 : dual(h, &d, 1, r, st);
+      dual_o = (long)N * D <= small_o ? 1 : dual(h, &d, 1, r, st);
       if (dual_o < 0) return -1;
       if (dual_o) CKR(skinny(h, h->grm, D, ls.BTo, r, D, h->gZo_b, r, st));
     }
