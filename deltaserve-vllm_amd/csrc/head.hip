@@ -30,8 +30,10 @@
 // dominates the others' sum is rounded by up to 2^-9 (its exponential is 1 only
 // against a reference that is its own), and L/R restores it to fp32. 300 rows
 // with one column 17 above the sum of 2000 others: dH off by up to 2.5e-3 without
-// it, 1e-7 with. It costs a dot product with ones per two values (the head of
-// 2048 rows × 2048: 1802 and 1799 µs without and with it).
+// it, 1e-7 with. R comes from the matrix cores (P times ones, a row's values
+// being in the operand layout already): the logits products of 2048 × 2048 and
+// 8192 × 4096 take 689 µs on average, 698 with dot products of two values, 684
+// without R and the target's column kept apart.
 // The target's term stays out of the sums because softmax − onehot cancels
 // there: with p_t near 1 the row's loss and its coefficient of W[target],
 // p_t − 1, are L/e_t and −L/(e_t + L), full precision in L, while e_t + L
@@ -120,7 +122,7 @@ struct EpiCEProb {
         // tests the masks of 128 columns spill)
         const float tl = (float)(tcol[fm] - 4 * lq);
         auto take = [&](float ref, auto skips) {
-          float part[4] = {0.f, 0.f, 0.f, 0.f}, rpart[2] = {0.f, 0.f};
+          float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int fn = 0; fn < FN; ++fn)
 #pragma unroll
@@ -130,16 +132,18 @@ struct EpiCEProb {
               if (decltype(skips)::value) e *= fminf(fabsf((float)(fn * 16 + i) - tl), 1.f);
               part[i] += e;
               pk[fn][i] = (bf16)e;
-              if (i & 1) {  // two rounded values per instruction: their dot with ones
-                const bf16x2 two = {pk[fn][i - 1], pk[fn][i]}, ones = {(bf16)1.f, (bf16)1.f};
-                rpart[i >> 1] = __builtin_amdgcn_fdot2_f32_bf16(two, ones, rpart[i >> 1], false);
-              }
             }
+          // the rounded values' row sums: products with ones, in which the order
+          // of a row's values among its four lanes does not matter
+          f32x4 r = {0.f, 0.f, 0.f, 0.f};
+          const bf16 o = (bf16)1.f;
+          const bf16x8 ones = {o, o, o, o, o, o, o, o};
+#pragma unroll
+          for (int fn = 0; fn < FN; fn += 2)
+            r = mfma16(ones, __builtin_shufflevector(pk[fn], pk[fn + 1], 0, 1, 2, 3, 4, 5, 6, 7), r);
           float v = (part[0] + part[1]) + (part[2] + part[3]);
-          float r = rpart[0] + rpart[1];
           v += __shfl_xor(v, 16, 64);
-          r += __shfl_xor(r, 16, 64);
-          return CEStat{ref, v + __shfl_xor(v, 32, 64), r + __shfl_xor(r, 32, 64)};
+          return CEStat{ref, v + __shfl_xor(v, 32, 64), r[0]};
         };
         const int m = mw + fm * 16 + l16;
         CEStat st = take(ref0[fm], std::false_type{});
