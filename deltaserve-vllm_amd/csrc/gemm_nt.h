@@ -1,9 +1,9 @@
 // bf16 "NT" GEMM for gfx950: C[M,N] = A[M,K1]·B[N,K1]ᵀ (+ A2[M,K2]·B2[N,K2]ᵀ)
 // with a pluggable epilogue.
 //
-// Every dense contraction of the backward is phrased in this one form (both
-// operands K-contiguous): forward recompute uses the frozen weight [out,in] as
-// is, the dX products use the transposed copy made once at bind time, and the
+// Every dense contraction of the backward is phrased in this one form: the
+// forward recompute reads the frozen weight [out, in] with K along its rows, the
+// dX products read the same weight in place as a [K, N] operand (b_kn), and the
 // LoRA factor rides along as a second K segment (K-concatenation), so
 // y = x·Wᵀ + (x·Aᵀ)·(s·B)ᵀ is one kernel with K = in + r.
 //
@@ -1053,6 +1053,9 @@ inline GemmTile gemm_tile(int cfg) {
   }
 }
 
+// The CUs of an MI355X, the one device the estimate is fitted on.
+constexpr int kGemmCus = 256;
+
 // Estimated time (µs) of an M × N × K product with tile `cfg` and ks K slices,
 // `ob` bytes read and written per output element by its epilogue. The
 // constants are a fit (rms 10 %) to 3700 timings of the five tiles at 1 to 16
@@ -1072,10 +1075,11 @@ inline double gemm_cost(int M, int N, int K, double ob, int cfg, int ks) {
   const double tiles = (double)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   const int nk = (K + 63) / 64, steps = (nk + ks - 1) / ks;
   const double blocks = tiles * ks;
-  const double per_cu = std::ceil(blocks / 256), rounds = std::ceil(blocks / (256 * t.occ));
+  const double per_cu = std::ceil(blocks / kGemmCus),
+               rounds = std::ceil(blocks / (kGemmCus * t.occ));
   const double operands = 2.0 * K * ((double)M + N);
   double us = 5.0 + std::max(per_cu * steps * t.step + rounds * 0.5, operands / 6.8e6);
-  us += per_cu * t.bm * t.bn * (ks > 1 ? 4.0 : ob) * std::min(blocks, 256.0) / 7.8e6;
+  us += per_cu * t.bm * t.bn * (ks > 1 ? 4.0 : ob) * std::min(blocks, (double)kGemmCus) / 7.8e6;
   if (ks > 1) us += 2.9 + (4.0 * ks * M * N + ob * M * N) / 3.9e6;
   return us;
 }
@@ -1098,7 +1102,7 @@ inline GemmPlan gemm_plan(int M, int N, int K, double ob, bool can_split, int gl
     // slices: at least 3 K tiles each, and the split's blocks within one round
     const int most = can_split && N % 8 == 0 ? std::min(16, nk / 3) : 1;
     for (int ks = 1; ks <= std::max(1, most); ++ks) {
-      if (ks > 1 && tiles * ks > 256 * t.occ) break;
+      if (ks > 1 && tiles * ks > kGemmCus * t.occ) break;
       const double c = gemm_cost(M, N, K, ob, cfg, ks);
       if (bt == 0 || c < bt) {
         bt = c;

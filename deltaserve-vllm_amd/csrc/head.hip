@@ -66,9 +66,9 @@ constexpr float kSumLimit = 0x1p57f;
 
 // Per run of TN vocabulary columns (a wave tile's width) of chunk [c0, c0 + Vc)
 // and row: (reference m_t, Σ exp(logit − m_t), Σ of those values as P holds
-// them) into stats[m, (c0 + column) / TN] and P[m, j] = bf16(exp(logit[m, c0 + j] − m_t)) for the chunk's columns
-// j < Vc; the row's target column counts as zero in all, its logit goes to
-// tgt_logit[m]. Columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are written as zero so
+// them) into stats[m, (c0 + column) / TN] and P[m, j] = bf16(exp(logit[m, c0 +
+// j] − m_t)) for the chunk's columns j < Vc; the row's target column counts as
+// zero in all, its logit goes to tgt_logit[m]. Columns [Vc, Nc8) (Nc8 = round_up(Vc, 8)) are written as zero so
 // the dH product runs its K loop over whole 16-byte chunks. m_t is run_m[m]
 // unless the run's sum passes kSumLimit (or is NaN), then the run's maximum.
 // Runs that hold a target (one in V / TN of a row's) or pass the limit take the
@@ -407,17 +407,18 @@ void head_plan(HeadArgs& a, int gemm_cfg, bool can_split) {
     const GemmTile t = gemm_tile(cfg);
     const long tiles = (long)((a.n + t.bm - 1) / t.bm) * ((a.D + t.bn - 1) / t.bn);
     for (int ks = 1; ks <= (can_split && a.D % 8 == 0 ? std::min(16, nk / 3) : 1); ++ks) {
-      if (ks > 1 && tiles * ks > 256 * t.occ) break;
+      if (ks > 1 && tiles * ks > kGemmCus * t.occ) break;
       // ks blocks per tile run as ks · tiles plain ones of a K / ks product
       // whose epilogue reads and writes the accumulator
       double c = gemm_cost(a.n, a.D, (nk + ks - 1) / ks * 64, 0.0, cfg, 1);
       const double blocks = (double)tiles * ks;
       if (ks > 1) {
         const double steps = (nk + ks - 1) / ks, operands = 2.0 * a.vchunk * ((double)a.n + a.D);
-        c = 5.0 + std::max(std::ceil(blocks / 256) * steps * t.step + 0.5, operands / 6.8e6) +
+        c = 5.0 + std::max(std::ceil(blocks / kGemmCus) * steps * t.step + 0.5, operands / 6.8e6) +
             4.0 * ks * a.n * a.D / 3.9e6 / nch;
       }
-      c += std::ceil(blocks / 256) * t.bm * t.bn * 8.0 * std::min(blocks, 256.0) / 7.8e6;
+      c += std::ceil(blocks / kGemmCus) * t.bm * t.bn * 8.0 *
+           std::min(blocks, (double)kGemmCus) / 7.8e6;
       if (bt == 0 || c < bt) {
         bt = c;
         a.dh_cfg = cfg;

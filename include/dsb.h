@@ -63,7 +63,8 @@ typedef struct dsb_desc {
   float beta1, beta2, adam_eps, weight_decay, max_grad_norm;
   uint32_t flags;            /* DSB_FLAG_* */
   int32_t vocab_chunk;       /* LM-head vocab columns per chunk and pause point, a multiple
-                                of 256 (0: 16384, the reference's VOCAB_CHUNK, head.py:25) */
+                                of 256 (0: 16384, the reference's VOCAB_CHUNK, head.py:25,
+                                several chunks at a time over few rows) */
   int32_t gemm_tile;         /* dense-product tile: 0 by shape, else 256, 128 or 64 */
 } dsb_desc;
 
