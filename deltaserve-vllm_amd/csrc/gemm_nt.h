@@ -35,7 +35,7 @@
 // Chunks past K, and rows past M or N in an 8-row block that has some before,
 // are fetched from an offset outside the buffer descriptor and land as zeros; a
 // load with nothing of its own to fetch takes rows that exist or the zero page
-// (gemm_ring.h).
+// where a wait may leave it in flight (gemm_ring.h).
 //
 // Block ids are remapped so each XCD (round-robin dispatch over 8 XCDs) gets a
 // contiguous run of tiles, grouped 4 deep along M for L2 reuse.
@@ -356,7 +356,8 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   // the last load of tile k + 1 that may still be in flight at step k's wait,
   // and at the prologue's wait for its first tile.
   constexpr int WSTEP = (NA - 2) * IAB + (NB > NA ? IB : 0);
-  constexpr int WPRO = WSTEP + IAB;
+  constexpr int WPRO = ring_prologue_wait(NA, NB, IA, IB, false);
+  constexpr bool CLAMPA = ring_clamps_a(NA);
   static_assert(WPRO < 64, "vmcnt range");
   // LDS: NA slots of A tiles, then NB of B tiles (elements). A K tile is
   // loaded NA − 1 steps ahead of its use, the B tile NB − 1 (256 × 256: one
@@ -420,10 +421,10 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     return make_rsrc((s1 ? p.B : p.B2) + n0 + (long)k0 * ld,
                      (int)(((long)(rows - 1) * ld + rowsB) * 2));
   };
-  // lane byte offset of its first row; A load j adds j·8·NW rows, up to the
-  // wave's last row block, B load j starts at row brow0(j) of the descriptor
+  // lane byte offset of its first row; A load j adds j·8·NW rows (CLAMPA: up to
+  // the wave's last row block), B load j starts at row brow0(j) of the descriptor
   // (uniform)
-  const int rw = ring_row_block(8 * wave, rowsA) + lrow;
+  const int rw = (CLAMPA ? ring_row_block(8 * wave, rowsA) : 8 * wave) + lrow;
   const int voA1 = (rw * (int)p.lda + lch * 8) * 2, voB1 = (lrow * (int)p.ldb + lch * 8) * 2;
   const int voA2 = (rw * (int)p.lda2 + lch * 8) * 2, voB2 = (lrow * (int)p.ldb2 + lch * 8) * 2;
   const int stA1 = 16 * NW * (int)p.lda;  // bytes per 8·NW rows
@@ -522,7 +523,8 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
   auto go_one = [&](const auto& f, int j) __attribute__((always_inline)) {
     constexpr bool EDGE = std::decay_t<decltype(f)>::kEdge;
     if (j < IA) {
-      dma16_m0(f.dA, j == 0 ? f.voA : f.voA + min(j * f.stA, f.lastA));
+      const int off = j * f.stA;
+      dma16_m0(f.dA, j == 0 ? f.voA : f.voA + (CLAMPA ? min(off, f.lastA) : off));
     } else if constexpr (KN) {
       const int off = f.s1B ? vkn1[j - IA] : vkn2[j - IA];
       if constexpr (EDGE) {
@@ -678,7 +680,10 @@ __attribute__((amdgpu_waves_per_eu(WM* WN / 4, WM* WN / 4))) void gemm_nt_kernel
     prologue(make_fill1);
   else
     prologue(make_fill);
-  wait_vm<WPRO>();
+  if (!CLAMPA && rowsA < BM)
+    wait_vm<ring_prologue_wait(NA, NB, IA, IB, true)>();
+  else
+    wait_vm<WPRO>();
   lds_barrier();
 #pragma unroll
   for (int i = 0; i < NR; ++i) read_one(a_base(0), b_base(0), 0, 0, i);

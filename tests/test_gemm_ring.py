@@ -1,4 +1,5 @@
-"""Every load of the GEMM's LDS ring touches memory.
+"""Every load of the GEMM's LDS ring that a wait may leave in flight touches
+memory.
 
 The ring's waits count outstanding loads, which holds only if loads complete
 in issue order, and a buffer load whose every lane falls outside its
@@ -31,7 +32,10 @@ def ring(tmp_path_factory):
                    "int last_block(int r, int s, int n) { return ring_last_block(r, s, n); }\n"
                    "int fast_end(int a, int b, int w, int n) { return ring_fast_end(a, b, w, n); }\n"
                    "int whole_tiles(int kn, int nk, int n) { return ring_whole_tiles(kn, nk, n); }\n"
-                   "int kn_live(int r, int n) { return ring_kn_live(r, n); }\n}\n")
+                   "int kn_live(int r, int n) { return ring_kn_live(r, n); }\n"
+                   "int clamps_a(int na) { return ring_clamps_a(na); }\n"
+                   "int prologue_wait(int na, int nb, int ia, int ib, int r) {\n"
+                   "  return ring_prologue_wait(na, nb, ia, ib, r); }\n}\n")
     so = d / "ring.so"
     subprocess.run(["g++", "-std=c++17", "-shared", "-fPIC", f"-I{CSRC}", str(src), "-o", str(so)],
                    check=True)
@@ -93,3 +97,54 @@ def test_k_tiles_exist(ring, BM, BN, NA, NB, kn):
                                 for j in range(BN // (8 * NW)):
                                     r = rpl * (wave + j * NW)
                                     assert bool(ring.kn_live(r, live)) == (r < live)
+
+
+@pytest.mark.parametrize("BM,BN,NA,NB", TILES)
+def test_waits_cover_their_tiles(ring, BM, BN, NA, NB):
+    """A wait that leaves n loads in flight guarantees a load that touches
+    memory if at least n more such loads were issued after it (were it still
+    in flight, so would they be). Walked over the kernel's issue order with A
+    row blocks past M completing at once where they may: the prologue's wait
+    for the first tile, each step's for the next one, the last steps' for what
+    is left."""
+    ia, ib = BM // (8 * NW), BN // (8 * NW)
+    for rows in _rows(BM):
+        for tiles in range(1, 2 * NB + 3):
+            for wave in range(NW):
+                live = [bool(ring.clamps_a(NA)) or 8 * (wave + j * NW) < rows for j in range(ia)]
+                log = []  # (operand, tile, touches memory) in issue order
+
+                def fill(a, b):
+                    if a is not None:
+                        # spare slots of a short block read the zero page
+                        log.extend(("A", a, a >= tiles or t) for t in live)
+                    if b is not None:
+                        log.extend([("B", b, True)] * ib)
+
+                def covered(tile, n):
+                    for op in "AB":
+                        at = [i for i, (o, k, t) in enumerate(log) if o == op and k == tile and t]
+                        if at and sum(t for _, _, t in log[at[-1] + 1:]) < n:
+                            return False
+                    return True
+
+                if NB > NA:
+                    fill(None, 0)
+                for t in range(NA):
+                    fill(t, t + NB - NA)
+                ragged = not ring.clamps_a(NA) and rows < BM
+                assert covered(0, ring.prologue_wait(NA, NB, ia, ib, int(ragged)))
+                step = (NA - 2) * (ia + ib) + (ib if NB > NA else 0)
+                for kt in range(tiles):
+                    left = tiles - kt
+                    if left > NA:
+                        n = step
+                    else:
+                        n = step if left >= NB else 2 * (ia + ib) if NA > 4 and left == 4 else \
+                            ia + ib if NA > 3 and left == 3 else 0
+                    if kt + 1 < tiles:
+                        assert covered(kt + 1, n), (rows, tiles, wave, kt)
+                    if kt < tiles - NB:
+                        fill(kt + NA, kt + NB)
+                    elif NB > NA and kt < tiles - NA:
+                        fill(kt + NA, None)
